@@ -47,6 +47,8 @@ bool launch_w4a8_norm1(float *out, const float *add, const uint8_t *nib, const u
 // selects the tile height and ring depth, blocks the grid (0: one tile per
 // wave).  False when the shape is not covered.
 bool w4a8_dec_path(int rows, int cols, int gs);
+// K that the kernel's own norm or quantization of the input row covers.
+bool w4a8_dec_fused_ok(int cols);
 bool launch_w4a8_dec(float *out, const float *add, const uint8_t *nib, const uint8_t *params, const int8_t *q_split,
                      const float *scales, const float *sums, int rows, int cols, int gs, const float *nx,
                      const float *nw, float eps, hipStream_t s, int variant = 0, int blocks = 0);

@@ -35,6 +35,118 @@ void set_last_error(const std::string &m) { g_last_error = m; }
 // per-token arithmetic does not depend on the split).
 constexpr int kChunk = 1024;
 
+// Device scratch of the synchronous device-pointer calls (activations and
+// their packed forms), kept between calls: a call takes a block for itself
+// alone and gives it back after its stream has finished, so calls on several
+// threads and streams never share one.  An allocation and free per call cost
+// more than the small kernels they served (four hipMalloc / hipFree pairs:
+// about 20 us of a 46 us one-token gate|up call).  At most kPoolBlocks blocks
+// of at most kPoolBlockBytes are kept; larger ones are freed after the call,
+// and an allocation that runs out of memory first frees what is kept.
+constexpr int kPoolBlocks = 4;
+constexpr size_t kPoolBlockBytes = size_t(32) << 20;
+
+struct PoolBlock {
+  void *p;
+  size_t n;
+  int dev;
+};
+static std::mutex g_pool_mutex;
+static std::vector<PoolBlock> g_pool;
+
+// Frees the kept blocks of the current device; true when there were any.
+static bool pool_trim() {
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess) return false;
+  std::vector<void *> drop;
+  {
+    std::lock_guard<std::mutex> lk(g_pool_mutex);
+    for (size_t i = g_pool.size(); i-- > 0;)
+      if (g_pool[i].dev == dev) {
+        drop.push_back(g_pool[i].p);
+        g_pool.erase(g_pool.begin() + i);
+      }
+  }
+  for (void *p : drop) (void)hipFree(p);
+  return !drop.empty();
+}
+
+static void *device_alloc(size_t n) {
+  void *p = nullptr;
+  hipError_t e = hipMalloc(&p, n);
+  if (e == hipErrorOutOfMemory && pool_trim()) {
+    (void)hipGetLastError();
+    e = hipMalloc(&p, n);
+  }
+  HIP_CHECK(e);
+  return p;
+}
+
+// One call's scratch of `n` bytes for work on stream s, which must not be
+// capturing (the call ends with a synchronisation, which a capture cannot
+// hold; nothing is enqueued then).
+class CallScratch {
+ public:
+  CallScratch(size_t n, hipStream_t s) : s_(s) {
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    HIP_CHECK(hipStreamIsCapturing(s, &st));
+    if (st != hipStreamCaptureStatusNone) HIP_CHECK(hipErrorStreamCaptureUnsupported);
+    HIP_CHECK(hipGetDevice(&b_.dev));
+    {
+      std::lock_guard<std::mutex> lk(g_pool_mutex);
+      int best = -1;  // the smallest kept block that fits
+      for (int i = 0; i < (int)g_pool.size(); ++i)
+        if (g_pool[i].dev == b_.dev && g_pool[i].n >= n && (best < 0 || g_pool[i].n < g_pool[best].n)) best = i;
+      if (best >= 0) {
+        b_ = g_pool[best];
+        g_pool.erase(g_pool.begin() + best);
+        return;
+      }
+    }
+    // Rounded up so that nearby sizes share a block.
+    b_.n = std::max<size_t>((n + (size_t(1) << 20) - 1) & ~((size_t(1) << 20) - 1), size_t(1) << 20);
+    b_.p = device_alloc(b_.n);
+  }
+  CallScratch(const CallScratch &) = delete;
+  CallScratch &operator=(const CallScratch &) = delete;
+  // The next n bytes, 256-byte aligned; the sizes of all pieces, each
+  // rounded up to 256, are the constructor's n.
+  template <class T>
+  T *take(size_t n) {
+    T *p = reinterpret_cast<T *>(static_cast<uint8_t *>(b_.p) + used_);
+    used_ += (n + 255) & ~size_t(255);
+    return p;
+  }
+  // Waits for the call's work; the block may then serve another call.
+  void finish() {
+    HIP_CHECK(hipStreamSynchronize(s_));
+    done_ = true;
+  }
+  ~CallScratch() {
+    if (!done_ && hipStreamSynchronize(s_) != hipSuccess) {
+      (void)hipFree(b_.p);  // the work's state is unknown: never reused
+      return;
+    }
+    PoolBlock drop = b_;
+    if (b_.n <= kPoolBlockBytes) {
+      std::lock_guard<std::mutex> lk(g_pool_mutex);
+      g_pool.push_back(b_);
+      drop.p = nullptr;
+      if ((int)g_pool.size() > kPoolBlocks) {
+        drop = g_pool.front();
+        g_pool.erase(g_pool.begin());
+      }
+    }
+    if (drop.p) (void)hipFree(drop.p);
+  }
+
+ private:
+  PoolBlock b_{nullptr, 0, 0};
+  hipStream_t s_;
+  size_t used_ = 0;
+  bool done_ = false;
+};
+
 struct DevBuf {
   void *p = nullptr;
   DevBuf() = default;
@@ -46,8 +158,7 @@ struct DevBuf {
   void alloc(size_t n) {
     if (p) (void)hipFree(p);
     p = nullptr;
-    if (n == 0) n = 256;
-    HIP_CHECK(hipMalloc(&p, n));
+    p = device_alloc(n == 0 ? 256 : n);
   }
   template <class T>
   T *as() const {
@@ -1307,6 +1418,41 @@ int rai_hidden_to_logits(rai_model *m, const float *hidden, float *out) {
   return rai_hidden_to_logits_batch(m, hidden, out, 1);
 }
 
+// Activations of a call on device pointers: quantized rows and, where a
+// matrix-core kernel takes them, their packed form.
+namespace rai {
+
+struct CallActs {
+  int8_t *qn, *qs;
+  float *sc, *su;
+  _Float16 *qa;
+  uint8_t *mm;
+};
+
+static size_t piece(size_t n) { return (n + 255) & ~size_t(255); }
+
+// True when an output row shares memory with the input row: the GEMV may then
+// not read the input itself while it writes.
+static bool overlaps(const float *out, size_t rows, const float *x, size_t cols) {
+  return (uintptr_t)out < (uintptr_t)(x + cols) && (uintptr_t)x < (uintptr_t)(out + rows);
+}
+
+// Quantizes x [m][cols] into `a` (a.qa, when set, receives the matrix-core
+// layout).  Whole groups of 32, 64 or 128 take the eight-lanes-per-group
+// kernel, which reads and writes whole lines (one 14336-column row at group
+// 128: 37 -> 3 us against one thread per group); the natural-order codes are
+// written only for the kernel that reads them (other groups).
+static void quantize_call(const float *x, int m, int cols, int gs, const CallActs &a, hipStream_t s) {
+  if (fused_quant_ok(cols, gs)) {
+    launch_quant(x, m, cols, gs, a.qs, nullptr, a.sc, a.su, s, a.qa);
+  } else {
+    launch_quantize(x, m, cols, gs, a.qn, a.qs, a.sc, a.su, s);
+    if (a.qa) launch_qa_pack(a.qs, m, cols, a.qa, s);
+  }
+}
+
+}  // namespace rai
+
 int rai_w4a8_matmul_dev(float *out, const uint8_t *nib, const uint8_t *params, const float *x, size_t rows,
                         size_t cols, size_t m, size_t gs, void *stream) {
   RAI_API_BODY({
@@ -1319,25 +1465,28 @@ int rai_w4a8_matmul_dev(float *out, const uint8_t *nib, const uint8_t *params, c
     if (rows > INT32_MAX || cols > INT32_MAX || m > INT32_MAX) rai::fail(RAI_E_SHAPE, "dimensions overflow");
     hipStream_t s = (hipStream_t)stream;
     const size_t groups = rai::ceil_div(cols, gs);
-    rai::DevBuf qn, qs, sc, su;
-    qn.alloc(m * cols);
-    qs.alloc(m * cols);
-    sc.alloc(m * groups * 4);
-    su.alloc(m * groups * 4);
-    rai::launch_quantize(x, (int)m, (int)cols, (int)gs, qn.as<int8_t>(), qs.as<int8_t>(), sc.as<float>(),
-                         su.as<float>(), s);
-    rai::DevBuf qa, mm;
-    const bool mfma = rai::w4a8_mfma_path((int)rows, (int)cols, (int)m, (int)gs);
-    if (mfma) {
-      qa.alloc(sizeof(_Float16) * rai::qa_pack_halves((int)m, (int)cols));
-      rai::launch_qa_pack(qs.as<int8_t>(), (int)m, (int)cols, qa.as<_Float16>(), s);
+    // One token at a short row: the GEMV launch quantizes the row itself.
+    if (m == 1 && !rai::overlaps(out, rows, x, cols) &&
+        rai::launch_w4a8_dec(out, nullptr, nib, params, nullptr, nullptr, nullptr, (int)rows, (int)cols,
+                             (int)gs, x, nullptr, 0.0f, s)) {
+      HIP_CHECK(hipGetLastError());
+      HIP_CHECK(hipStreamSynchronize(s));
+      return RAI_OK;
     }
-    if (rai::w4a8_mm_path((int)rows, (int)cols, (int)m, (int)gs)) mm.alloc(rai::mm_pack_bytes((int)m, (int)cols));
-    rai::launch_w4a8(out, nullptr, nib, params, x, qn.as<int8_t>(), qs.as<int8_t>(), sc.as<float>(),
-                     su.as<float>(), (int)rows, (int)cols, (int)m, (int)gs, s, mfma ? qa.as<_Float16>() : nullptr,
-                     mm.as<uint8_t>());
+    const bool mfma = rai::w4a8_mfma_path((int)rows, (int)cols, (int)m, (int)gs);
+    const bool mm = rai::w4a8_mm_path((int)rows, (int)cols, (int)m, (int)gs);
+    const size_t nq = m * cols, ng = m * groups * 4;
+    const size_t nqa = mfma ? sizeof(_Float16) * rai::qa_pack_halves((int)m, (int)cols) : 0;
+    const size_t nmm = mm ? rai::mm_pack_bytes((int)m, (int)cols) : 0;
+    rai::CallScratch ws(2 * rai::piece(nq) + 2 * rai::piece(ng) + rai::piece(nqa) + rai::piece(nmm), s);
+    rai::CallActs a{ws.take<int8_t>(nq), ws.take<int8_t>(nq), ws.take<float>(ng), ws.take<float>(ng), nullptr, nullptr};
+    if (mfma) a.qa = ws.take<_Float16>(nqa);
+    if (mm) a.mm = ws.take<uint8_t>(nmm);
+    rai::quantize_call(x, (int)m, (int)cols, (int)gs, a, s);
+    rai::launch_w4a8(out, nullptr, nib, params, x, a.qn, a.qs, a.sc, a.su, (int)rows, (int)cols, (int)m, (int)gs, s,
+                     a.qa, a.mm);
     HIP_CHECK(hipGetLastError());
-    HIP_CHECK(hipStreamSynchronize(s));  // scratch is freed on return
+    ws.finish();  // the scratch serves the next call
   });
 }
 
@@ -1362,17 +1511,27 @@ static void fused_projections(float *const *outs, const rai_qlinear *const *lin,
   }
   hipStream_t s = (hipStream_t)stream;
   const size_t cols = lin[0]->cols, gs = lin[0]->group_size, groups = rai::ceil_div(cols, gs);
-  rai::DevBuf qn, qs, sc, su;
-  qn.alloc(cols);
-  qs.alloc(cols);
-  sc.alloc(groups * 4);
-  su.alloc(groups * 4);
-  rai::launch_quantize(x, 1, (int)cols, (int)gs, qn.as<int8_t>(), qs.as<int8_t>(), sc.as<float>(), su.as<float>(), s);
+  // Short rows: every GEMV launch quantizes the row itself.
+  bool self = true;
+  for (int i = 0; i < n && self; ++i)
+    self = rai::w4a8_dec_path((int)lin[i]->rows, (int)cols, (int)gs) && !rai::overlaps(outs[i], lin[i]->rows, x, cols);
+  if (self && rai::w4a8_dec_fused_ok((int)cols)) {
+    for (int i = 0; i < n; ++i)
+      rai::launch_w4a8_dec(outs[i], nullptr, lin[i]->nibbles, lin[i]->params, nullptr, nullptr, nullptr,
+                           (int)lin[i]->rows, (int)cols, (int)gs, x, nullptr, 0.0f, s);
+    HIP_CHECK(hipGetLastError());
+    HIP_CHECK(hipStreamSynchronize(s));
+    return;
+  }
+  rai::CallScratch ws(2 * rai::piece(cols) + 2 * rai::piece(groups * 4), s);
+  const rai::CallActs a{ws.take<int8_t>(cols), ws.take<int8_t>(cols), ws.take<float>(groups * 4),
+                        ws.take<float>(groups * 4), nullptr, nullptr};
+  rai::quantize_call(x, 1, (int)cols, (int)gs, a, s);
   for (int i = 0; i < n; ++i)
-    rai::launch_w4a8(outs[i], nullptr, lin[i]->nibbles, lin[i]->params, x, qn.as<int8_t>(), qs.as<int8_t>(),
-                     sc.as<float>(), su.as<float>(), (int)lin[i]->rows, (int)cols, 1, (int)gs, s, nullptr, nullptr);
+    rai::launch_w4a8(outs[i], nullptr, lin[i]->nibbles, lin[i]->params, x, a.qn, a.qs, a.sc, a.su, (int)lin[i]->rows,
+                     (int)cols, 1, (int)gs, s, nullptr, nullptr);
   HIP_CHECK(hipGetLastError());
-  HIP_CHECK(hipStreamSynchronize(s));  // scratch is freed on return
+  ws.finish();  // the scratch serves the next call
 }
 
 int rai_w4a8_fused_qkv_dev(float *q_out, float *k_out, float *v_out, const rai_qlinear *q, const rai_qlinear *k,
@@ -1467,11 +1626,18 @@ int rai_w4a8_matmul_noalloc_dev(float *out, const uint8_t *nib, const uint8_t *p
     _Float16 *qa = reinterpret_cast<_Float16 *>(base + 2 * rai::kNaTokenCols + 8 * rai::kNaGroups);
     uint8_t *mmp = base + 2 * rai::kNaTokenCols + 8 * rai::kNaGroups + rai::kNaQaBytes;
     hipStream_t s = (hipStream_t)stream;
-    // Every scratch byte a kernel reads is written earlier in this call (the
-    // pack writes the padding rows of the last token group as zeros), so the
-    // previous call's contents never reach the output.
-    rai::launch_quantize(x, (int)m, (int)cols, (int)gs, qn, qs, sc, su, s);
-    if (mfma) rai::launch_qa_pack(qs, (int)m, (int)cols, qa, s);
+    // Every scratch byte behind a stored output is written earlier in this
+    // call (the padding rows of the last token group may hold an earlier
+    // call's values, but reach only the outputs of padding tokens, which are
+    // not stored).
+    // One token at a short row: the GEMV launch quantizes the row itself.
+    if (m == 1 && !rai::overlaps(out, rows, x, cols) &&
+        rai::launch_w4a8_dec(out, nullptr, nib, params, nullptr, nullptr, nullptr, (int)rows, (int)cols,
+                             (int)gs, x, nullptr, 0.0f, s)) {
+      HIP_CHECK(hipGetLastError());
+      return RAI_OK;
+    }
+    rai::quantize_call(x, (int)m, (int)cols, (int)gs, {qn, qs, sc, su, mfma ? qa : nullptr, nullptr}, s);
     rai::launch_w4a8(out, nullptr, nib, params, x, qn, qs, sc, su, (int)rows, (int)cols, (int)m, (int)gs, s,
                      mfma ? qa : nullptr, mm ? mmp : nullptr);
     HIP_CHECK(hipGetLastError());

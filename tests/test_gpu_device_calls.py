@@ -1,0 +1,37 @@
+"""The device-pointer calls against the CPU oracle: every group size, token
+counts on both sides of each kernel's range, rows that leave partial tiles,
+and K that leaves partial tiles of groups.  Bar: bit-exact."""
+import numpy as np
+import pytest
+
+from rai_amd.workload import gemv_operands
+
+pytestmark = pytest.mark.gpu
+
+
+def _bits(a):
+    return np.ascontiguousarray(a, np.float32).view(np.uint32)
+
+
+def _call(rai, name, out, nib, params, x, rows, cols, m, gs):
+    rc = getattr(rai.lib(), name)(out.ptr, nib.ptr, params.ptr, x.ptr, rows, cols, m, gs, None)
+    assert rc == 0, rai.lib().rai_last_error()
+    assert rai.lib().rai_device_synchronize() == 0
+    return out.to_host(np.float32, m * rows)
+
+
+@pytest.mark.parametrize("name", ["rai_w4a8_matmul_dev", "rai_w4a8_matmul_noalloc_dev"])
+@pytest.mark.parametrize("n,m,gs", [(512, 1, 32), (512, 1, 64), (384, 1, 128), (4608, 1, 32), (512, 5, 32),
+                                    (320, 70, 64)])
+def test_output_over_its_own_input(rai, ora, name, n, m, gs):
+    """The output rows may lie on the input rows (the input is quantized
+    before anything is written); an infinite and a zero group among them."""
+    nib, params, x = gemv_operands(n, n, m, gs, seed=n + m + gs)
+    x = x.reshape(m, n)
+    x[0, gs // 2] = np.inf
+    x[m - 1, gs:2 * gs] = 0.0
+    want = ora.w4a8_matmul(nib, params, x, n, n, m, gs)
+    dev = rai.DeviceArray.from_host
+    buf = dev(np.ascontiguousarray(x, np.float32))
+    got = _call(rai, name, buf, dev(nib), dev(params), buf, n, n, m, gs)
+    assert np.array_equal(_bits(got).reshape(-1), _bits(want).reshape(-1))
