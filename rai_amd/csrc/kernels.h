@@ -23,7 +23,7 @@ void launch_quantize(const float *x, int m, int k, int gs, int8_t *q_nat, int8_t
 // layers.rs:503-531, fused into the epilogue).
 // `qa` (may be null): the activations packed by launch_qa_pack, which
 // enables the matrix-core kernel for 2..kMfmaMaxTokens tokens at group 32.
-// `mm` (may be null): mm_pack_bytes(m, cols) bytes of scratch, which
+// `mm` (may be null): mm_pack_bytes(m, cols, gs) bytes of scratch, which
 // enables the matrix-core GEMM for more than kMfmaMaxTokens tokens.
 // `params_tiled` (may be null): launch_params_tile16's copy of `params`,
 // which the matrix-core GEMV then reads.
@@ -126,16 +126,28 @@ bool launch_w4a8_mfma(float *out, const float *add, const uint8_t *nib, const ui
 // size as the input; requires params_tile16_ok.
 bool params_tile16_ok(int rows, int cols, int gs);
 void launch_params_tile16(const uint8_t *params, int rows, int cols, uint8_t *tiled, hipStream_t s);
-// Matrix-core W4A8 GEMM (gemm_mm.hip): group 32, K a multiple of 512,
+// Matrix-core W4A8 GEMM (gemm_mm.hip): whole groups of 32, 64 or 128,
 // more than kMfmaMaxTokens tokens.  Packs the block-split activations into
-// `pack` (mm_pack_bytes(m, cols) bytes), then runs the GEMM.
+// `pack` (mm_pack_bytes(m, cols, gs) bytes), then runs the GEMM.
 bool w4a8_mm_path(int rows, int cols, int m, int gs);
-size_t mm_pack_bytes(int m, int cols);
+size_t mm_pack_bytes(int m, int cols, int gs);
 void launch_w4a8_mm(float *out, const float *add, const uint8_t *nib, const uint8_t *params, const int8_t *q_split,
-                    const float *scales, const float *sums, int rows, int cols, int m, uint8_t *pack,
+                    const float *scales, const float *sums, int rows, int cols, int m, int gs, uint8_t *pack,
                     hipStream_t s);
-// True when launch_w4a8 takes the tiled fast path for this shape.
-bool w4a8_fast_path(int cols, int gs);
+// Token tiles of a grouped (MoE) GEMM: tile t runs expert tiles[t].x over the
+// entries tiles[t].y .. + tiles[t].z (at most 32); *ntiles of them are live.
+// src (may be null) maps an entry to its row of the quantized activations.
+struct MmMoe {
+  const int4 *tiles = nullptr;
+  const int *ntiles = nullptr, *src = nullptr;
+  const uint8_t *const *nib_tab = nullptr, *const *par_tab = nullptr;
+  int tstride = 0;
+};
+size_t mm_pack_tiles_bytes(int tiles, int cols, int gs);
+// True when launch_w4a8 takes one of the whole-group kernels, which load
+// codes and parameters in dwords and more (whole groups of 32, 64 or 128,
+// both arrays 4-byte aligned) and read the block-split activations only.
+bool w4a8_fast_path(int cols, int gs, const void *nib, const void *params);
 
 void launch_lane_sums(int32_t *out, const uint8_t *nib, const int8_t *q_nat, int rows, int cols,
                       int m, int gs, hipStream_t s);

@@ -1448,8 +1448,9 @@ bool launch_w4a8_norm1(float *out, const float *add, const uint8_t *nib, const u
   return true;
 }
 
-bool w4a8_fast_path(int cols, int gs) {
-  return (gs == 32 || gs == 64 || gs == 128) && cols % gs == 0;
+bool w4a8_fast_path(int cols, int gs, const void *nib, const void *params) {
+  return (gs == 32 || gs == 64 || gs == 128) && cols % gs == 0 &&
+         ((uintptr_t)nib | (uintptr_t)params) % 4 == 0;
 }
 
 void launch_w4a8(float *out, const float *add, const uint8_t *nib, const uint8_t *params, const float *x,
@@ -1457,18 +1458,26 @@ void launch_w4a8(float *out, const float *add, const uint8_t *nib, const uint8_t
                  const float *sums, int rows, int cols, int m, int gs, hipStream_t s,
                  const _Float16 *qa, uint8_t *mm, const uint8_t *params_tiled) {
   const int groups = (cols + gs - 1) / gs;
-  if (launch_w4a8_mfma(out, add, nib, params, qa, q_split, scales, sums, rows, cols, m, gs, s, params_tiled)) return;
-  if (mm && q_split && w4a8_mm_path(rows, cols, m, gs)) {
-    launch_w4a8_mm(out, add, nib, params, q_split, scales, sums, rows, cols, m, mm, s);
+  // Partial groups, other group sizes and misaligned arrays: one thread per
+  // output.
+  if (!q_split || !w4a8_fast_path(cols, gs, nib, params)) {
+    dim3 grid((rows + 127) / 128, m);
+    hipLaunchKernelGGL(k_w4a8_simple, grid, dim3(128), 0, s, out, add, nib, params, x, q_nat, scales,
+                       sums, rows, cols, m, gs, groups);
     return;
   }
-  if (m == 1 && q_split &&
+  if (launch_w4a8_mfma(out, add, nib, params, qa, q_split, scales, sums, rows, cols, m, gs, s, params_tiled)) return;
+  if (mm && w4a8_mm_path(rows, cols, m, gs)) {
+    launch_w4a8_mm(out, add, nib, params, q_split, scales, sums, rows, cols, m, gs, mm, s);
+    return;
+  }
+  if (m == 1 &&
       launch_w4a8_dec(out, add, nib, params, q_split, scales, sums, rows, cols, gs, nullptr, nullptr, 0.0f, s))
     return;
   // Decode (one token) at group 32, measured on the 7B shapes (4096..32000
   // rows, K 4096 / 14336): 16-row tiles for many rows, 8-row tiles for long
   // rows, 8-row whole-K blocks otherwise.
-  if (gs == 32 && m == 1 && w4a8_fast_path(cols, gs)) {
+  if (gs == 32 && m == 1) {
     if (rows >= 16384) {
       launch_small_mt<32, 1, 16>(out, add, nib, params, q_split, scales, sums, rows, cols, m, groups, s);
       return;
@@ -1484,7 +1493,7 @@ void launch_w4a8(float *out, const float *add, const uint8_t *nib, const uint8_t
   }
   // The whole-K kernel wins where few, long rows leave the streaming kernel
   // with too few blocks (measured on 1024..32000 x 2048..14336, g32).
-  if (w4a8_fast_path(cols, gs) && m == 1 && cols >= 4096 && rows <= cols) {
+  if (m == 1 && cols >= 4096 && rows <= cols) {
     bool done;
     if (gs == 32)
       done = launch_m1<32>(out, add, nib, params, q_split, scales, sums, rows, cols, groups, s);
@@ -1494,7 +1503,7 @@ void launch_w4a8(float *out, const float *add, const uint8_t *nib, const uint8_t
       done = launch_m1<128>(out, add, nib, params, q_split, scales, sums, rows, cols, groups, s);
     if (done) return;
   }
-  if (w4a8_fast_path(cols, gs) && m <= 16) {
+  if (m <= 16) {
     if (gs == 32)
       launch_small_gs<32>(out, add, nib, params, q_split, scales, sums, rows, cols, m, groups, s);
     else if (gs == 64)
@@ -1503,18 +1512,12 @@ void launch_w4a8(float *out, const float *add, const uint8_t *nib, const uint8_t
       launch_small_gs<128>(out, add, nib, params, q_split, scales, sums, rows, cols, m, groups, s);
     return;
   }
-  if (w4a8_fast_path(cols, gs)) {
-    if (gs == 32)
-      launch_fast_gs<32>(out, add, nib, params, q_split, scales, sums, rows, cols, m, groups, s);
-    else if (gs == 64)
-      launch_fast_gs<64>(out, add, nib, params, q_split, scales, sums, rows, cols, m, groups, s);
-    else
-      launch_fast_gs<128>(out, add, nib, params, q_split, scales, sums, rows, cols, m, groups, s);
-    return;
-  }
-  dim3 grid((rows + 127) / 128, m);
-  hipLaunchKernelGGL(k_w4a8_simple, grid, dim3(128), 0, s, out, add, nib, params, x, q_nat, scales,
-                     sums, rows, cols, m, gs, groups);
+  if (gs == 32)
+    launch_fast_gs<32>(out, add, nib, params, q_split, scales, sums, rows, cols, m, groups, s);
+  else if (gs == 64)
+    launch_fast_gs<64>(out, add, nib, params, q_split, scales, sums, rows, cols, m, groups, s);
+  else
+    launch_fast_gs<128>(out, add, nib, params, q_split, scales, sums, rows, cols, m, groups, s);
 }
 
 void launch_lane_sums(int32_t *out, const uint8_t *nib, const int8_t *q_nat, int rows, int cols,

@@ -278,7 +278,7 @@ struct Workspace {
     q_nat.alloc(K * maxm);
     q_split.alloc(K * maxm);
     qa.alloc(sizeof(_Float16) * qa_pack_halves(std::min(maxm, kMfmaMaxTokens), (int)K));
-    if (maxm > kMfmaMaxTokens) qmm.alloc(mm_pack_bytes(maxm, (int)K));
+    if (maxm > kMfmaMaxTokens) qmm.alloc(mm_pack_bytes(maxm, (int)K, (int)c.group_size));
     hq.alloc(H * maxm);
     qscale.alloc(sizeof(float) * G * maxm);
     qsum.alloc(sizeof(float) * G * maxm);
@@ -1441,9 +1441,10 @@ static bool overlaps(const float *out, size_t rows, const float *x, size_t cols)
 // layout).  Whole groups of 32, 64 or 128 take the eight-lanes-per-group
 // kernel, which reads and writes whole lines (one 14336-column row at group
 // 128: 37 -> 3 us against one thread per group); the natural-order codes are
-// written only for the kernel that reads them (other groups).
-static void quantize_call(const float *x, int m, int cols, int gs, const CallActs &a, hipStream_t s) {
-  if (fused_quant_ok(cols, gs)) {
+// written only for the kernel that reads them (`fast` is w4a8_fast_path of the
+// weights).
+static void quantize_call(const float *x, int m, int cols, int gs, bool fast, const CallActs &a, hipStream_t s) {
+  if (fast) {
     launch_quant(x, m, cols, gs, a.qs, nullptr, a.sc, a.su, s, a.qa);
   } else {
     launch_quantize(x, m, cols, gs, a.qn, a.qs, a.sc, a.su, s);
@@ -1466,23 +1467,24 @@ int rai_w4a8_matmul_dev(float *out, const uint8_t *nib, const uint8_t *params, c
     hipStream_t s = (hipStream_t)stream;
     const size_t groups = rai::ceil_div(cols, gs);
     // One token at a short row: the GEMV launch quantizes the row itself.
-    if (m == 1 && !rai::overlaps(out, rows, x, cols) &&
+    if (m == 1 && rai::w4a8_fast_path((int)cols, (int)gs, nib, params) && !rai::overlaps(out, rows, x, cols) &&
         rai::launch_w4a8_dec(out, nullptr, nib, params, nullptr, nullptr, nullptr, (int)rows, (int)cols,
                              (int)gs, x, nullptr, 0.0f, s)) {
       HIP_CHECK(hipGetLastError());
       HIP_CHECK(hipStreamSynchronize(s));
       return RAI_OK;
     }
-    const bool mfma = rai::w4a8_mfma_path((int)rows, (int)cols, (int)m, (int)gs);
-    const bool mm = rai::w4a8_mm_path((int)rows, (int)cols, (int)m, (int)gs);
+    const bool fast = rai::w4a8_fast_path((int)cols, (int)gs, nib, params);
+    const bool mfma = fast && rai::w4a8_mfma_path((int)rows, (int)cols, (int)m, (int)gs);
+    const bool mm = fast && rai::w4a8_mm_path((int)rows, (int)cols, (int)m, (int)gs);
     const size_t nq = m * cols, ng = m * groups * 4;
     const size_t nqa = mfma ? sizeof(_Float16) * rai::qa_pack_halves((int)m, (int)cols) : 0;
-    const size_t nmm = mm ? rai::mm_pack_bytes((int)m, (int)cols) : 0;
+    const size_t nmm = mm ? rai::mm_pack_bytes((int)m, (int)cols, (int)gs) : 0;
     rai::CallScratch ws(2 * rai::piece(nq) + 2 * rai::piece(ng) + rai::piece(nqa) + rai::piece(nmm), s);
     rai::CallActs a{ws.take<int8_t>(nq), ws.take<int8_t>(nq), ws.take<float>(ng), ws.take<float>(ng), nullptr, nullptr};
     if (mfma) a.qa = ws.take<_Float16>(nqa);
     if (mm) a.mm = ws.take<uint8_t>(nmm);
-    rai::quantize_call(x, (int)m, (int)cols, (int)gs, a, s);
+    rai::quantize_call(x, (int)m, (int)cols, (int)gs, fast, a, s);
     rai::launch_w4a8(out, nullptr, nib, params, x, a.qn, a.qs, a.sc, a.su, (int)rows, (int)cols, (int)m, (int)gs, s,
                      a.qa, a.mm);
     HIP_CHECK(hipGetLastError());
@@ -1512,9 +1514,10 @@ static void fused_projections(float *const *outs, const rai_qlinear *const *lin,
   hipStream_t s = (hipStream_t)stream;
   const size_t cols = lin[0]->cols, gs = lin[0]->group_size, groups = rai::ceil_div(cols, gs);
   // Short rows: every GEMV launch quantizes the row itself.
-  bool self = true;
+  bool self = true, fast = true;
+  for (int i = 0; i < n; ++i) fast = fast && rai::w4a8_fast_path((int)cols, (int)gs, lin[i]->nibbles, lin[i]->params);
   for (int i = 0; i < n && self; ++i)
-    self = rai::w4a8_dec_path((int)lin[i]->rows, (int)cols, (int)gs) && !rai::overlaps(outs[i], lin[i]->rows, x, cols);
+    self = fast && rai::w4a8_dec_path((int)lin[i]->rows, (int)cols, (int)gs) && !rai::overlaps(outs[i], lin[i]->rows, x, cols);
   if (self && rai::w4a8_dec_fused_ok((int)cols)) {
     for (int i = 0; i < n; ++i)
       rai::launch_w4a8_dec(outs[i], nullptr, lin[i]->nibbles, lin[i]->params, nullptr, nullptr, nullptr,
@@ -1526,7 +1529,9 @@ static void fused_projections(float *const *outs, const rai_qlinear *const *lin,
   rai::CallScratch ws(2 * rai::piece(cols) + 2 * rai::piece(groups * 4), s);
   const rai::CallActs a{ws.take<int8_t>(cols), ws.take<int8_t>(cols), ws.take<float>(groups * 4),
                         ws.take<float>(groups * 4), nullptr, nullptr};
-  rai::quantize_call(x, 1, (int)cols, (int)gs, a, s);
+  rai::quantize_call(x, 1, (int)cols, (int)gs, fast, a, s);
+  // One misaligned projection: the natural-order codes for it as well as the
+  // block-split ones, from the kernel that writes both.
   for (int i = 0; i < n; ++i)
     rai::launch_w4a8(outs[i], nullptr, lin[i]->nibbles, lin[i]->params, x, a.qn, a.qs, a.sc, a.su, (int)lin[i]->rows,
                      (int)cols, 1, (int)gs, s, nullptr, nullptr);
@@ -1563,13 +1568,15 @@ int rai_w4a8_fused_gate_up_dev(float *gate_out, float *up_out, const rai_qlinear
 // device on the first call there.  Layout (bytes): q_nat [m*cols], q_split
 // [m*cols], scales [m*groups] f32, sums [m*groups] f32, matrix-core
 // activations (2..64 tokens), the matrix-core GEMM's activation records
-// (more than 64 tokens at group 32: at most ceil(m/32) * cols/32 * 2304
-// bytes, which for m > 64 and m * cols <= 2^20 stays below 3/65 * 72 * 2^20).
+// (more than 64 tokens: ceil(m/32) tiles of the group count padded to 4, 2
+// or 2 (groups of 32, 64, 128) records of 64 gs + 260 bytes; with m > 64 and
+// m * cols <= 2^20 the largest is 1024 tiles of 4 records at cols = 32, gs =
+// 32: 9.02 MiB).
 namespace rai {
 constexpr size_t kNaTokenCols = size_t(1) << 20;  // m * cols
 constexpr size_t kNaGroups = size_t(1) << 16;     // m * ceil(cols / gs)
 constexpr size_t kNaQaBytes = size_t(2) << 20;
-constexpr size_t kNaMmBytes = size_t(7) << 19;  // 3.5 MiB
+constexpr size_t kNaMmBytes = (size_t(9) << 20) + (size_t(1) << 19);  // 9.5 MiB
 constexpr size_t kNaScratchBytes = 2 * kNaTokenCols + 8 * kNaGroups + kNaQaBytes + kNaMmBytes;
 constexpr int kNaMaxDevices = 64;
 }  // namespace rai
@@ -1612,11 +1619,12 @@ int rai_w4a8_matmul_noalloc_dev(float *out, const uint8_t *nib, const uint8_t *p
       rai::fail(RAI_E_SHAPE, "num_tokens * cols exceeds the allocation-free scratch (at most " +
                                  std::to_string(rai::kNaTokenCols) + " token columns and " +
                                  std::to_string(rai::kNaGroups) + " token groups)");
-    const bool mfma = rai::w4a8_mfma_path((int)rows, (int)cols, (int)m, (int)gs);
+    const bool fast = rai::w4a8_fast_path((int)cols, (int)gs, nib, params);
+    const bool mfma = fast && rai::w4a8_mfma_path((int)rows, (int)cols, (int)m, (int)gs);
     if (mfma && sizeof(_Float16) * rai::qa_pack_halves((int)m, (int)cols) > rai::kNaQaBytes)
       rai::fail(RAI_E_SHAPE, "activation tile exceeds the allocation-free scratch");
-    const bool mm = rai::w4a8_mm_path((int)rows, (int)cols, (int)m, (int)gs);
-    if (mm && rai::mm_pack_bytes((int)m, (int)cols) > rai::kNaMmBytes)
+    const bool mm = fast && rai::w4a8_mm_path((int)rows, (int)cols, (int)m, (int)gs);
+    if (mm && rai::mm_pack_bytes((int)m, (int)cols, (int)gs) > rai::kNaMmBytes)
       rai::fail(RAI_E_SHAPE, "activation records exceed the allocation-free scratch");
     uint8_t *base = rai::noalloc_scratch();
     int8_t *qn = reinterpret_cast<int8_t *>(base);
@@ -1631,13 +1639,13 @@ int rai_w4a8_matmul_noalloc_dev(float *out, const uint8_t *nib, const uint8_t *p
     // call's values, but reach only the outputs of padding tokens, which are
     // not stored).
     // One token at a short row: the GEMV launch quantizes the row itself.
-    if (m == 1 && !rai::overlaps(out, rows, x, cols) &&
+    if (m == 1 && rai::w4a8_fast_path((int)cols, (int)gs, nib, params) && !rai::overlaps(out, rows, x, cols) &&
         rai::launch_w4a8_dec(out, nullptr, nib, params, nullptr, nullptr, nullptr, (int)rows, (int)cols,
                              (int)gs, x, nullptr, 0.0f, s)) {
       HIP_CHECK(hipGetLastError());
       return RAI_OK;
     }
-    rai::quantize_call(x, (int)m, (int)cols, (int)gs, {qn, qs, sc, su, mfma ? qa : nullptr, nullptr}, s);
+    rai::quantize_call(x, (int)m, (int)cols, (int)gs, fast, {qn, qs, sc, su, mfma ? qa : nullptr, nullptr}, s);
     rai::launch_w4a8(out, nullptr, nib, params, x, qn, qs, sc, su, (int)rows, (int)cols, (int)m, (int)gs, s,
                      mfma ? qa : nullptr, mm ? mmp : nullptr);
     HIP_CHECK(hipGetLastError());
@@ -1669,7 +1677,7 @@ int rai_w4a8_time_dev(float *out, const uint8_t *nib, const uint8_t *params, con
       qa.alloc(sizeof(_Float16) * rai::qa_pack_halves((int)m, (int)cols));
       rai::launch_qa_pack(qs.as<int8_t>(), (int)m, (int)cols, qa.as<_Float16>(), s);
     }
-    if (rai::w4a8_mm_path((int)rows, (int)cols, (int)m, (int)gs)) mm.alloc(rai::mm_pack_bytes((int)m, (int)cols));
+    if (rai::w4a8_mm_path((int)rows, (int)cols, (int)m, (int)gs)) mm.alloc(rai::mm_pack_bytes((int)m, (int)cols, (int)gs));
     const size_t nib_bytes = rows * cols / 2, par_bytes = rows * groups * 4;
     // The parameters' tile-layout copies, as a loaded model holds them.
     rai::DevBuf tiled;

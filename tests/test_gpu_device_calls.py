@@ -35,3 +35,36 @@ def test_output_over_its_own_input(rai, ora, name, n, m, gs):
     buf = dev(np.ascontiguousarray(x, np.float32))
     got = _call(rai, name, buf, dev(nib), dev(params), buf, n, n, m, gs)
     assert np.array_equal(_bits(got).reshape(-1), _bits(want).reshape(-1))
+
+
+def _tokens(x, m, cols, gs, seed):
+    """Ordinary rows, and among them: values so small that the input sums are
+    subnormal, a scale past 2^88 in one group, a zero row, infinite sums."""
+    x = x.reshape(m, cols).astype(np.float32)
+    r = np.random.default_rng(seed)
+    x[r.integers(m)] *= np.float32(1e-39)
+    x[r.integers(m), :gs] *= np.float32(1e30)
+    x[r.integers(m)] = 0.0
+    return x
+
+
+# K: one group, fewer groups than a step or a stage of the kernel, one past a
+# stage, several stages with a remainder.
+MM = [(32, 32), (32, 96), (32, 544), (32, 1568), (32, 2048), (64, 64), (64, 320), (64, 576), (64, 1728),
+      (128, 128), (128, 384), (128, 640), (128, 2176)]
+
+
+@pytest.mark.parametrize("gs,cols", MM)
+@pytest.mark.parametrize("rows,m", [(1, 65), (127, 96), (130, 97), (300, 160)])
+def test_gemm_every_group_size(rai, ora, gs, cols, rows, m):
+    """More than 64 tokens: the matrix-core GEMM."""
+    nib, params, x = gemv_operands(rows, cols, m, gs, seed=rows + cols + m)
+    for special in (False, True):
+        if special:
+            x = _tokens(x, m, cols, gs, cols + m)
+        want = ora.w4a8_matmul(nib, params, x, rows, cols, m, gs)
+        dev = rai.DeviceArray.from_host
+        xd = dev(np.ascontiguousarray(x, np.float32))
+        for name in ("rai_w4a8_matmul_dev", "rai_w4a8_matmul_noalloc_dev"):
+            got = _call(rai, name, rai.DeviceArray(4 * m * rows), dev(nib), dev(params), xd, rows, cols, m, gs)
+            assert np.array_equal(_bits(got).reshape(-1), _bits(want).reshape(-1)), (name, special)
