@@ -418,4 +418,19 @@ void launch_w4a8_mm(float *out, const float *add, const uint8_t *nib, const uint
     go(launch_mm_t<128>);
 }
 
+bool moe_mm_path(int rows, int cols, int gs) { return w4a8_mm_path(rows, cols, kMfmaMaxTokens + 1, gs); }
+
+void launch_moe_mm(float *out, int ld, const MmMoe &moe, int max_tiles, const int8_t *q_split, const float *scales,
+                   const float *sums, int rows, int cols, int gs, uint8_t *pack, hipStream_t s) {
+  auto go = [&](auto launch) {
+    launch(out, nullptr, nullptr, nullptr, q_split, scales, sums, rows, cols, 0, max_tiles, ld, pack, moe, s);
+  };
+  if (gs == 32)
+    go(launch_mm_t<32>);
+  else if (gs == 64)
+    go(launch_mm_t<64>);
+  else
+    go(launch_mm_t<128>);
+}
+
 }  // namespace rai

@@ -144,6 +144,12 @@ struct MmMoe {
   int tstride = 0;
 };
 size_t mm_pack_tiles_bytes(int tiles, int cols, int gs);
+// Packs the entries' rows (q_split, scales, sums; null: `pack` holds them
+// already) and runs every tile (max_tiles launched) against its expert's
+// matrix; entry e's output row is out + e * ld.
+bool moe_mm_path(int rows, int cols, int gs);
+void launch_moe_mm(float *out, int ld, const MmMoe &moe, int max_tiles, const int8_t *q_split, const float *scales,
+                   const float *sums, int rows, int cols, int gs, uint8_t *pack, hipStream_t s);
 // True when launch_w4a8 takes one of the whole-group kernels, which load
 // codes and parameters in dwords and more (whole groups of 32, 64 or 128,
 // both arrays 4-byte aligned) and read the block-split activations only.
@@ -303,9 +309,11 @@ void launch_sample_plain(const float *logits, int V, uint32_t *ctx, int len, flo
 // Device MoE (moe.hip): group 32/64/128, hidden and FFN multiples of 256,
 // at most 1024 experts.
 bool moe_device_path(int hidden, int ffn, int gs, int experts);
-// ent_exp (may be null) receives each entry row's expert.
+// ent_exp (may be null) receives each entry row's expert; tiles / ntiles
+// (may be null) the grouped GEMM's token tiles, at most moe_max_tiles.
+inline int moe_max_tiles(int entries, int E) { return entries / 32 + (entries < E ? entries : E); }
 void launch_moe_plan(const int *sel, int m, int K, int E, int *off, int *ent_of, int *ent_tok, int *ent_exp,
-                     hipStream_t s);
+                     int4 *tiles, int *ntiles, hipStream_t s);
 void launch_moe_gather(const int8_t *q, const float *sc, const float *su, const int *ent_tok, const int *off, int E,
                        int max_entries, int cols, int groups, int8_t *qg, float *scg, float *sug, hipStream_t s);
 void launch_moe_gemv(float *out, int ld, const uint8_t *const *nibp, const uint8_t *const *parp, int nmat, int rows,

@@ -55,11 +55,15 @@ __device__ __forceinline__ int blk_dot(uint32_t codes, uint32_t q_even, uint32_t
 
 // One block; entries i = t * K + k with sel[i] >= 0.  off[0..E] are the
 // exclusive prefix sums of the per-expert counts; ent_of[i] the entry row of
-// (t, k) (-1 when the slot is empty); ent_tok[row] its token.
+// (t, k) (-1 when the slot is empty); ent_tok[row] its token.  tiles (may be
+// null): the token tiles of the grouped GEMM, {expert, first entry row, rows
+// (at most 32)}, expert by expert, *ntiles of them.
 __global__ __launch_bounds__(1024) void k_moe_plan(const int *__restrict__ sel, int n, int K, int E,
                                                    int *__restrict__ off, int *__restrict__ ent_of,
-                                                   int *__restrict__ ent_tok, int *__restrict__ ent_exp) {
-  extern __shared__ int cnt[];  // E + 1
+                                                   int *__restrict__ ent_tok, int *__restrict__ ent_exp,
+                                                   int4 *__restrict__ tiles, int *__restrict__ ntiles) {
+  extern __shared__ int cnt[];  // E + 1, then E + 1 tile offsets
+  int *toff = cnt + E + 1;
   for (int e = threadIdx.x; e <= E; e += blockDim.x) cnt[e] = 0;
   __syncthreads();
   for (int i = threadIdx.x; i < n; i += blockDim.x) {
@@ -68,16 +72,22 @@ __global__ __launch_bounds__(1024) void k_moe_plan(const int *__restrict__ sel, 
   }
   __syncthreads();
   if (threadIdx.x == 0) {
-    int run = 0;
+    int run = 0, trun = 0;
     for (int e = 0; e < E; ++e) {
       const int c = cnt[e];
       cnt[e] = run;
       off[e] = run;
       run += c;
+      toff[e] = trun;
+      trun += (c + 31) / 32;
     }
-    off[E] = run;
+    off[E] = cnt[E] = run;
+    if (ntiles) *ntiles = trun;
   }
   __syncthreads();
+  if (tiles)
+    for (int e = threadIdx.x; e < E; e += blockDim.x)
+      for (int r = cnt[e], t = toff[e]; r < cnt[e + 1]; r += 32, ++t) tiles[t] = make_int4(e, r, min(32, cnt[e + 1] - r), 0);
   for (int i = threadIdx.x; i < n; i += blockDim.x) {
     const int e = sel[i];
     if (e >= 0 && e < E) {
@@ -284,9 +294,9 @@ bool moe_device_path(int hidden, int ffn, int gs, int experts) {
 }
 
 void launch_moe_plan(const int *sel, int m, int K, int E, int *off, int *ent_of, int *ent_tok, int *ent_exp,
-                     hipStream_t s) {
-  hipLaunchKernelGGL(k_moe_plan, dim3(1), dim3(1024), sizeof(int) * (E + 1), s, sel, m * K, K, E, off, ent_of,
-                     ent_tok, ent_exp);
+                     int4 *tiles, int *ntiles, hipStream_t s) {
+  hipLaunchKernelGGL(k_moe_plan, dim3(1), dim3(1024), sizeof(int) * 2 * (E + 1), s, sel, m * K, K, E, off, ent_of,
+                     ent_tok, ent_exp, tiles, ntiles);
 }
 
 void launch_moe_gather(const int8_t *q, const float *sc, const float *su, const int *ent_tok, const int *off, int E,

@@ -250,7 +250,7 @@ struct Workspace {
   // MoE
   DevBuf sel, wts, eo, xg, yg, gg, ug, idx, wcol;
   // Device MoE path: entry plan, gathered quantized inputs, gate|up outputs.
-  DevBuf moff, ment_of, ment_tok, ment_exp, mq, msc, msu, mgu, mlogit;
+  DevBuf moff, ment_of, ment_tok, ment_exp, mtiles, mq, msc, msu, mgu, mlogit;
   int logit_rows = 0;
   void init(const rai_model &m, int maxm_, int logit_rows_) {
     const rai_model_config &c = m.cfg;
@@ -294,7 +294,12 @@ struct Workspace {
       ug.alloc(sizeof(float) * maxm * F);
       idx.alloc(sizeof(int) * maxm * c.experts_per_token);
       const size_t ne = (size_t)maxm * c.experts_per_token;
-      moff.alloc(sizeof(int) * (c.num_experts + 1));
+      moff.alloc(sizeof(int) * (c.num_experts + 2));  // and the tile count
+      const int nt = moe_max_tiles((int)ne, (int)c.num_experts);
+      mtiles.alloc(sizeof(int4) * nt);
+      if (maxm > kMfmaMaxTokens && moe_device_path((int)H, (int)F, (int)c.group_size, (int)c.num_experts))
+        qmm.alloc(std::max(mm_pack_bytes(maxm, (int)K, (int)c.group_size),
+                           mm_pack_tiles_bytes(nt, (int)std::max(H, F), (int)c.group_size)));
       ment_of.alloc(sizeof(int) * ne);
       ment_tok.alloc(sizeof(int) * ne);
       ment_exp.alloc(sizeof(int) * ne);
@@ -638,7 +643,7 @@ static void moe_block_device(const rai_model &md, int li, Workspace &w, int m, h
     }
   }
   launch_moe_plan(w.sel.as<int>(), m, K, E, w.moff.as<int>(), w.ment_of.as<int>(), w.ment_tok.as<int>(),
-                  w.ment_exp.as<int>(), s);
+                  w.ment_exp.as<int>(), nullptr, nullptr, s);
   launch_moe_gather(w.q_split.as<int8_t>(), w.qscale.as<float>(), w.qsum.as<float>(), w.ment_tok.as<int>(),
                     w.moff.as<int>(), E, ne, H, H / gs, w.mq.as<int8_t>(), w.msc.as<float>(), w.msu.as<float>(), s);
   launch_moe_gemv(w.mgu.as<float>(), 2 * F, tab, tab + 2 * E, 2, F, H, gs, E, w.mq.as<int8_t>(), w.msc.as<float>(),
@@ -650,53 +655,45 @@ static void moe_block_device(const rai_model &md, int li, Workspace &w, int m, h
   launch_moe_combine(w.hid.as<float>(), w.eo.as<float>(), w.wts.as<float>(), w.ment_of.as<int>(), m, K, H, s);
 }
 
-// Prefill-sized batches (more than kMfmaMaxTokens tokens): the same plan
-// and gather, then the per-expert offsets on the host (one synchronisation
-// per layer) and each expert's rows through the regular W4A8 kernels, which
-// are far faster than the grouped one once an expert holds many rows.
+// Prefill-sized batches (more than kMfmaMaxTokens tokens): the plan splits
+// every expert's entries into tiles of at most 32, and one GEMM launch per
+// projection runs all tiles of all experts (launch_moe_mm), so the chip is
+// filled whatever the counts are and the host waits for nothing.  Against one
+// GEMM per expert behind a synchronisation (64 experts, 512 tokens, hidden
+// 2048, FFN 1024: 89 GEMM, 70 GEMV and 106 pack launches per layer) the whole
+// block went from 5.5 to 1.4 ms.
+static bool moe_tiles_ok(const rai_model_config &c) {
+  const int H = c.hidden_size, F = c.intermediate_size, gs = c.group_size;
+  return moe_mm_path(2 * F, H, gs) && moe_mm_path(H, F, gs);
+}
+
 static void moe_block_device_large(const rai_model &md, int li, Workspace &w, int m, hipStream_t s) {
   const rai_model_config &c = md.cfg;
   const DLayer &L = md.layers[li];
   const int H = c.hidden_size, F = c.intermediate_size, E = c.num_experts, K = c.experts_per_token;
-  const int gs = c.group_size, ne = m * K, G = H / gs, GF = F / gs;
+  const int gs = c.group_size, ne = m * K, nt = moe_max_tiles(ne, E);
+  const uint8_t *const *tab = md.moe_tab.as<const uint8_t *>() + (size_t)6 * E * li;
+  float *gu = w.mgu.as<float>();
   launch_router(w.normed.as<float>(), L.router, m, H, E, K, c.norm_topk_prob, w.sel.as<int>(),
                 w.wts.as<float>(), w.mlogit.as<float>(), s);
+  int *ntiles = w.moff.as<int>() + E + 1;
   launch_moe_plan(w.sel.as<int>(), m, K, E, w.moff.as<int>(), w.ment_of.as<int>(), w.ment_tok.as<int>(), nullptr,
-                  s);
-  launch_moe_gather(w.q_split.as<int8_t>(), w.qscale.as<float>(), w.qsum.as<float>(), w.ment_tok.as<int>(),
-                    w.moff.as<int>(), E, ne, H, G, w.mq.as<int8_t>(), w.msc.as<float>(), w.msu.as<float>(), s);
-  std::vector<int> off(E + 1);
-  HIP_CHECK(hipMemcpyAsync(off.data(), w.moff.p, sizeof(int) * (E + 1), hipMemcpyDeviceToHost, s));
-  HIP_CHECK(hipStreamSynchronize(s));
-  float *gate = w.mgu.as<float>(), *up = gate + (size_t)ne * F;
-  auto run = [&](const DLinear &lin, const int8_t *q, const float *sc, const float *su, int groups, int o, int cnt,
-                 float *out) {
-    const _Float16 *qa = nullptr;
-    if (w4a8_mfma_path(lin.rows, lin.cols, cnt, lin.gs)) {
-      launch_qa_pack(q + (size_t)o * lin.cols, cnt, lin.cols, w.qa.as<_Float16>(), s);
-      qa = w.qa.as<_Float16>();
-    }
-    launch_w4a8(out, nullptr, lin.nib, lin.params, nullptr, nullptr, q + (size_t)o * lin.cols,
-                sc + (size_t)o * groups, su + (size_t)o * groups, lin.rows, lin.cols, cnt, lin.gs, s, qa,
-                w.qmm.as<uint8_t>());
-  };
-  for (int e = 0; e < E; ++e) {
-    const int o = off[e], cnt = off[e + 1] - off[e];
-    if (cnt == 0) continue;
-    const DLinear *ex = &L.experts[(size_t)e * 3];
-    run(ex[0], w.mq.as<int8_t>(), w.msc.as<float>(), w.msu.as<float>(), G, o, cnt, gate + (size_t)o * F);
-    run(ex[1], w.mq.as<int8_t>(), w.msc.as<float>(), w.msu.as<float>(), G, o, cnt, up + (size_t)o * F);
+                  w.mtiles.as<int4>(), ntiles, s);
+  // gate and up: one matrix where they lie back to back, else two launches on
+  // the same packed rows.
+  MmMoe t{w.mtiles.as<int4>(), ntiles, w.ment_tok.as<int>(), tab, tab + 2 * E, 2};
+  launch_moe_mm(gu, 2 * F, t, nt, w.q_split.as<int8_t>(), w.qscale.as<float>(), w.qsum.as<float>(),
+                L.experts_gu ? 2 * F : F, H, gs, w.qmm.as<uint8_t>(), s);
+  if (!L.experts_gu) {
+    t.nib_tab = tab + 1;
+    t.par_tab = tab + 2 * E + 1;
+    launch_moe_mm(gu + F, 2 * F, t, nt, nullptr, nullptr, nullptr, F, H, gs, w.qmm.as<uint8_t>(), s);
   }
-  const int total = off[E];
-  if (total > 0)
-    launch_silu_quant(gate, up, total, F, F, gs, w.mq.as<int8_t>(), nullptr, w.msc.as<float>(), w.msu.as<float>(),
-                      s, nullptr);
-  for (int e = 0; e < E; ++e) {
-    const int o = off[e], cnt = off[e + 1] - off[e];
-    if (cnt == 0) continue;
-    run(L.experts[(size_t)e * 3 + 2], w.mq.as<int8_t>(), w.msc.as<float>(), w.msu.as<float>(), GF, o, cnt,
-        w.eo.as<float>() + (size_t)o * H);
-  }
+  launch_silu_quant(gu, gu + F, ne, F, 2 * F, gs, w.mq.as<int8_t>(), nullptr, w.msc.as<float>(), w.msu.as<float>(),
+                    s, nullptr);
+  const MmMoe d{w.mtiles.as<int4>(), ntiles, nullptr, tab + 4 * E, tab + 5 * E, 1};
+  launch_moe_mm(w.eo.as<float>(), H, d, nt, w.mq.as<int8_t>(), w.msc.as<float>(), w.msu.as<float>(), H, F, gs,
+                w.qmm.as<uint8_t>(), s);
   launch_moe_combine(w.hid.as<float>(), w.eo.as<float>(), w.wts.as<float>(), w.ment_of.as<int>(), m, K, H, s);
 }
 
@@ -849,7 +846,7 @@ static void forward_enqueue(rai_model &md, rai_kv &kv, Workspace &w, int m, size
     const bool gu1 = norm1 && L.gate_up.rows && fused_quant_ok(F, gs) &&
                      w4a8_norm1_path(L.gate_up.rows, L.gate_up.cols, L.gate_up.gs);
     if (!gu1) norm_then_quant(L.post_norm);
-    if (c.num_experts > 0 && moe_on_device(md) && m > kMfmaMaxTokens && !st) {
+    if (c.num_experts > 0 && moe_on_device(md) && m > kMfmaMaxTokens && moe_tiles_ok(c)) {
       moe_block_device_large(md, li, w, m, s);
     } else if (c.num_experts > 0 && moe_on_device(md)) {
       moe_block_device(md, li, w, m, s);

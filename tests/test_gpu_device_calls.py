@@ -68,3 +68,17 @@ def test_gemm_every_group_size(rai, ora, gs, cols, rows, m):
         for name in ("rai_w4a8_matmul_dev", "rai_w4a8_matmul_noalloc_dev"):
             got = _call(rai, name, rai.DeviceArray(4 * m * rows), dev(nib), dev(params), xd, rows, cols, m, gs)
             assert np.array_equal(_bits(got).reshape(-1), _bits(want).reshape(-1)), (name, special)
+
+
+@pytest.mark.parametrize("gs,experts,topk,m", [(32, 8, 3, 70), (64, 16, 2, 150), (128, 5, 5, 65), (32, 64, 8, 97)])
+def test_sparse_layer_prefill(rai, ora, gs, experts, topk, m):
+    """More than 64 tokens through a sparse layer: every expert's tiles in one
+    launch (experts without a token, with one tile and with several)."""
+    img = rai.synth_model(256, 2, 4, 4, 64, 512, 500, 256, group_size=gs, num_experts=experts,
+                          experts_per_token=topk, seed=gs + m)
+    gm, om = rai.RaiModel.from_bytes(img), ora.Model(img, 128)
+    h = np.random.default_rng(m).normal(0.0, 1.0, (m, 256)).astype(np.float32)
+    h[m // 2:] = h[0] + 1e-3 * h[m // 2:]  # crowd some experts
+    got = gm.forward_batch(h, np.arange(m), gm.create_kv_cache(256))
+    want = om.forward_batch(h, np.arange(m), om.create_kv(256))
+    assert np.array_equal(_bits(got).reshape(-1), _bits(want).reshape(-1))
