@@ -163,6 +163,12 @@ void launch_tied_lm_head(float *logits, const float *hidden, const uint8_t *code
                          const uint8_t *params, int vocab, int n, int gs, int m, int8_t *hq,
                          float *hscales, float *hsums, hipStream_t s);
 
+// Its kernel for whole groups of 32, 64 or 128 (tied_head.hip); hq 16-byte
+// aligned.
+bool tied_head_wave_path(int n, int gs, const void *codes, const void *params);
+void launch_tied_head_wave(float *logits, const float *hidden, const uint8_t *codes, const uint8_t *params, int vocab,
+                           int n, int gs, int m, int8_t *hq, float *hscales, float *hsums, hipStream_t s);
+
 // Embedding rows (gemm.rs:1926-1970, model.rs:371-403) for token ids read
 // from `tokens` (device), or, when tokens == null, from
 // ctx[last] followed by ctx[start .. start+m-1) (the lookup verify batch).

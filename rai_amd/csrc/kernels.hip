@@ -1531,6 +1531,10 @@ void launch_lane_sums(int32_t *out, const uint8_t *nib, const int8_t *q_nat, int
 void launch_tied_lm_head(float *logits, const float *hidden, const uint8_t *codes,
                          const uint8_t *params, int vocab, int n, int gs, int m, int8_t *hq,
                          float *hscales, float *hsums, hipStream_t s) {
+  if (tied_head_wave_path(n, gs, codes, params)) {
+    launch_tied_head_wave(logits, hidden, codes, params, vocab, n, gs, m, hq, hscales, hsums, s);
+    return;
+  }
   const int groups = (n + gs - 1) / gs;
   hipLaunchKernelGGL(k_quantize63, dim3((groups + 63) / 64, m), dim3(64), 0, s, hidden, m, n, gs,
                      groups, hq, hscales, hsums);

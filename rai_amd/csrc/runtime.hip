@@ -1800,14 +1800,12 @@ int rai_tied_lm_head_dev(float *logits, const float *hidden, const uint8_t *code
     if (n == 0 || n % 2) rai::fail(RAI_E_SHAPE, "hidden_size must be non-zero and even");
     hipStream_t s = (hipStream_t)stream;
     const size_t groups = rai::ceil_div(n, gs);
-    rai::DevBuf hq, sc, su;
-    hq.alloc(n);
-    sc.alloc(groups * 4);
-    su.alloc(groups * 4);
-    rai::launch_tied_lm_head(logits, hidden, codes, params, (int)vocab, (int)n, (int)gs, 1, hq.as<int8_t>(),
-                             sc.as<float>(), su.as<float>(), s);
+    rai::CallScratch ws(rai::piece(n) + 2 * rai::piece(groups * 4), s);
+    int8_t *hq = ws.take<int8_t>(n);
+    float *sc = ws.take<float>(groups * 4), *su = ws.take<float>(groups * 4);
+    rai::launch_tied_lm_head(logits, hidden, codes, params, (int)vocab, (int)n, (int)gs, 1, hq, sc, su, s);
     HIP_CHECK(hipGetLastError());
-    HIP_CHECK(hipStreamSynchronize(s));
+    ws.finish();  // the scratch serves the next call
   });
 }
 

@@ -82,3 +82,33 @@ def test_sparse_layer_prefill(rai, ora, gs, experts, topk, m):
     got = gm.forward_batch(h, np.arange(m), gm.create_kv_cache(256))
     want = om.forward_batch(h, np.arange(m), om.create_kv(256))
     assert np.array_equal(_bits(got).reshape(-1), _bits(want).reshape(-1))
+
+
+def _table(vocab, hidden, gs, seed):
+    r = np.random.default_rng(seed)
+    codes = r.integers(0, 256, vocab * hidden, dtype=np.uint8)
+    par = np.stack([r.uniform(0.0005, 0.002, (vocab, hidden // gs)), r.normal(0.0, 0.05, (vocab, hidden // gs))], 2)
+    return codes, np.ascontiguousarray(par.astype(np.float16)).view(np.uint8).reshape(-1)
+
+
+# Units of 32 columns: under one chunk of 64, one chunk, one past it, several.
+@pytest.mark.parametrize("gs,hidden", [(32, 32), (32, 2048), (32, 2080), (64, 192), (64, 2112), (64, 4096),
+                                       (128, 128), (128, 2176), (128, 5120)])
+@pytest.mark.parametrize("vocab", [1, 15, 200])
+def test_tied_head_every_group_size(rai, ora, gs, hidden, vocab):
+    codes, par = _table(vocab, hidden, gs, hidden + vocab)
+    h = np.random.default_rng(vocab).normal(0.0, 1.0, hidden).astype(np.float32)
+    for scale in (1.0, 1e-39, 1e30):
+        hh = (h * np.float32(scale)).astype(np.float32)
+        hh[: gs // 2] = 0.0
+        want = ora.tied_lm_head(hh, codes, par, vocab, gs)
+        assert np.array_equal(_bits(rai.tied_lm_head(hh, codes, par, vocab, gs)), _bits(want)), scale
+
+
+@pytest.mark.parametrize("m", [1, 4, 9])
+def test_tied_logits_of_a_batch(rai, ora, m):
+    img = rai.synth_model(256, 1, 4, 4, 64, 512, 333, 64, group_size=32, tied=True, seed=m)
+    gm, om = rai.RaiModel.from_bytes(img), ora.Model(img, 128)
+    h = np.random.default_rng(m).normal(0.0, 1.0, (m, 256)).astype(np.float32)
+    got, want = gm.hidden_to_logits_batch(h, m), om.hidden_to_logits_batch(h, m)
+    assert np.array_equal(_bits(got).reshape(-1), _bits(want).reshape(-1))
