@@ -1,24 +1,27 @@
-// One-token W4A8 GEMV (decode), group 32, wave-streamed.
+// One-token W4A8 GEMV (decode), groups of 32, 64 or 128, wave-streamed.
 //
 // Same arithmetic as the reference's AVX2 kernel for one input row
-// (gemm.rs:458-537, 1774-1919): per (row, group) the four 8-column block
-// sums S_l (exact int32 via v_dot4), cs = fl(ws * as), the lane products
-// fl(float(S_l) * cs) and the zero term fl(wz * xsum); per row four lane
-// chains and one zero chain accumulated in group order, and at the end
-// hsum8(f0..f3, 0, 0, 0, 0) + zc.
+// (gemm.rs:458-537, 1774-1919): per (row, group) the reference lanes' sums
+// S_l (exact int32 via v_dot4; lane l takes the 8-column blocks l, l + 4, ...
+// of a group of 32, l, l + 8, ... of 64 or 128), cs = fl(ws * as), the lane
+// products fl(float(S_l) * cs) and the zero term fl(wz * xsum); per row four
+// (group 32) or eight lane chains and one zero chain accumulated in group
+// order, and at the end hsum8(f) + zc.
 //
 // Work split.  Every wave owns tiles of R rows and walks them chunk by chunk
-// (32 groups = 1024 columns per chunk).  Lane (h = lane / 32, k = lane % 32)
-// holds group k of the chunk for the R/2 rows 2i + h, so one load
-// instruction reads two 512-byte runs of packed codes and two 128-byte runs
-// of group parameters.  Loads stream through a ring of D chunks in
+// (1024 columns, 32 units of 32).  Lane (h = lane / 32, k = lane % 32)
+// holds unit k of the chunk for the R/2 rows 2i + h, so one load
+// instruction reads two 512-byte runs of packed codes and two runs
+// of group parameters.  A group of 32 is one unit; the two lanes of a group
+// of 64 hold four chains' products each; the four of a group of 128 add
+// their block sums pairwise (lane k and k ^ 2 by DPP: blocks l and l + 8)
+// and keep two chains' products each.  Loads stream through a ring of D chunks in
 // registers: every load is issued (past the last chunk it points beyond the
 // buffer, which a raw buffer load answers with zeros without touching
 // memory), so the compiler's wait counts stay exact and D chunks stay in
 // flight across tile boundaries.  The lane products go through a
-// wave-private LDS area (two buffers) and come back transposed: lane
-// c = l * R + r runs chain l of row r over the chunk's 32 products in group
-// order, one chunk behind the products, so the chain's dependent adds
+// wave-private LDS area (two buffers) and come back transposed: one lane
+// runs chain l of row r over the chunk's products in group order, one chunk behind the products, so the chain's dependent adds
 // interleave with the next chunk's product instructions.  No block
 // barrier is taken after the prologue, which stages the activations
 // (int8 codes in the block-split order, scales and sums; ST = 1, 2, 4
@@ -44,9 +47,8 @@ namespace {
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int kDecWaves = 4;       // waves per block
-constexpr int kDecChunk = 32;      // groups per chunk
-constexpr int kDecRowStride = 36;  // floats per (chain, row) run of 32 products, padded
-constexpr int kDecMaxGroups = 448; // K <= 14336 staged in LDS
+constexpr int kDecChunk = 32;      // 32-column units per chunk
+constexpr int kDecMaxUnits = 448;  // K <= 14336 staged in LDS
 
 __device__ __forceinline__ float dec_f16(uint32_t bits) {
   return __half2float(__ushort_as_half((uint16_t)bits));
@@ -62,12 +64,21 @@ __device__ __forceinline__ int dec_block_dot(uint32_t codes, uint32_t q_even, ui
                                 false);
 }
 
-template <int R>
+template <int GS, int R>
 struct DecCfg {
-  static_assert(R % 2 == 0 && 5 * R <= 64, "one chain per lane");
-  static constexpr int IPL = R / 2;                    // (row, group) items per lane and chunk
-  static constexpr int LSTR = R * kDecRowStride;       // floats per chain
-  static constexpr int WAVE_FLOATS = 10 * LSTR + 64;   // two product buffers + final chain values
+  static constexpr int NL = GS == 32 ? 4 : 8;          // reference lanes
+  static constexpr int NC = NL + 1;                    // chains per row
+  static_assert(R % 2 == 0 && NC * R <= 64, "one chain per lane");
+  static constexpr int LPG = GS / 32;                  // units (lanes) per group
+  static constexpr int GPC = kDecChunk / LPG;          // groups per chunk
+  static constexpr int IPL = R / 2;                    // (row, unit) items per lane and chunk
+  static constexpr int STR = GPC + 4;                  // floats per run of a chunk's products, padded
+  static constexpr int BUF = NC * R * STR;             // floats per product buffer
+  static constexpr int WAVE_FLOATS = 2 * BUF + 64;     // two product buffers + final chain values
+  // Run of chain l of row r (and the lane that sums it): chain-major at group
+  // 32, row-major otherwise, where the lanes of one group write different
+  // chains and these runs fall on different banks.
+  __device__ static constexpr int run(int l, int r) { return GS == 32 ? l * R + r : r * NC + l; }
 };
 
 // LDS bytes of a block: activations (codes, scales, sums) and the waves'
@@ -75,10 +86,10 @@ struct DecCfg {
 // norm's chain-major row scratch.
 __host__ __device__ inline int dec_act_bytes(int cols) { return (cols + 8 * (cols / 32) + 15) & ~15; }
 
-template <int R>
+template <int GS, int R>
 size_t dec_smem(int cols, bool fused) {
   const size_t act = dec_act_bytes(cols);
-  const size_t waves = sizeof(float) * (size_t)kDecWaves * DecCfg<R>::WAVE_FLOATS;
+  const size_t waves = sizeof(float) * (size_t)kDecWaves * DecCfg<GS, R>::WAVE_FLOATS;
   return act + std::max(waves, fused ? sizeof(float) * (size_t)rms_scratch_floats(cols) : size_t(0));
 }
 
@@ -115,7 +126,7 @@ __device__ __forceinline__ void rope_store_pair(const DecRope &rp, float *out, i
   }
 }
 
-template <int R, int D, int ST, int EPI>
+template <int GS, int R, int D, int ST, int EPI>
 __global__ __launch_bounds__(256) void k_w4a8_dec(float *out, const float *add, const uint8_t *__restrict__ nib,
                                                   const uint8_t *__restrict__ params,
                                                   const int8_t *__restrict__ q_split,
@@ -124,18 +135,20 @@ __global__ __launch_bounds__(256) void k_w4a8_dec(float *out, const float *add, 
                                                   int tiles_per_wave, const float *__restrict__ nx,
                                                   const float *__restrict__ nw, float eps, DecRope rope,
                                                   DecMoe moe) {
-  using C = DecCfg<R>;
-  constexpr int IPL = C::IPL, LSTR = C::LSTR;
+  using C = DecCfg<GS, R>;
+  constexpr int IPL = C::IPL, NL = C::NL, NC = C::NC, LPG = C::LPG, GPC = C::GPC, STR = C::STR;
+  constexpr int RH = R / 2;  // rows of each half of a head in a rope tile
   // MOE: one grid row per MoE entry; GLU: the block's gate|up output group
   // through silu_mul and its quantization (both for an entry's experts).
   constexpr bool MOE = EPI == kEpiMoe || EPI == kEpiMoeGlu, GLU = EPI == kEpiGlu || EPI == kEpiMoeGlu;
   constexpr bool ROPE = EPI == kEpiRope;
   static_assert(EPI != kEpiGlu || (R == 8 && ST == 0), "a gate|up block: 4 waves x 8 rows, fused input norm");
   static_assert(EPI != kEpiMoeGlu || R == 8, "an entry's gate|up block: 4 waves x 8 rows");
-  static_assert(!ROPE || R == 8, "a rope tile: 4 rows of each half of a head");
+  static_assert(!GLU || GS == 32, "a gate|up block's 32 outputs are one group");
+  static_assert(!ROPE || RH % 2 == 0, "a rope tile: R / 2 rows of each half of a head");
   static_assert(!MOE || (ST >= 1 && ST <= 4), "an entry row: quantized activations staged from memory");
   extern __shared__ __align__(16) unsigned char smem[];
-  const int groups = cols / 32;
+  const int groups = cols / GS, units = cols / 32;
   if constexpr (MOE) {
     // Grid row = MoE entry (token, slot): its expert's matrix, its
     // activation row and its output row (the whole block leaves together
@@ -158,7 +171,7 @@ __global__ __launch_bounds__(256) void k_w4a8_dec(float *out, const float *add, 
       out += (size_t)ent * moe.ld;
     }
   }
-  const int nchunks = (groups + kDecChunk - 1) / kDecChunk;
+  const int nchunks = (units + kDecChunk - 1) / kDecChunk;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int h = lane >> 5, k = lane & 31;
   // LDS: q [cols] bytes | scales [groups] | sums [groups] | waves' areas.
@@ -167,7 +180,7 @@ __global__ __launch_bounds__(256) void k_w4a8_dec(float *out, const float *add, 
   float *ssh = ash + groups;
   float *wbase = reinterpret_cast<float *>(smem + dec_act_bytes(cols));
   float *pw_lds = wbase + wave * C::WAVE_FLOATS;
-  float *fin = pw_lds + 10 * LSTR;
+  float *fin = pw_lds + 2 * C::BUF;
 
   // Wave w of W walks tiles w, w + W, ...; every wave runs the same number
   // of tiles, those past the matrix read zeros and store nothing.
@@ -177,22 +190,22 @@ __global__ __launch_bounds__(256) void k_w4a8_dec(float *out, const float *add, 
   const int rowb = cols / 2;
   // First row of the wave's tile t.  GLU: block b owns output group b of
   // silu(gate) * up, i.e. gate rows 32b.. (tile 0) and up rows
-  // rows/2 + 32b.. (tile 1), 8 per wave.  ROPE: tile u of head u / (hd/8)
-  // holds the rotation pairs (i, i + hd/2), i = 4 (u % (hd/8)) + 0..3: local
-  // rows 0..3 are i, local rows 4..7 are i + hd/2.
+  // rows/2 + 32b.. (tile 1), 8 per wave.  ROPE: tile u of head u / (hd/R)
+  // holds the rotation pairs (i, i + hd/2), i = R/2 (u % (hd/R)) + 0..: local
+  // rows 0..R/2-1 are i, the others i + hd/2.
   const int rhalf = ROPE ? rope.hd / 2 : 0;
   auto tile_row0 = [&](int t) {
     if constexpr (GLU) {
       return (t ? rows / 2 : 0) + 32 * (int)blockIdx.x + R * wave;
     } else if constexpr (ROPE) {
-      const int u = wg + t * W, per = rope.hd / 8;
-      return (u / per) * rope.hd + 4 * (u % per);
+      const int u = wg + t * W, per = rope.hd / R;
+      return (u / per) * rope.hd + RH * (u % per);
     } else {
       return (wg + t * W) * R;
     }
   };
   // Row offset of local row r (0..R-1) from tile_row0.
-  auto lrow = [&](int r) { return (ROPE && r >= 4) ? rhalf - 4 + r : r; };
+  auto lrow = [&](int r) { return (ROPE && r >= RH) ? rhalf - RH + r : r; };
   const __amdgpu_buffer_rsrc_t rc =
       __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t *>(nib), 0, rows * rowb, 0x00020000);
   const __amdgpu_buffer_rsrc_t rp =
@@ -202,13 +215,13 @@ __global__ __launch_bounds__(256) void k_w4a8_dec(float *out, const float *add, 
   // quantized row, its scales and sums), then the weight ring: loads
   // complete in issue order, so staging the activations never waits for
   // the ring.
-  // Rotation entries of the lane's pair (rope tiles: lanes 0..3, one tile
+  // Rotation entries of the lane's pair (rope tiles: lanes 0..R/2-1, one tile
   // per wave), requested first.
   int rpos = 0;
   float rcos = 0.0f, rsin = 0.0f;
   if constexpr (ROPE) {
     rpos = rope.st ? rope.st[0] : rope.pos0;
-    const int r = tile_row0(0) + min(lane, 3);
+    const int r = tile_row0(0) + min(lane, RH - 1);
     const int i = r % rope.hd;
     const bool rot = r < rows && r / rope.hd < rope.nh + rope.nkv;
     const size_t ci = (size_t)rpos * rhalf + (rot ? i : 0);
@@ -216,15 +229,15 @@ __global__ __launch_bounds__(256) void k_w4a8_dec(float *out, const float *add, 
     rsin = rope.sin_t[ci];
   }
   constexpr bool FUSED = ST == 0, QONLY = ST == 8;
-  constexpr int NP = (FUSED || QONLY) ? 4 : 1;
+  constexpr int NP = (FUSED || QONLY) ? 128 / GS : 1;  // 32 groups each: K <= 4096
   constexpr int QV = (FUSED || QONLY) ? 1 : ST;
-  float xr[NP][4], wr[NP][4];
+  float xr[NP][GS / 8], wr[NP][GS / 8];
   uint4 qv[QV];
   float av[2], sv[2];
   if constexpr (FUSED) {
-    rmsnorm_regs_load<32, NP>(nx, nw, cols, xr, wr);
+    rmsnorm_regs_load<GS, NP>(nx, nw, cols, xr, wr);
   } else if constexpr (QONLY) {
-    xr_only<32, NP>(nx, cols, xr);
+    xr_only<GS, NP>(nx, cols, xr);
   } else {
     const __amdgpu_buffer_rsrc_t rq =
         __builtin_amdgcn_make_buffer_rsrc(const_cast<int8_t *>(q_split), 0, cols, 0x00020000);
@@ -248,15 +261,15 @@ __global__ __launch_bounds__(256) void k_w4a8_dec(float *out, const float *add, 
   int lt = 0, lch = 0;
   auto load = [&](u32x4 (&c)[IPL], uint32_t (&p)[IPL]) {
     const int row = tile_row0(lt) + h;  // local row h; item i adds lrow(2i) rows
-    const int g = lch * kDecChunk + k;
-    uint32_t vc = (uint32_t)row * rowb + g * 16;
-    uint32_t vp = ((uint32_t)row * groups + g) * 4;
-    // Past the last iteration, and on the lanes past the groups of a
+    const int un = lch * kDecChunk + k;
+    uint32_t vc = (uint32_t)row * rowb + un * 16;
+    uint32_t vp = ((uint32_t)row * groups + un / LPG) * 4;
+    // Past the last iteration, and on the lanes past the units of a
     // partial last chunk: zeros without a memory access.  Zero codes and
     // parameters give +0 or -0 products, which leave a chain unchanged (a
     // chain starts at +0 and a sum of floats is -0 only when both terms
     // are).
-    if (lt >= tiles_per_wave || g >= groups) {
+    if (lt >= tiles_per_wave || un >= units) {
       vc = 0x80000000u;  // past num_records
       vp = 0x80000000u;
     }
@@ -284,9 +297,9 @@ __global__ __launch_bounds__(256) void k_w4a8_dec(float *out, const float *add, 
 
   // Stage the activations in LDS while the ring fills.
   if constexpr (FUSED) {
-    rmsnorm_quant_regs<32, NP>(xr, wr, cols, eps, wbase, qsh, 32, ash, ssh);
+    rmsnorm_quant_regs<GS, NP>(xr, wr, cols, eps, wbase, qsh, GS, ash, ssh);
   } else if constexpr (QONLY) {
-    quant_regs<32, NP>(xr, cols, qsh, 32, ash, ssh);
+    quant_regs<GS, NP>(xr, cols, qsh, GS, ash, ssh);
   } else {
     // Unconditional stores to the clamped slots (threads past the row
     // rewrite the last slot with the value already there): a conditional
@@ -302,20 +315,21 @@ __global__ __launch_bounds__(256) void k_w4a8_dec(float *out, const float *add, 
   __syncthreads();
 
   float acc = 0.0f, gate_v = 0.0f, up_v = 0.0f;
-  // Chain lane: row crow, chain cl (lanes past the 5R chains re-read chain
-  // 4 and their sums are never used).
-  const int crow = lane % R, cl = min(lane / R, 4);
-  const bool chain_lane = lane < 5 * R;
-  const int cbase = cl * LSTR + crow * kDecRowStride;
+  // Chain lane: the run it sums (lanes past the NC * R chains re-read the
+  // last one and their sums are never used).
+  const bool chain_lane = lane < NC * R;
+  const int cbase = min(lane, NC * R - 1) * STR;
+  // Group of the lane's unit in the chunk, and the unit's place in it.
+  const int kg = k / LPG, ku = k % LPG;
   // Activations of the iteration's chunk (read one iteration ahead).
   uint4 q0, q1;
   float as, xsum;
   auto read_act = [&](int ch) {
-    const int gq = min(ch * kDecChunk + k, groups - 1);
-    q0 = *reinterpret_cast<const uint4 *>(qsh + gq * 32);
-    q1 = *reinterpret_cast<const uint4 *>(qsh + gq * 32 + 16);
-    as = ash[gq];
-    xsum = ssh[gq];
+    const int un = min(ch * kDecChunk + k, units - 1);
+    q0 = *reinterpret_cast<const uint4 *>(qsh + un * 32);
+    q1 = *reinterpret_cast<const uint4 *>(qsh + un * 32 + 16);
+    as = ash[un / LPG];
+    xsum = ssh[un / LPG];
   };
   // End of tile t: the row sums from the chain values in acc.
   auto finish = [&](int t) {
@@ -325,17 +339,19 @@ __global__ __launch_bounds__(256) void k_w4a8_dec(float *out, const float *add, 
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
     const int row = tile_row0(t) + lrow(lane);
     if (lane < R && row < rows) {
-      // hsum8 of (f0, f1, f2, f3, 0, 0, 0, 0) in the _mm256 order.
-      const float f0 = fin[lane], f1 = fin[R + lane], f2 = fin[2 * R + lane], f3 = fin[3 * R + lane];
-      const float zero = 0.0f;
-      const float v = ((f0 + zero) + (f1 + zero)) + ((f2 + zero) + (f3 + zero)) + fin[4 * R + lane];
+      // hsum8 in the _mm256 order (lanes 4..7 are +0 at group 32).
+      float f[8];
+#pragma unroll
+      for (int l = 0; l < 8; ++l) f[l] = l < NL ? fin[C::run(l, lane)] : 0.0f;
+      const float v =
+          (((f[0] + f[4]) + (f[1] + f[5])) + ((f[2] + f[6]) + (f[3] + f[7]))) + fin[C::run(NL, lane)];
       if constexpr (GLU) {
         if (t == 0)
           gate_v = v;
         else
           up_v = v;
       } else if constexpr (ROPE) {
-        fin[40 + lane] = v;
+        fin[NC * R + lane] = v;
       } else {
         out[row] = add ? add[row] + v : v;
       }
@@ -344,8 +360,9 @@ __global__ __launch_bounds__(256) void k_w4a8_dec(float *out, const float *add, 
       __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
       __builtin_amdgcn_wave_barrier();
       __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-      if (lane < 4 && tile_row0(t) < rows)
-        rope_store_pair(rope, out, tile_row0(t) + lane, rpos, rcos, rsin, fin[40 + lane], fin[44 + lane]);
+      if (lane < RH && tile_row0(t) < rows)
+        rope_store_pair(rope, out, tile_row0(t) + lane, rpos, rcos, rsin, fin[NC * R + lane],
+                        fin[NC * R + RH + lane]);
     }
   };
 
@@ -353,9 +370,9 @@ __global__ __launch_bounds__(256) void k_w4a8_dec(float *out, const float *add, 
   // LDS buffer it & 1 while the chain lanes add chunk it - 1's (read from
   // LDS at the end of iteration it - 1), so a chain's dependent adds issue
   // between independent product instructions.
-  float4 cv[8];
+  float cv[GPC];
 #pragma unroll
-  for (int u = 0; u < 8; ++u) cv[u] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+  for (int u = 0; u < GPC; ++u) cv[u] = 0.0f;
   int ct = 0, cch = 0;   // tile and chunk of the iteration
   int pt = 0, pch = -1;  // tile and chunk of the pending chain values (none yet)
   read_act(0);
@@ -364,10 +381,10 @@ __global__ __launch_bounds__(256) void k_w4a8_dec(float *out, const float *add, 
     for (int j = 0; j < D; ++j) {
       const int it = it0 + j;
       if (it < it_total) {
-        float *pb = pw_lds + (it & 1) * (5 * LSTR);
+        float *pb = pw_lds + (it & 1) * C::BUF;
         acc = pch == 0 ? 0.0f : acc;  // a tile's chains start at its first chunk
-        // Products of the lane's items, block-major in 8 slots of IPL / 2
-        // block dots each, and in every slot 4 of the pending chain's adds:
+        // Products of the lane's items, block-major in 8 slots of block
+        // dots, and in every slot an eighth of the pending chain's adds:
         // a dependent add takes several issue slots to complete, and the
         // scheduling barriers keep the independent product work between
         // consecutive adds.
@@ -376,23 +393,39 @@ __global__ __launch_bounds__(256) void k_w4a8_dec(float *out, const float *add, 
         for (int i = 0; i < IPL; ++i) {
           const uint32_t pw = ring_p[j][i];
           cs[i] = dec_f16(pw & 0xFFFF) * as;
-          pb[4 * LSTR + (2 * i + h) * kDecRowStride + k] = dec_f16(pw >> 16) * xsum;
+          // The lanes of one group write the same zero term.
+          pb[C::run(NL, 2 * i) * STR + (C::run(0, 1) - C::run(0, 0)) * STR * h + kg] = dec_f16(pw >> 16) * xsum;
         }
+        auto dot = [&](int b, int i) {
+          const u32x4 cw = ring_c[j][i];
+          const uint32_t code = b == 0 ? cw.x : b == 1 ? cw.y : b == 2 ? cw.z : cw.w;
+          const uint4 qq = b < 2 ? q0 : q1;
+          return dec_block_dot(code, (b & 1) ? qq.z : qq.x, (b & 1) ? qq.w : qq.y);
+        };
+        // Product of lane sum S for chain l of item i's row.
+        auto put = [&](int l, int i, int S) {
+          pb[(C::run(0, 2 * i) + (C::run(0, 1) - C::run(0, 0)) * h + (C::run(1, 0) - C::run(0, 0)) * l) * STR + kg] =
+              (float)S * cs[i];
+        };
+        constexpr int NE = (GS == 128 ? 2 : 4) * IPL;  // products per lane
 #pragma unroll
         for (int sl = 0; sl < 8; ++sl) {
 #pragma unroll
-          for (int e = sl * IPL / 2; e < (sl + 1) * IPL / 2; ++e) {
+          for (int e = sl * NE / 8; e < (sl + 1) * NE / 8; ++e) {
             const int b = e / IPL, i = e % IPL;  // block b of item i
-            const u32x4 cw = ring_c[j][i];
-            const uint32_t code = b == 0 ? cw.x : b == 1 ? cw.y : b == 2 ? cw.z : cw.w;
-            const uint4 qq = b < 2 ? q0 : q1;
-            const int sb = dec_block_dot(code, (b & 1) ? qq.z : qq.x, (b & 1) ? qq.w : qq.y);
-            pb[b * LSTR + (2 * i + h) * kDecRowStride + k] = (float)sb * cs[i];
+            if constexpr (GS == 32) {
+              put(b, i, dot(b, i));
+            } else if constexpr (GS == 64) {
+              put(4 * ku + b, i, dot(b, i));
+            } else {
+              const int s0 = dot(b, i), s2 = dot(b + 2, i);
+              const int t0 = s0 + __builtin_amdgcn_update_dpp(0, s0, kDppXor2, 0xF, 0xF, true);
+              const int t2 = s2 + __builtin_amdgcn_update_dpp(0, s2, kDppXor2, 0xF, 0xF, true);
+              put(4 * (ku & 1) + (ku & 2) + b, i, (ku & 2) ? t2 : t0);
+            }
           }
-          acc = acc + cv[sl].x;
-          acc = acc + cv[sl].y;
-          acc = acc + cv[sl].z;
-          acc = acc + cv[sl].w;
+#pragma unroll
+          for (int e = sl * GPC / 8; e < (sl + 1) * GPC / 8; ++e) acc = acc + cv[e];
           __builtin_amdgcn_sched_barrier(0);
         }
         if (pch == nchunks - 1) finish(pt);
@@ -410,7 +443,13 @@ __global__ __launch_bounds__(256) void k_w4a8_dec(float *out, const float *add, 
         read_act(cch);
         const float4 *pc = reinterpret_cast<const float4 *>(pb + cbase);
 #pragma unroll
-        for (int u = 0; u < 8; ++u) cv[u] = pc[u];
+        for (int u = 0; u < GPC / 4; ++u) {
+          const float4 p4 = pc[u];
+          cv[4 * u] = p4.x;
+          cv[4 * u + 1] = p4.y;
+          cv[4 * u + 2] = p4.z;
+          cv[4 * u + 3] = p4.w;
+        }
       }
       load(ring_c[j], ring_p[j]);
       __builtin_amdgcn_sched_barrier(0);
@@ -419,12 +458,7 @@ __global__ __launch_bounds__(256) void k_w4a8_dec(float *out, const float *add, 
   // The last chunk's chain.
   acc = pch == 0 ? 0.0f : acc;
 #pragma unroll
-  for (int u = 0; u < 8; ++u) {
-    acc = acc + cv[u].x;
-    acc = acc + cv[u].y;
-    acc = acc + cv[u].z;
-    acc = acc + cv[u].w;
-  }
+  for (int u = 0; u < GPC; ++u) acc = acc + cv[u];
   if (pch == nchunks - 1) finish(pt);
   if constexpr (GLU) {
     // silu_mul_inplace (layers.rs:850-883) of the block's 32 outputs and
@@ -456,14 +490,14 @@ __global__ __launch_bounds__(256) void k_w4a8_dec(float *out, const float *add, 
   }
 }
 
-template <int R, int D, int ST>
+template <int GS, int R, int D, int ST>
 void launch_dec_t(float *out, const float *add, const uint8_t *nib, const uint8_t *params, const int8_t *q_split,
                   const float *scales, const float *sums, int rows, int cols, const float *nx, const float *nw,
                   float eps, int blocks, hipStream_t s) {
-  const size_t smem = dec_smem<R>(cols, ST == 0);  // the norm's row scratch
+  const size_t smem = dec_smem<GS, R>(cols, ST == 0);  // the norm's row scratch
   static size_t configured = 0;
   if (smem > configured) {
-    (void)hipFuncSetAttribute(reinterpret_cast<const void *>(&k_w4a8_dec<R, D, ST, kEpiPlain>),
+    (void)hipFuncSetAttribute(reinterpret_cast<const void *>(&k_w4a8_dec<GS, R, D, ST, kEpiPlain>),
                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
     configured = smem;
   }
@@ -472,50 +506,51 @@ void launch_dec_t(float *out, const float *add, const uint8_t *nib, const uint8_
   blocks = std::max(1, std::min(blocks, 1024));
   const int waves = blocks * kDecWaves;
   const int per_wave = (tiles + waves - 1) / waves;
-  hipLaunchKernelGGL((k_w4a8_dec<R, D, ST, kEpiPlain>), dim3(blocks), dim3(256), smem, s, out, add, nib, params,
+  hipLaunchKernelGGL((k_w4a8_dec<GS, R, D, ST, kEpiPlain>), dim3(blocks), dim3(256), smem, s, out, add, nib, params,
                      q_split, scales, sums, rows, cols, per_wave, nx, nw, eps, DecRope{}, DecMoe{});
 }
 
-template <int R, int D>
+template <int GS, int R, int D>
 void launch_dec_rd(float *out, const float *add, const uint8_t *nib, const uint8_t *params, const int8_t *q_split,
                    const float *scales, const float *sums, int rows, int cols, const float *nx, const float *nw,
                    float eps, int blocks, hipStream_t s) {
   if (nx && nw)
-    launch_dec_t<R, D, 0>(out, add, nib, params, q_split, scales, sums, rows, cols, nx, nw, eps, blocks, s);
+    launch_dec_t<GS, R, D, 0>(out, add, nib, params, q_split, scales, sums, rows, cols, nx, nw, eps, blocks, s);
   else if (nx)
-    launch_dec_t<R, D, 8>(out, add, nib, params, q_split, scales, sums, rows, cols, nx, nw, eps, blocks, s);
+    launch_dec_t<GS, R, D, 8>(out, add, nib, params, q_split, scales, sums, rows, cols, nx, nw, eps, blocks, s);
   else if (cols <= 16 * 256)
-    launch_dec_t<R, D, 1>(out, add, nib, params, q_split, scales, sums, rows, cols, nx, nw, eps, blocks, s);
+    launch_dec_t<GS, R, D, 1>(out, add, nib, params, q_split, scales, sums, rows, cols, nx, nw, eps, blocks, s);
   else if (cols <= 16 * 512)
-    launch_dec_t<R, D, 2>(out, add, nib, params, q_split, scales, sums, rows, cols, nx, nw, eps, blocks, s);
+    launch_dec_t<GS, R, D, 2>(out, add, nib, params, q_split, scales, sums, rows, cols, nx, nw, eps, blocks, s);
   else
-    launch_dec_t<R, D, 4>(out, add, nib, params, q_split, scales, sums, rows, cols, nx, nw, eps, blocks, s);
+    launch_dec_t<GS, R, D, 4>(out, add, nib, params, q_split, scales, sums, rows, cols, nx, nw, eps, blocks, s);
 }
 
-template <int R, int D, int ST>
+template <int GS, int R, int D, int ST>
 void launch_dec_moe_t(float *out, const DecMoe &moe, const int8_t *q_split, const float *scales, const float *sums,
                       int rows, int cols, int blocks, int entries, hipStream_t s) {
-  const size_t smem = dec_smem<R>(cols, false);
+  const size_t smem = dec_smem<GS, R>(cols, false);
   static size_t configured = 0;
   if (smem > configured) {
-    (void)hipFuncSetAttribute(reinterpret_cast<const void *>(&k_w4a8_dec<R, D, ST, kEpiMoe>),
+    (void)hipFuncSetAttribute(reinterpret_cast<const void *>(&k_w4a8_dec<GS, R, D, ST, kEpiMoe>),
                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
     configured = smem;
   }
   const int tiles = (rows + R - 1) / R, waves = blocks * kDecWaves;
   const int per_wave = (tiles + waves - 1) / waves;
-  hipLaunchKernelGGL((k_w4a8_dec<R, D, ST, kEpiMoe>), dim3(blocks, entries), dim3(256), smem, s, out, nullptr,
+  hipLaunchKernelGGL((k_w4a8_dec<GS, R, D, ST, kEpiMoe>), dim3(blocks, entries), dim3(256), smem, s, out, nullptr,
                      nullptr, nullptr, q_split, scales, sums, rows, cols, per_wave, nullptr, nullptr, 0.0f,
                      DecRope{}, moe);
 }
 
 }  // namespace
 
-// Group 32, whole groups, K staged in LDS, byte offsets of every tile the
+// Whole groups of 32, 64 or 128, K staged in LDS, byte offsets of every tile the
 // waves address (including the zero-reading ones past the matrix) inside
 // 31 bits.
 bool w4a8_dec_path(int rows, int cols, int gs) {
-  if (gs != 32 || rows <= 0 || cols % 32 != 0 || cols / 32 > kDecMaxGroups || cols < 256) return false;
+  if ((gs != 32 && gs != 64 && gs != 128) || rows <= 0 || cols % gs != 0 || cols / 32 > kDecMaxUnits || cols < 256)
+    return false;
   const long long span = ((long long)rows + 4096LL * 12) * (cols / 2);
   return span < (1LL << 31) - (1LL << 20);
 }
@@ -548,15 +583,28 @@ bool launch_w4a8_dec(float *out, const float *add, const uint8_t *nib, const uin
                      const float *nw, float eps, hipStream_t s, int variant, int blocks) {
   if (!w4a8_dec_path(rows, cols, gs)) return false;
   if (nx && !w4a8_dec_fused_ok(cols)) return false;
+  // Groups of 64 and 128 (nine chains a row): four-row tiles, a ring of four
+  // chunks, one tile per wave up to 16384 rows.  Against the tiled VALU
+  // kernel they took before (with the norm and quantization launches of their
+  // own): a 4096-wide layer and head at group 128, 1000 positions, 211 -> 170
+  // us.
+  if (gs != 32) {
+    if (blocks == 0 && rows >= 16384) blocks = 512;
+    if (gs == 64)
+      launch_dec_rd<64, 4, 4>(out, add, nib, params, q_split, scales, sums, rows, cols, nx, nw, eps, blocks, s);
+    else
+      launch_dec_rd<128, 4, 4>(out, add, nib, params, q_split, scales, sums, rows, cols, nx, nw, eps, blocks, s);
+    return true;
+  }
   if (variant == 0) dec_choice(rows, nw != nullptr, variant, blocks);
   switch (variant) {
-    case 1: launch_dec_rd<4, 6>(out, add, nib, params, q_split, scales, sums, rows, cols, nx, nw, eps, blocks, s); break;
-    case 2: launch_dec_rd<8, 3>(out, add, nib, params, q_split, scales, sums, rows, cols, nx, nw, eps, blocks, s); break;
-    case 3: launch_dec_rd<12, 2>(out, add, nib, params, q_split, scales, sums, rows, cols, nx, nw, eps, blocks, s); break;
-    case 4: launch_dec_rd<4, 4>(out, add, nib, params, q_split, scales, sums, rows, cols, nx, nw, eps, blocks, s); break;
-    case 5: launch_dec_rd<8, 4>(out, add, nib, params, q_split, scales, sums, rows, cols, nx, nw, eps, blocks, s); break;
-    case 6: launch_dec_rd<12, 3>(out, add, nib, params, q_split, scales, sums, rows, cols, nx, nw, eps, blocks, s); break;
-    default: launch_dec_rd<8, 3>(out, add, nib, params, q_split, scales, sums, rows, cols, nx, nw, eps, blocks, s); break;
+    case 1: launch_dec_rd<32, 4, 6>(out, add, nib, params, q_split, scales, sums, rows, cols, nx, nw, eps, blocks, s); break;
+    case 2: launch_dec_rd<32, 8, 3>(out, add, nib, params, q_split, scales, sums, rows, cols, nx, nw, eps, blocks, s); break;
+    case 3: launch_dec_rd<32, 12, 2>(out, add, nib, params, q_split, scales, sums, rows, cols, nx, nw, eps, blocks, s); break;
+    case 4: launch_dec_rd<32, 4, 4>(out, add, nib, params, q_split, scales, sums, rows, cols, nx, nw, eps, blocks, s); break;
+    case 5: launch_dec_rd<32, 8, 4>(out, add, nib, params, q_split, scales, sums, rows, cols, nx, nw, eps, blocks, s); break;
+    case 6: launch_dec_rd<32, 12, 3>(out, add, nib, params, q_split, scales, sums, rows, cols, nx, nw, eps, blocks, s); break;
+    default: launch_dec_rd<32, 8, 3>(out, add, nib, params, q_split, scales, sums, rows, cols, nx, nw, eps, blocks, s); break;
   }
   return true;
 }
@@ -575,12 +623,21 @@ bool launch_w4a8_dec_moe(float *out, const DecMoe &moe, const int8_t *q_split, c
   blocks = std::min(blocks, full);
   // A ring of two chunks (four: 11.0 -> 9.6 us per OLMoE-shaped launch,
   // decode and verify averaged).
-  if (cols <= 16 * 256)
-    launch_dec_moe_t<4, 2, 1>(out, moe, q_split, scales, sums, rows, cols, blocks, max_entries, s);
-  else if (cols <= 16 * 512)
-    launch_dec_moe_t<4, 2, 2>(out, moe, q_split, scales, sums, rows, cols, blocks, max_entries, s);
+  auto go = [&](auto g) {
+    constexpr int GS = decltype(g)::value;
+    if (cols <= 16 * 256)
+      launch_dec_moe_t<GS, 4, 2, 1>(out, moe, q_split, scales, sums, rows, cols, blocks, max_entries, s);
+    else if (cols <= 16 * 512)
+      launch_dec_moe_t<GS, 4, 2, 2>(out, moe, q_split, scales, sums, rows, cols, blocks, max_entries, s);
+    else
+      launch_dec_moe_t<GS, 4, 2, 4>(out, moe, q_split, scales, sums, rows, cols, blocks, max_entries, s);
+  };
+  if (gs == 32)
+    go(std::integral_constant<int, 32>{});
+  else if (gs == 64)
+    go(std::integral_constant<int, 64>{});
   else
-    launch_dec_moe_t<4, 2, 4>(out, moe, q_split, scales, sums, rows, cols, blocks, max_entries, s);
+    go(std::integral_constant<int, 128>{});
   return true;
 }
 
@@ -591,19 +648,19 @@ bool launch_w4a8_dec_moe(float *out, const DecMoe &moe, const int8_t *q_split, c
 // averaged).
 bool launch_w4a8_dec_moe_glu(const DecMoe &moe, const int8_t *q_split, const float *scales, const float *sums,
                              int rows, int cols, int gs, int max_entries, hipStream_t s) {
-  if (!w4a8_dec_path(rows, cols, gs) || rows % 64 != 0 || max_entries <= 0 || max_entries > 65535 ||
+  if (gs != 32 || !w4a8_dec_path(rows, cols, gs) || rows % 64 != 0 || max_entries <= 0 || max_entries > 65535 ||
       cols > 16 * 1024 || !moe.qo || !moe.so || !moe.uo)
     return false;
-  const size_t smem = dec_smem<8>(cols, false);
+  const size_t smem = dec_smem<32, 8>(cols, false);
   auto go = [&](auto st) {
     constexpr int ST = decltype(st)::value;
     static size_t configured = 0;
     if (smem > configured) {
-      (void)hipFuncSetAttribute(reinterpret_cast<const void *>(&k_w4a8_dec<8, 2, ST, kEpiMoeGlu>),
+      (void)hipFuncSetAttribute(reinterpret_cast<const void *>(&k_w4a8_dec<32, 8, 2, ST, kEpiMoeGlu>),
                                 hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
       configured = smem;
     }
-    hipLaunchKernelGGL((k_w4a8_dec<8, 2, ST, kEpiMoeGlu>), dim3(rows / 64, max_entries), dim3(256), smem, s,
+    hipLaunchKernelGGL((k_w4a8_dec<32, 8, 2, ST, kEpiMoeGlu>), dim3(rows / 64, max_entries), dim3(256), smem, s,
                        nullptr, nullptr, nullptr, nullptr, q_split, scales, sums, rows, cols, 2, nullptr, nullptr,
                        0.0f, DecRope{}, moe);
   };
@@ -622,15 +679,15 @@ bool launch_w4a8_dec_moe_glu(const DecMoe &moe, const int8_t *q_split, const flo
 // 16.3 us and qkv 10.1 -> 9.2 us (one chunk: 18.4 and 10.4).
 bool launch_w4a8_glu1(const uint8_t *nib, const uint8_t *params, const float *x, const float *norm_w, float eps,
                       int rows, int cols, int gs, int8_t *q_out, float *scale_out, float *sum_out, hipStream_t s) {
-  if (!w4a8_dec_path(rows, cols, gs) || !w4a8_dec_fused_ok(cols) || rows % 64 != 0) return false;
-  const size_t smem = dec_smem<8>(cols, true);
+  if (gs != 32 || !w4a8_dec_path(rows, cols, gs) || !w4a8_dec_fused_ok(cols) || rows % 64 != 0) return false;
+  const size_t smem = dec_smem<32, 8>(cols, true);
   static size_t configured = 0;
   if (smem > configured) {
-    (void)hipFuncSetAttribute(reinterpret_cast<const void *>(&k_w4a8_dec<8, 2, 0, kEpiGlu>),
+    (void)hipFuncSetAttribute(reinterpret_cast<const void *>(&k_w4a8_dec<32, 8, 2, 0, kEpiGlu>),
                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
     configured = smem;
   }
-  hipLaunchKernelGGL((k_w4a8_dec<8, 2, 0, kEpiGlu>), dim3(rows / 64), dim3(256), smem, s, nullptr, nullptr, nib,
+  hipLaunchKernelGGL((k_w4a8_dec<32, 8, 2, 0, kEpiGlu>), dim3(rows / 64), dim3(256), smem, s, nullptr, nullptr, nib,
                      params, q_out, scale_out, sum_out, rows, cols, 2, x, norm_w, eps, DecRope{}, DecMoe{});
   return true;
 }
@@ -640,16 +697,25 @@ bool launch_w4a8_qkv_rope1(float *out, const uint8_t *nib, const uint8_t *params
                            hipStream_t s) {
   if (!w4a8_dec_path(rows, cols, gs) || !w4a8_dec_fused_ok(cols)) return false;
   if (rope.hd % 8 != 0 || rows != (rope.nh + 2 * rope.nkv) * rope.hd) return false;
-  const size_t smem = dec_smem<8>(cols, true);
-  static size_t configured = 0;
-  if (smem > configured) {
-    (void)hipFuncSetAttribute(reinterpret_cast<const void *>(&k_w4a8_dec<8, 2, 0, kEpiRope>),
-                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
-    configured = smem;
-  }
-  const int tiles = rows / 8, blocks = (tiles + kDecWaves - 1) / kDecWaves;
-  hipLaunchKernelGGL((k_w4a8_dec<8, 2, 0, kEpiRope>), dim3(blocks), dim3(256), smem, s, out, nullptr, nib, params,
-                     nullptr, nullptr, nullptr, rows, cols, 1, x, norm_w, eps, rope, DecMoe{});
+  auto go = [&](auto g, auto r) {
+    constexpr int GS = decltype(g)::value, R = decltype(r)::value;
+    const size_t smem = dec_smem<GS, R>(cols, true);
+    static size_t configured = 0;
+    if (smem > configured) {
+      (void)hipFuncSetAttribute(reinterpret_cast<const void *>(&k_w4a8_dec<GS, R, 2, 0, kEpiRope>),
+                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
+      configured = smem;
+    }
+    const int tiles = rows / R, blocks = (tiles + kDecWaves - 1) / kDecWaves;
+    hipLaunchKernelGGL((k_w4a8_dec<GS, R, 2, 0, kEpiRope>), dim3(blocks), dim3(256), smem, s, out, nullptr, nib,
+                       params, nullptr, nullptr, nullptr, rows, cols, 1, x, norm_w, eps, rope, DecMoe{});
+  };
+  if (gs == 32)
+    go(std::integral_constant<int, 32>{}, std::integral_constant<int, 8>{});
+  else if (gs == 64)
+    go(std::integral_constant<int, 64>{}, std::integral_constant<int, 4>{});
+  else
+    go(std::integral_constant<int, 128>{}, std::integral_constant<int, 4>{});
   return true;
 }
 

@@ -1431,7 +1431,8 @@ void launch_quantize(const float *x, int m, int k, int gs, int8_t *q_nat, int8_t
 }
 
 bool w4a8_norm1_path(int rows, int cols, int gs) {
-  return gs == 32 && rows > 0 && cols % 32 == 0 && cols / 32 <= 128 && cols >= 256;
+  if (gs != 32) return w4a8_dec_path(rows, cols, gs) && w4a8_dec_fused_ok(cols);
+  return rows > 0 && cols % 32 == 0 && cols / 32 <= 128 && cols >= 256;
 }
 
 bool launch_w4a8_norm1(float *out, const float *add, const uint8_t *nib, const uint8_t *params, const float *x,

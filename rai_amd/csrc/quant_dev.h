@@ -382,7 +382,7 @@ __device__ __forceinline__ void rmsnorm_quant_regs(const float (&xr)[P][GS / 8],
     }
   }
   __syncthreads();
-  const float inv = rmsnorm_inv_t<P>(xs, n, eps);
+  const float inv = rmsnorm_inv_t<P * GS / 32>(xs, n, eps);
 #pragma unroll
   for (int p = 0; p < P; ++p) {
     const int g = p * 32 + tid / 8;

@@ -112,3 +112,38 @@ def test_tied_logits_of_a_batch(rai, ora, m):
     h = np.random.default_rng(m).normal(0.0, 1.0, (m, 256)).astype(np.float32)
     got, want = gm.hidden_to_logits_batch(h, m), om.hidden_to_logits_batch(h, m)
     assert np.array_equal(_bits(got).reshape(-1), _bits(want).reshape(-1))
+
+
+# One token: the GEMV that quantizes its row (K <= 4096) or takes it quantized;
+# K under a chunk of 1024 columns, one past it, several, with odd group counts.
+@pytest.mark.parametrize("gs,cols", [(32, 256), (32, 1056), (32, 4096), (32, 4128), (64, 256), (64, 1088), (64, 4096),
+                                     (64, 6976), (128, 256), (128, 1152), (128, 3968), (128, 4224), (128, 14336)])
+@pytest.mark.parametrize("rows", [1, 6, 17, 530])
+def test_one_token_every_group_size(rai, ora, gs, cols, rows):
+    nib, params, x = gemv_operands(rows, cols, 1, gs, seed=rows + cols)
+    for scale in (1.0, 1e-39, 1e30):
+        xs = (x.reshape(-1) * np.float32(scale)).astype(np.float32)
+        want = ora.w4a8_matmul(nib, params, xs, rows, cols, 1, gs)
+        dev = rai.DeviceArray.from_host
+        for name in ("rai_w4a8_matmul_dev", "rai_w4a8_matmul_noalloc_dev"):
+            got = _call(rai, name, rai.DeviceArray(4 * rows), dev(nib), dev(params), dev(xs), rows, cols, 1, gs)
+            assert np.array_equal(_bits(got), _bits(want).reshape(-1)), (name, scale)
+
+
+@pytest.mark.parametrize("gs", [32, 64, 128])
+@pytest.mark.parametrize("hidden,heads,kv,hd,ffn,experts", [(256, 4, 2, 64, 384, 0), (1152, 9, 3, 128, 1280, 0),
+                                                            (512, 8, 8, 64, 256, 8)])
+def test_decode_steps_every_group_size(rai, ora, gs, hidden, heads, kv, hd, ffn, experts):
+    """One-token forward passes (fused norm, rope and quantization) and the
+    head, token after token on one cache."""
+    img = rai.synth_model(hidden, 2, heads, kv, hd, ffn, 400, 64, group_size=gs, num_experts=experts,
+                          experts_per_token=min(experts, 3), seed=gs + hidden)
+    gm, om = rai.RaiModel.from_bytes(img), ora.Model(img, 0)
+    gk, ok = gm.create_kv_cache(64), om.create_kv(64)
+    r = np.random.default_rng(hidden)
+    for pos in range(3):
+        h = r.normal(0.0, 1.0, (1, hidden)).astype(np.float32)
+        got, want = gm.forward_batch(h, [pos], gk), om.forward_batch(h, np.array([pos]), ok)
+        assert np.array_equal(_bits(got).reshape(-1), _bits(want).reshape(-1)), pos
+        gl, ol = gm.hidden_to_logits_batch(got, 1), om.hidden_to_logits_batch(want, 1)
+        assert np.array_equal(_bits(gl).reshape(-1), _bits(ol).reshape(-1)), pos
