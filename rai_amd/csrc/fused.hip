@@ -156,7 +156,7 @@ __global__ __launch_bounds__(256) void k_silu_quant(float *__restrict__ gate,
   int8_t *qs = q_split + (size_t)t * n;
   int8_t *qn = q_nat ? q_nat + (size_t)t * n : nullptr;
   quantize_group8<NB>(v, j, col0, ok, qs, qn, scales + (size_t)t * groups + g,
-                      sums + (size_t)t * groups + g, qa ? qa4_slot(qa, t, ok ? g : 0, groups) : nullptr);
+                      sums + (size_t)t * groups + g, qa ? qa_slot_of<GS>(qa, t, ok ? g : 0, groups) : nullptr);
 }
 
 // Per-group quantization of m rows of n (quantize_input_split +
@@ -181,7 +181,7 @@ __global__ __launch_bounds__(256) void k_quant(const float *__restrict__ x, int 
   int8_t *qs = q_split + (size_t)t * n;
   int8_t *qn = q_nat ? q_nat + (size_t)t * n : nullptr;
   quantize_group8<NB>(v, j, col0, ok, qs, qn, scales + (size_t)t * groups + g,
-                      sums + (size_t)t * groups + g, qa ? qa4_slot(qa, t, ok ? g : 0, groups) : nullptr);
+                      sums + (size_t)t * groups + g, qa ? qa_slot_of<GS>(qa, t, ok ? g : 0, groups) : nullptr);
 }
 
 // -------------------------------------------------------------- attention --
@@ -1673,9 +1673,9 @@ void launch_norm_quant(const float *x, const float *w, float *normed, int m, int
   if (gs == 32)
     launch_norm_quant_t<32>(x, w, normed, m, n, eps, q_split, q_nat, scales, sums, s, qa);
   else if (gs == 64)
-    launch_norm_quant_t<64>(x, w, normed, m, n, eps, q_split, q_nat, scales, sums, s);
+    launch_norm_quant_t<64>(x, w, normed, m, n, eps, q_split, q_nat, scales, sums, s, qa);
   else
-    launch_norm_quant_t<128>(x, w, normed, m, n, eps, q_split, q_nat, scales, sums, s);
+    launch_norm_quant_t<128>(x, w, normed, m, n, eps, q_split, q_nat, scales, sums, s, qa);
 }
 
 void launch_quant(const float *x, int m, int n, int gs, int8_t *q_split, int8_t *q_nat,
@@ -1684,9 +1684,9 @@ void launch_quant(const float *x, int m, int n, int gs, int8_t *q_split, int8_t 
   if (gs == 32)
     hipLaunchKernelGGL(k_quant<32>, grid, dim3(256), 0, s, x, n, q_split, q_nat, scales, sums, qa);
   else if (gs == 64)
-    hipLaunchKernelGGL(k_quant<64>, grid, dim3(256), 0, s, x, n, q_split, q_nat, scales, sums, nullptr);
+    hipLaunchKernelGGL(k_quant<64>, grid, dim3(256), 0, s, x, n, q_split, q_nat, scales, sums, qa);
   else
-    hipLaunchKernelGGL(k_quant<128>, grid, dim3(256), 0, s, x, n, q_split, q_nat, scales, sums, nullptr);
+    hipLaunchKernelGGL(k_quant<128>, grid, dim3(256), 0, s, x, n, q_split, q_nat, scales, sums, qa);
 }
 
 void launch_silu_quant(float *gate, const float *up, int m, int n, int ld, int gs,
@@ -1695,9 +1695,9 @@ void launch_silu_quant(float *gate, const float *up, int m, int n, int ld, int g
   if (gs == 32)
     launch_silu_quant_t<32>(gate, up, m, n, ld, q_split, q_nat, scales, sums, s, qa);
   else if (gs == 64)
-    launch_silu_quant_t<64>(gate, up, m, n, ld, q_split, q_nat, scales, sums, s, nullptr);
+    launch_silu_quant_t<64>(gate, up, m, n, ld, q_split, q_nat, scales, sums, s, qa);
   else
-    launch_silu_quant_t<128>(gate, up, m, n, ld, q_split, q_nat, scales, sums, s, nullptr);
+    launch_silu_quant_t<128>(gate, up, m, n, ld, q_split, q_nat, scales, sums, s, qa);
 }
 
 // Floats per score row: the positions, then a slot for the softmax's

@@ -21,8 +21,8 @@ void launch_quantize(const float *x, int m, int k, int gs, int8_t *q_nat, int8_t
 // `add` (may be null, may equal `out`): a residual [m][rows] added to each
 // output, out = add + matmul (the reference's vec_add after o_proj/down,
 // layers.rs:503-531, fused into the epilogue).
-// `qa` (may be null): the activations packed by launch_qa_pack, which
-// enables the matrix-core kernel for 2..kMfmaMaxTokens tokens at group 32.
+// `qa` (may be null): the activations in the streamed kernel's lane order
+// (w4a8_wants_qa), which enables it for 2..kMfmaMaxTokens tokens.
 // `mm` (may be null): mm_pack_bytes(m, cols, gs) bytes of scratch, which
 // enables the matrix-core GEMM for more than kMfmaMaxTokens tokens.
 // `params_tiled` (may be null): launch_params_tile16's copy of `params`,
@@ -102,23 +102,29 @@ bool launch_w4a8_dec_moe(float *out, const DecMoe &moe, const int8_t *q_split, c
 bool launch_w4a8_dec_moe_glu(const DecMoe &moe, const int8_t *q_split, const float *scales, const float *sums,
                              int rows, int cols, int gs, int max_entries, hipStream_t s);
 
-// Matrix-core W4A8 (gemv.hip): group 32, K a multiple of 256, 2..64 tokens
-// (past 64 the GEMM of gemm_mm.hip is faster on every measured shape).
+// Matrix-core W4A8 for 2..64 tokens (past 64 the GEMM of gemm_mm.hip is faster
+// on every measured shape).  The register-pipelined kernel of gemv.hip:
+// group 32, K a multiple of 512 up to 14336; it builds its operands from the
+// block-split int8 activations.  `params_tiled` (may be null): the same
+// parameters in the layout of launch_params_tile16, read instead of `params`
+// where it applies.
 constexpr int kMfmaMaxTokens = 64;
-bool w4a8_mfma_path(int rows, int cols, int m, int gs);
-// Halves of the packed activation buffer for m tokens of `cols` columns.
-size_t qa_pack_halves(int m, int cols);
-// Packs block-split int8 activations [m][cols] into the MFMA A-operand
-// layout (f16, zero rows for the padding tokens of the last 4-token group).
-void launch_qa_pack(const int8_t *q_split, int m, int cols, _Float16 *qa, hipStream_t s);
-// `params_tiled` (may be null): the same parameters in the layout of
-// launch_params_tile16, read instead of `params` where it applies.
-// `q_split` (may be null): the block-split int8 activations the packed
-// `qa` was made from, from which the register-pipelined kernel builds its
-// A operands itself.
-bool launch_w4a8_mfma(float *out, const float *add, const uint8_t *nib, const uint8_t *params, const _Float16 *qa,
-                      const int8_t *q_split, const float *scales, const float *sums, int rows, int cols, int m,
-                      int gs, hipStream_t s, const uint8_t *params_tiled = nullptr);
+bool gemv_rp_path(int rows, int cols, int m, int gs);
+void launch_gemv_rp(float *out, const float *add, const uint8_t *nib, const uint8_t *params, const int8_t *q_split,
+                    const float *scales, const float *sums, int rows, int cols, int m, hipStream_t s,
+                    const uint8_t *params_tiled);
+bool gemv_rp_cols(int cols, int gs);
+// The streamed kernel of gemv_stream.hip: whole groups of 32, 64 or 128, the
+// activations in its lane order (`qa`, qa_bytes of them, written by the
+// quantizing kernels below; rows of tokens past m are not read).
+bool gemv_stream_path(int rows, int cols, int m, int gs);
+size_t qa_bytes(int m, int cols, int gs);
+void launch_gemv_stream(float *out, const float *add, const uint8_t *nib, const uint8_t *params, const _Float16 *qa,
+                        const float *scales, const float *sums, int rows, int cols, int m, int gs, hipStream_t s);
+// True when a product over `cols` columns wants its activations as `qa`.
+inline bool w4a8_wants_qa(int cols, int m, int gs) {
+  return !gemv_rp_cols(cols, gs) && gemv_stream_path(1, cols, m, gs);
+}
 // The parameter array of a group-32 matrix (rows x cols/32 dwords, f16
 // scale and zero point per row and group) rearranged in 16-row tiles:
 // [rows / 16][cols / 128][16 rows][4 groups] dwords, the layout the
@@ -188,9 +194,8 @@ void launch_rmsnorm(const float *x, const float *w, float *out, float *resid, in
 bool fused_quant_ok(int n, int gs);
 // RMSNorm of m rows of n (layers.rs:325-376) + per-group quantization of
 // the result (gemm.rs:147-374); `normed` and `q_nat` may be null.
-// qa (may be null; group 32 only): also write the quantized rows in the
-// matrix-core activation layout (launch_qa_pack's output, padding rows of
-// the last 4-token group left untouched), which saves that pack.
+// qa (may be null): also write the quantized rows in the streamed kernel's
+// lane order (qa_bytes; rows of tokens past m left untouched).
 void launch_norm_quant(const float *x, const float *w, float *normed, int m, int n, float eps,
                        int gs, int8_t *q_split, int8_t *q_nat, float *scales, float *sums,
                        hipStream_t s, _Float16 *qa = nullptr);

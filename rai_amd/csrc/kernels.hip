@@ -773,22 +773,6 @@ void launch_small_mt(float *out, const float *add, const uint8_t *nib, const uin
     launch_small_t<GS, MT, R, PD, false>(out, add, nib, params, q_split, scales, sums, rows, cols, m, groups, s);
 }
 
-template <int GS>
-void launch_small_gs(float *out, const float *add, const uint8_t *nib, const uint8_t *params, const int8_t *q_split,
-                     const float *scales, const float *sums, int rows, int cols, int m, int groups,
-                     hipStream_t s) {
-  if (m <= 1)
-    launch_small_mt<GS, 1>(out, add, nib, params, q_split, scales, sums, rows, cols, m, groups, s);
-  else if (m <= 2)
-    launch_small_mt<GS, 2>(out, add, nib, params, q_split, scales, sums, rows, cols, m, groups, s);
-  else if (m <= 4)
-    launch_small_mt<GS, 4>(out, add, nib, params, q_split, scales, sums, rows, cols, m, groups, s);
-  else if (m <= 8 || GS > 32)  // groups 64/128 carry 9 chains: at most 8 tokens per tile
-    launch_small_mt<GS, 8>(out, add, nib, params, q_split, scales, sums, rows, cols, m, groups, s);
-  else
-    launch_small_mt<GS, 16>(out, add, nib, params, q_split, scales, sums, rows, cols, m, groups, s);
-}
-
 // --------------------------------------------------------- lane sums dbg --
 
 __global__ void k_lane_sums(int32_t *__restrict__ out, const uint8_t *__restrict__ nib,
@@ -1467,7 +1451,14 @@ void launch_w4a8(float *out, const float *add, const uint8_t *nib, const uint8_t
                        sums, rows, cols, m, gs, groups);
     return;
   }
-  if (launch_w4a8_mfma(out, add, nib, params, qa, q_split, scales, sums, rows, cols, m, gs, s, params_tiled)) return;
+  if (gemv_rp_path(rows, cols, m, gs)) {
+    launch_gemv_rp(out, add, nib, params, q_split, scales, sums, rows, cols, m, s, params_tiled);
+    return;
+  }
+  if (qa && gemv_stream_path(rows, cols, m, gs)) {
+    launch_gemv_stream(out, add, nib, params, qa, scales, sums, rows, cols, m, gs, s);
+    return;
+  }
   if (mm && w4a8_mm_path(rows, cols, m, gs)) {
     launch_w4a8_mm(out, add, nib, params, q_split, scales, sums, rows, cols, m, gs, mm, s);
     return;
@@ -1504,15 +1495,16 @@ void launch_w4a8(float *out, const float *add, const uint8_t *nib, const uint8_t
       done = launch_m1<128>(out, add, nib, params, q_split, scales, sums, rows, cols, groups, s);
     if (done) return;
   }
-  if (m <= 16) {
+  if (m == 1) {
     if (gs == 32)
-      launch_small_gs<32>(out, add, nib, params, q_split, scales, sums, rows, cols, m, groups, s);
+      launch_small_mt<32, 1>(out, add, nib, params, q_split, scales, sums, rows, cols, m, groups, s);
     else if (gs == 64)
-      launch_small_gs<64>(out, add, nib, params, q_split, scales, sums, rows, cols, m, groups, s);
+      launch_small_mt<64, 1>(out, add, nib, params, q_split, scales, sums, rows, cols, m, groups, s);
     else
-      launch_small_gs<128>(out, add, nib, params, q_split, scales, sums, rows, cols, m, groups, s);
+      launch_small_mt<128, 1>(out, add, nib, params, q_split, scales, sums, rows, cols, m, groups, s);
     return;
   }
+  // Several tokens and a matrix of 2 GiB or more.
   if (gs == 32)
     launch_fast_gs<32>(out, add, nib, params, q_split, scales, sums, rows, cols, m, groups, s);
   else if (gs == 64)

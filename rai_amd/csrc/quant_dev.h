@@ -29,11 +29,17 @@ __device__ __forceinline__ int split_col(int c) {
 // natural layouts (qn_grp may be null; either may be in LDS).
 // All 64 lanes of the wave must call this together.
 // Lanes with ok == false take part in the shuffles and store nothing.
-// Matrix-core activation slot of (token t, group g) for group 32 (see
-// k_qa_pack4 in gemv.hip): qa4[t/4][g/4][b][4(t%4) + g%4][8] f16; block b of
-// the slot is 128 halves further.
-__device__ __forceinline__ _Float16 *qa4_slot(_Float16 *qa, int t, int g, int groups) {
-  return qa + ((((size_t)(t >> 2) * (groups >> 2) + (g >> 2)) * 64) + 4 * (t & 3) + (g & 3)) * 8;
+// Matrix-core activation slot of (token t, group g) for k_gemv_stream
+// (gemv_stream.hip): qa[t / 16][g / 4][block place][16 (g % 4) + t % 16][8]
+// f16, where the place of 8-column block b of the group is b, at group 128
+// 2 (b % 8) + b / 8 (the two blocks of a reference lane side by side).
+template <int GS>
+__device__ __forceinline__ _Float16 *qa_slot_of(_Float16 *qa, int t, int g, int groups) {
+  return qa + (((size_t)(t >> 4) * ((groups + 3) >> 2) + (g >> 2)) * (GS / 8) * 64 + 16 * (g & 3) + (t & 15)) * 8;
+}
+template <int NB>
+__device__ __forceinline__ constexpr int qa_block(int b) {
+  return 512 * (NB == 16 ? 2 * (b & 7) + (b >> 3) : b);
 }
 
 // Lane moves inside 16-lane rows (DPP, no LDS round trip): lane i reads
@@ -78,7 +84,7 @@ __device__ __forceinline__ void quantize_group8_to(const float (&v)[NB], int j, 
     if (qn_grp) qn_grp[col] = q;
     // f16 element e of a block is its column (0, 4, 1, 5, 2, 6, 3, 7)[e];
     // odd columns are stored divided by 16 (the codes enter at 16 n).
-    if (qa_slot) qa_slot[c8 * 128 + 2 * (j & 3) + (j >> 2)] = (_Float16)((j & 1) ? r * 0.0625f : r);
+    if (qa_slot) qa_slot[qa_block<NB>(c8) + 2 * (j & 3) + (j >> 2)] = (_Float16)((j & 1) ? r * 0.0625f : r);
   }
   if (j == 0) {
     *scale_out = scale;
@@ -169,7 +175,7 @@ __device__ __forceinline__ void rmsnorm_quant_block(const float *__restrict__ ro
     }
     quantize_group8_to<NB>(v, j, ok, qs + (size_t)(ok ? g : 0) * qstr, qn ? qn + col0 : nullptr,
                            scale_out + (ok ? g : 0), sum_out + (ok ? g : 0),
-                           qa ? qa4_slot(qa, token, ok ? g : 0, groups) : nullptr);
+                           qa ? qa_slot_of<GS>(qa, token, ok ? g : 0, groups) : nullptr);
   }
 }
 
@@ -360,7 +366,7 @@ __device__ __forceinline__ float rmsnorm_inv_t(const float *xt, int n, float eps
 // (x and the norm weights) by a 256-thread block; xs: LDS scratch of
 // rms_scratch_floats(n) floats, 16-byte aligned.  Optional outputs: the
 // natural-order codes qn, the normalised row nrow and the matrix-core slots
-// of token `token` in qa (group 32).
+// of token `token` in qa.
 template <int GS, int P>
 __device__ __forceinline__ void rmsnorm_quant_regs(const float (&xr)[P][GS / 8], const float (&wr)[P][GS / 8],
                                                    int n, float eps, float *xs, int8_t *qs, int qstr,
@@ -395,7 +401,7 @@ __device__ __forceinline__ void rmsnorm_quant_regs(const float (&xr)[P][GS / 8],
     }
     quantize_group8_to<NB>(v, j, ok, qs + (size_t)(ok ? g : 0) * qstr, qn ? qn + (ok ? g : 0) * GS : nullptr,
                            scale_out + (ok ? g : 0), sum_out + (ok ? g : 0),
-                           qa ? qa4_slot(qa, token, ok ? g : 0, groups) : nullptr);
+                           qa ? qa_slot_of<GS>(qa, token, ok ? g : 0, groups) : nullptr);
   }
 }
 

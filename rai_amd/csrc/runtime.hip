@@ -277,7 +277,7 @@ struct Workspace {
     am.alloc(sizeof(uint32_t) * maxm);
     q_nat.alloc(K * maxm);
     q_split.alloc(K * maxm);
-    qa.alloc(sizeof(_Float16) * qa_pack_halves(std::min(maxm, kMfmaMaxTokens), (int)K));
+    qa.alloc(qa_bytes(std::min(maxm, kMfmaMaxTokens), (int)K, (int)c.group_size));
     if (maxm > kMfmaMaxTokens) qmm.alloc(mm_pack_bytes(maxm, (int)K, (int)c.group_size));
     hq.alloc(H * maxm);
     qscale.alloc(sizeof(float) * G * maxm);
@@ -568,17 +568,10 @@ static void linear(const DLinear &L, const float *x, const Workspace &w, float *
               w.qa.as<_Float16>(), w.qmm.as<uint8_t>(), L.params_tiled);
 }
 
-// After any quantization of m rows of k columns into the workspace: pack
-// the activations for the matrix-core kernel when it applies.
-static void pack_for_mfma(const rai_model &md, int m, int k, const Workspace &w, hipStream_t s) {
-  if (w4a8_mfma_path(1, k, m, md.cfg.group_size))
-    launch_qa_pack(w.q_split.as<int8_t>(), m, k, w.qa.as<_Float16>(), s);
-}
-
 // The matrix-core activation buffer for a fused quantizer to fill directly
-// (null when the matrix-core GEMV does not apply).
+// (null when no product on these rows reads it).
 static _Float16 *mfma_acts(const rai_model &md, int m, int k, const Workspace &w) {
-  return w4a8_mfma_path(1, k, m, md.cfg.group_size) ? w.qa.as<_Float16>() : nullptr;
+  return w4a8_wants_qa(k, m, md.cfg.group_size) ? w.qa.as<_Float16>() : nullptr;
 }
 
 static void quantize(const rai_model &md, const float *x, int m, int k, const Workspace &w,
@@ -589,7 +582,6 @@ static void quantize(const rai_model &md, const float *x, int m, int k, const Wo
   } else {
     launch_quantize(x, m, k, md.cfg.group_size, w.q_nat.as<int8_t>(), w.q_split.as<int8_t>(),
                     w.qscale.as<float>(), w.qsum.as<float>(), s);
-    pack_for_mfma(md, m, k, w, s);
   }
 }
 
@@ -1445,7 +1437,6 @@ static void quantize_call(const float *x, int m, int cols, int gs, bool fast, co
     launch_quant(x, m, cols, gs, a.qs, nullptr, a.sc, a.su, s, a.qa);
   } else {
     launch_quantize(x, m, cols, gs, a.qn, a.qs, a.sc, a.su, s);
-    if (a.qa) launch_qa_pack(a.qs, m, cols, a.qa, s);
   }
 }
 
@@ -1472,14 +1463,14 @@ int rai_w4a8_matmul_dev(float *out, const uint8_t *nib, const uint8_t *params, c
       return RAI_OK;
     }
     const bool fast = rai::w4a8_fast_path((int)cols, (int)gs, nib, params);
-    const bool mfma = fast && rai::w4a8_mfma_path((int)rows, (int)cols, (int)m, (int)gs);
+    const bool wqa = fast && rai::w4a8_wants_qa((int)cols, (int)m, (int)gs);
     const bool mm = fast && rai::w4a8_mm_path((int)rows, (int)cols, (int)m, (int)gs);
     const size_t nq = m * cols, ng = m * groups * 4;
-    const size_t nqa = mfma ? sizeof(_Float16) * rai::qa_pack_halves((int)m, (int)cols) : 0;
+    const size_t nqa = wqa ? rai::qa_bytes((int)m, (int)cols, (int)gs) : 0;
     const size_t nmm = mm ? rai::mm_pack_bytes((int)m, (int)cols, (int)gs) : 0;
     rai::CallScratch ws(2 * rai::piece(nq) + 2 * rai::piece(ng) + rai::piece(nqa) + rai::piece(nmm), s);
     rai::CallActs a{ws.take<int8_t>(nq), ws.take<int8_t>(nq), ws.take<float>(ng), ws.take<float>(ng), nullptr, nullptr};
-    if (mfma) a.qa = ws.take<_Float16>(nqa);
+    if (wqa) a.qa = ws.take<_Float16>(nqa);
     if (mm) a.mm = ws.take<uint8_t>(nmm);
     rai::quantize_call(x, (int)m, (int)cols, (int)gs, fast, a, s);
     rai::launch_w4a8(out, nullptr, nib, params, x, a.qn, a.qs, a.sc, a.su, (int)rows, (int)cols, (int)m, (int)gs, s,
@@ -1563,8 +1554,8 @@ int rai_w4a8_fused_gate_up_dev(float *gate_out, float *up_out, const rai_qlinear
 // device address (in host code it names a host-side stand-in); it uses the
 // address hipGetSymbolAddress returns on each device, looked up once per
 // device on the first call there.  Layout (bytes): q_nat [m*cols], q_split
-// [m*cols], scales [m*groups] f32, sums [m*groups] f32, matrix-core
-// activations (2..64 tokens), the matrix-core GEMM's activation records
+// [m*cols], scales [m*groups] f32, sums [m*groups] f32, then the
+// streamed kernel's activations (2..64 tokens) or the GEMM's activation records
 // (more than 64 tokens: ceil(m/32) tiles of the group count padded to 4, 2
 // or 2 (groups of 32, 64, 128) records of 64 gs + 260 bytes; with m > 64 and
 // m * cols <= 2^20 the largest is 1024 tiles of 4 records at cols = 32, gs =
@@ -1572,9 +1563,8 @@ int rai_w4a8_fused_gate_up_dev(float *gate_out, float *up_out, const rai_qlinear
 namespace rai {
 constexpr size_t kNaTokenCols = size_t(1) << 20;  // m * cols
 constexpr size_t kNaGroups = size_t(1) << 16;     // m * ceil(cols / gs)
-constexpr size_t kNaQaBytes = size_t(2) << 20;
-constexpr size_t kNaMmBytes = (size_t(9) << 20) + (size_t(1) << 19);  // 9.5 MiB
-constexpr size_t kNaScratchBytes = 2 * kNaTokenCols + 8 * kNaGroups + kNaQaBytes + kNaMmBytes;
+constexpr size_t kNaMmBytes = size_t(12) << 20;
+constexpr size_t kNaScratchBytes = 2 * kNaTokenCols + 8 * kNaGroups + kNaMmBytes;
 constexpr int kNaMaxDevices = 64;
 }  // namespace rai
 
@@ -1617,9 +1607,11 @@ int rai_w4a8_matmul_noalloc_dev(float *out, const uint8_t *nib, const uint8_t *p
                                  std::to_string(rai::kNaTokenCols) + " token columns and " +
                                  std::to_string(rai::kNaGroups) + " token groups)");
     const bool fast = rai::w4a8_fast_path((int)cols, (int)gs, nib, params);
-    const bool mfma = fast && rai::w4a8_mfma_path((int)rows, (int)cols, (int)m, (int)gs);
-    if (mfma && sizeof(_Float16) * rai::qa_pack_halves((int)m, (int)cols) > rai::kNaQaBytes)
-      rai::fail(RAI_E_SHAPE, "activation tile exceeds the allocation-free scratch");
+    // The streamed kernel's activations share the records' place; past its
+    // size (two tokens of more than 393216 columns) the product takes the
+    // tiled VALU kernel.
+    const bool wqa = fast && rai::w4a8_wants_qa((int)cols, (int)m, (int)gs) &&
+                     rai::qa_bytes((int)m, (int)cols, (int)gs) <= rai::kNaMmBytes;
     const bool mm = fast && rai::w4a8_mm_path((int)rows, (int)cols, (int)m, (int)gs);
     if (mm && rai::mm_pack_bytes((int)m, (int)cols, (int)gs) > rai::kNaMmBytes)
       rai::fail(RAI_E_SHAPE, "activation records exceed the allocation-free scratch");
@@ -1628,13 +1620,11 @@ int rai_w4a8_matmul_noalloc_dev(float *out, const uint8_t *nib, const uint8_t *p
     int8_t *qs = reinterpret_cast<int8_t *>(base + rai::kNaTokenCols);
     float *sc = reinterpret_cast<float *>(base + 2 * rai::kNaTokenCols);
     float *su = sc + rai::kNaGroups;
-    _Float16 *qa = reinterpret_cast<_Float16 *>(base + 2 * rai::kNaTokenCols + 8 * rai::kNaGroups);
-    uint8_t *mmp = base + 2 * rai::kNaTokenCols + 8 * rai::kNaGroups + rai::kNaQaBytes;
+    uint8_t *mmp = base + 2 * rai::kNaTokenCols + 8 * rai::kNaGroups;
+    _Float16 *qa = wqa ? reinterpret_cast<_Float16 *>(mmp) : nullptr;
     hipStream_t s = (hipStream_t)stream;
     // Every scratch byte behind a stored output is written earlier in this
-    // call (the padding rows of the last token group may hold an earlier
-    // call's values, but reach only the outputs of padding tokens, which are
-    // not stored).
+    // call (tokens past the last are not read).
     // One token at a short row: the GEMV launch quantizes the row itself.
     if (m == 1 && rai::w4a8_fast_path((int)cols, (int)gs, nib, params) && !rai::overlaps(out, rows, x, cols) &&
         rai::launch_w4a8_dec(out, nullptr, nib, params, nullptr, nullptr, nullptr, (int)rows, (int)cols,
@@ -1642,9 +1632,9 @@ int rai_w4a8_matmul_noalloc_dev(float *out, const uint8_t *nib, const uint8_t *p
       HIP_CHECK(hipGetLastError());
       return RAI_OK;
     }
-    rai::quantize_call(x, (int)m, (int)cols, (int)gs, fast, {qn, qs, sc, su, mfma ? qa : nullptr, nullptr}, s);
+    rai::quantize_call(x, (int)m, (int)cols, (int)gs, fast, {qn, qs, sc, su, qa, nullptr}, s);
     rai::launch_w4a8(out, nullptr, nib, params, x, qn, qs, sc, su, (int)rows, (int)cols, (int)m, (int)gs, s,
-                     mfma ? qa : nullptr, mm ? mmp : nullptr);
+                     qa, mm ? mmp : nullptr);
     HIP_CHECK(hipGetLastError());
   });
 }
@@ -1666,15 +1656,15 @@ int rai_w4a8_time_dev(float *out, const uint8_t *nib, const uint8_t *params, con
     hipEvent_t e0, e1;
     HIP_CHECK(hipEventCreate(&e0));
     HIP_CHECK(hipEventCreate(&e1));
-    rai::launch_quantize(x, (int)m, (int)cols, (int)gs, qn.as<int8_t>(), qs.as<int8_t>(), sc.as<float>(),
-                         su.as<float>(), s);
+    const bool fast = rai::w4a8_fast_path((int)cols, (int)gs, nib, params);
+    const bool mfma = fast && rai::gemv_rp_path((int)rows, (int)cols, (int)m, (int)gs);
     rai::DevBuf qa, mm;
-    const bool mfma = rai::w4a8_mfma_path((int)rows, (int)cols, (int)m, (int)gs);
-    if (mfma) {
-      qa.alloc(sizeof(_Float16) * rai::qa_pack_halves((int)m, (int)cols));
-      rai::launch_qa_pack(qs.as<int8_t>(), (int)m, (int)cols, qa.as<_Float16>(), s);
-    }
-    if (rai::w4a8_mm_path((int)rows, (int)cols, (int)m, (int)gs)) mm.alloc(rai::mm_pack_bytes((int)m, (int)cols, (int)gs));
+    if (fast && rai::w4a8_wants_qa((int)cols, (int)m, (int)gs)) qa.alloc(rai::qa_bytes((int)m, (int)cols, (int)gs));
+    rai::quantize_call(x, (int)m, (int)cols, (int)gs, fast,
+                       {qn.as<int8_t>(), qs.as<int8_t>(), sc.as<float>(), su.as<float>(), qa.as<_Float16>(), nullptr},
+                       s);
+    if (fast && rai::w4a8_mm_path((int)rows, (int)cols, (int)m, (int)gs))
+      mm.alloc(rai::mm_pack_bytes((int)m, (int)cols, (int)gs));
     const size_t nib_bytes = rows * cols / 2, par_bytes = rows * groups * 4;
     // The parameters' tile-layout copies, as a loaded model holds them.
     rai::DevBuf tiled;
@@ -1688,7 +1678,7 @@ int rai_w4a8_time_dev(float *out, const uint8_t *nib, const uint8_t *params, con
     auto run = [&](size_t c) {
       rai::launch_w4a8(out, nullptr, nib + c * nib_bytes, params + c * par_bytes, x, qn.as<int8_t>(),
                        qs.as<int8_t>(), sc.as<float>(), su.as<float>(), (int)rows, (int)cols, (int)m, (int)gs, s,
-                       mfma ? qa.as<_Float16>() : nullptr, mm.as<uint8_t>(),
+                       qa.as<_Float16>(), mm.as<uint8_t>(),
                        tiled.p ? tiled.as<uint8_t>() + c * par_bytes : nullptr);
     };
     run(0);  // warm-up

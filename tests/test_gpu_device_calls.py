@@ -147,3 +147,39 @@ def test_decode_steps_every_group_size(rai, ora, gs, hidden, heads, kv, hd, ffn,
         assert np.array_equal(_bits(got).reshape(-1), _bits(want).reshape(-1)), pos
         gl, ol = gm.hidden_to_logits_batch(got, 1), om.hidden_to_logits_batch(want, 1)
         assert np.array_equal(_bits(gl).reshape(-1), _bits(ol).reshape(-1)), pos
+
+
+# 2..64 tokens: one to four token tiles of 16; row counts that take one, two
+# and four waves per row tile; K of one group, of a partial step of four groups
+# and of several steps; K the register-pipelined kernel does not take.
+@pytest.mark.parametrize("gs,cols", [(32, 32), (32, 160), (32, 416), (32, 768), (32, 1056), (64, 64), (64, 320),
+                                     (64, 1088), (128, 128), (128, 640), (128, 2688)])
+@pytest.mark.parametrize("rows,m", [(1, 2), (17, 4), (70, 9), (50, 16), (33, 17), (40, 64), (5000, 49), (16400, 33)])
+def test_small_batches_every_group_size(rai, ora, gs, cols, rows, m):
+    if rows > 1000 and cols > 700:
+        cols = 4 * gs + gs  # the oracle's time
+    nib, params, x = gemv_operands(rows, cols, m, gs, seed=rows + cols + m)
+    for special in (False, True):
+        if special:
+            x = _tokens(x, m, cols, gs, cols + m)
+        want = ora.w4a8_matmul(nib, params, x, rows, cols, m, gs)
+        dev = rai.DeviceArray.from_host
+        xd = dev(np.ascontiguousarray(x, np.float32))
+        for name in ("rai_w4a8_matmul_dev", "rai_w4a8_matmul_noalloc_dev"):
+            got = _call(rai, name, rai.DeviceArray(4 * m * rows), dev(nib), dev(params), xd, rows, cols, m, gs)
+            assert np.array_equal(_bits(got).reshape(-1), _bits(want).reshape(-1)), (name, special)
+
+
+@pytest.mark.parametrize("gs", [64, 128])
+@pytest.mark.parametrize("m", [2, 9, 40])
+def test_small_batch_layers(rai, ora, gs, m):
+    """The model path: norm, attention output, silu_mul and head activations
+    in the streamed kernel's order."""
+    img = rai.synth_model(1152, 2, 9, 3, 128, 1280, 400, 128, group_size=gs, seed=gs + m)
+    gm, om = rai.RaiModel.from_bytes(img), ora.Model(img, 0)
+    h = np.random.default_rng(m).normal(0.0, 1.0, (m, 1152)).astype(np.float32)
+    got = gm.forward_batch(h, np.arange(m), gm.create_kv_cache(128))
+    want = om.forward_batch(h, np.arange(m), om.create_kv(128))
+    assert np.array_equal(_bits(got).reshape(-1), _bits(want).reshape(-1))
+    gl, ol = gm.hidden_to_logits_batch(got, m), om.hidden_to_logits_batch(want, m)
+    assert np.array_equal(_bits(gl).reshape(-1), _bits(ol).reshape(-1))
