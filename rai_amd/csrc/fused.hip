@@ -35,7 +35,7 @@ template <int NB>
 __device__ __forceinline__ void quantize_group8(const float (&v)[NB], int j, int col0, bool ok,
                                                 int8_t *__restrict__ qs, int8_t *__restrict__ qn,
                                                 float *__restrict__ scale_out,
-                                                float *__restrict__ sum_out, _Float16 *qa_slot = nullptr) {
+                                                float *__restrict__ sum_out, QaSlot qa_slot = {}) {
   quantize_group8_to<NB>(v, j, ok, qs + col0, qn ? qn + col0 : nullptr, scale_out, sum_out, qa_slot);
 }
 
@@ -156,7 +156,7 @@ __global__ __launch_bounds__(256) void k_silu_quant(float *__restrict__ gate,
   int8_t *qs = q_split + (size_t)t * n;
   int8_t *qn = q_nat ? q_nat + (size_t)t * n : nullptr;
   quantize_group8<NB>(v, j, col0, ok, qs, qn, scales + (size_t)t * groups + g,
-                      sums + (size_t)t * groups + g, qa ? qa_slot_of<GS>(qa, t, ok ? g : 0, groups) : nullptr);
+                      sums + (size_t)t * groups + g, qa ? qa_slot_of<GS>(qa, t, ok ? g : 0, groups) : QaSlot{});
 }
 
 // Per-group quantization of m rows of n (quantize_input_split +
@@ -181,7 +181,7 @@ __global__ __launch_bounds__(256) void k_quant(const float *__restrict__ x, int 
   int8_t *qs = q_split + (size_t)t * n;
   int8_t *qn = q_nat ? q_nat + (size_t)t * n : nullptr;
   quantize_group8<NB>(v, j, col0, ok, qs, qn, scales + (size_t)t * groups + g,
-                      sums + (size_t)t * groups + g, qa ? qa_slot_of<GS>(qa, t, ok ? g : 0, groups) : nullptr);
+                      sums + (size_t)t * groups + g, qa ? qa_slot_of<GS>(qa, t, ok ? g : 0, groups) : QaSlot{});
 }
 
 // -------------------------------------------------------------- attention --

@@ -118,9 +118,12 @@ bool gemv_rp_cols(int cols, int gs);
 // activations in its lane order (`qa`, qa_bytes of them, written by the
 // quantizing kernels below; rows of tokens past m are not read).
 bool gemv_stream_path(int rows, int cols, int m, int gs);
+// One step's activations: gs / 8 blocks of 64 lanes x 8 f16, then 64 scales
+// and 64 input sums.
+constexpr int qa_rec_bytes(int gs) { return gs * 128 + 512; }
 size_t qa_bytes(int m, int cols, int gs);
 void launch_gemv_stream(float *out, const float *add, const uint8_t *nib, const uint8_t *params, const _Float16 *qa,
-                        const float *scales, const float *sums, int rows, int cols, int m, int gs, hipStream_t s);
+                        int rows, int cols, int m, int gs, hipStream_t s);
 // True when a product over `cols` columns wants its activations as `qa`.
 inline bool w4a8_wants_qa(int cols, int m, int gs) {
   return !gemv_rp_cols(cols, gs) && gemv_stream_path(1, cols, m, gs);

@@ -1456,7 +1456,7 @@ void launch_w4a8(float *out, const float *add, const uint8_t *nib, const uint8_t
     return;
   }
   if (qa && gemv_stream_path(rows, cols, m, gs)) {
-    launch_gemv_stream(out, add, nib, params, qa, scales, sums, rows, cols, m, gs, s);
+    launch_gemv_stream(out, add, nib, params, qa, rows, cols, m, gs, s);
     return;
   }
   if (mm && w4a8_mm_path(rows, cols, m, gs)) {

@@ -29,13 +29,21 @@ __device__ __forceinline__ int split_col(int c) {
 // natural layouts (qn_grp may be null; either may be in LDS).
 // All 64 lanes of the wave must call this together.
 // Lanes with ok == false take part in the shuffles and store nothing.
-// Matrix-core activation slot of (token t, group g) for k_gemv_stream
-// (gemv_stream.hip): qa[t / 16][g / 4][block place][16 (g % 4) + t % 16][8]
-// f16, where the place of 8-column block b of the group is b, at group 128
+// Place of (token t, group g) in the activations of k_gemv_stream
+// (gemv_stream.hip): record [t / 16][g / 4] holds, in lane order
+// 16 (g % 4) + t % 16, GS / 8 blocks of eight f16, then the scale and the
+// input sum.  The place of 8-column block b is b, at group 128
 // 2 (b % 8) + b / 8 (the two blocks of a reference lane side by side).
+struct QaSlot {
+  _Float16 *blk = nullptr;  // block 0; the next one 512 halves further
+  float *sc = nullptr;      // scale; the sum 64 floats further
+};
 template <int GS>
-__device__ __forceinline__ _Float16 *qa_slot_of(_Float16 *qa, int t, int g, int groups) {
-  return qa + (((size_t)(t >> 4) * ((groups + 3) >> 2) + (g >> 2)) * (GS / 8) * 64 + 16 * (g & 3) + (t & 15)) * 8;
+__device__ __forceinline__ QaSlot qa_slot_of(_Float16 *qa, int t, int g, int groups) {
+  constexpr int REC = GS * 128 + 512;
+  uint8_t *rec = reinterpret_cast<uint8_t *>(qa) + ((size_t)(t >> 4) * ((groups + 3) >> 2) + (g >> 2)) * REC;
+  const int lane = 16 * (g & 3) + (t & 15);
+  return {reinterpret_cast<_Float16 *>(rec) + lane * 8, reinterpret_cast<float *>(rec + GS * 128) + lane};
 }
 template <int NB>
 __device__ __forceinline__ constexpr int qa_block(int b) {
@@ -55,7 +63,7 @@ constexpr int kDppShl1 = 0x101, kDppShl2 = 0x102, kDppShl4 = 0x104, kDppHalfMirr
 template <int NB>
 __device__ __forceinline__ void quantize_group8_to(const float (&v)[NB], int j, bool ok, int8_t *qs_grp,
                                                    int8_t *qn_grp, float *scale_out, float *sum_out,
-                                                   _Float16 *qa_slot = nullptr) {
+                                                   QaSlot qa_slot = {}) {
   float a = 0.0f, amax = 0.0f;
 #pragma unroll
   for (int c = 0; c < NB; ++c) {
@@ -84,11 +92,15 @@ __device__ __forceinline__ void quantize_group8_to(const float (&v)[NB], int j, 
     if (qn_grp) qn_grp[col] = q;
     // f16 element e of a block is its column (0, 4, 1, 5, 2, 6, 3, 7)[e];
     // odd columns are stored divided by 16 (the codes enter at 16 n).
-    if (qa_slot) qa_slot[qa_block<NB>(c8) + 2 * (j & 3) + (j >> 2)] = (_Float16)((j & 1) ? r * 0.0625f : r);
+    if (qa_slot.blk) qa_slot.blk[qa_block<NB>(c8) + 2 * (j & 3) + (j >> 2)] = (_Float16)((j & 1) ? r * 0.0625f : r);
   }
   if (j == 0) {
     *scale_out = scale;
     *sum_out = total;
+    if (qa_slot.sc) {
+      qa_slot.sc[0] = scale;
+      qa_slot.sc[64] = total;
+    }
   }
 }
 
@@ -175,7 +187,7 @@ __device__ __forceinline__ void rmsnorm_quant_block(const float *__restrict__ ro
     }
     quantize_group8_to<NB>(v, j, ok, qs + (size_t)(ok ? g : 0) * qstr, qn ? qn + col0 : nullptr,
                            scale_out + (ok ? g : 0), sum_out + (ok ? g : 0),
-                           qa ? qa_slot_of<GS>(qa, token, ok ? g : 0, groups) : nullptr);
+                           qa ? qa_slot_of<GS>(qa, token, ok ? g : 0, groups) : QaSlot{});
   }
 }
 
@@ -401,7 +413,7 @@ __device__ __forceinline__ void rmsnorm_quant_regs(const float (&xr)[P][GS / 8],
     }
     quantize_group8_to<NB>(v, j, ok, qs + (size_t)(ok ? g : 0) * qstr, qn ? qn + (ok ? g : 0) * GS : nullptr,
                            scale_out + (ok ? g : 0), sum_out + (ok ? g : 0),
-                           qa ? qa_slot_of<GS>(qa, token, ok ? g : 0, groups) : nullptr);
+                           qa ? qa_slot_of<GS>(qa, token, ok ? g : 0, groups) : QaSlot{});
   }
 }
 
