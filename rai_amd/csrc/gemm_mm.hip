@@ -1,4 +1,4 @@
-// W4A8 GEMM for prefill-sized token counts (M > 64) on the gfx950 matrix
+// W4A8 GEMM for prefill-sized token counts (w4a8_route) on the gfx950 matrix
 // cores, groups of 32, 64 or 128: the reference's matmul_chunk_i8 /
 // matmul_row_tile (gemm.rs:540-784) with the same per-lane integer sums and
 // the same f32 epilogue order, so the outputs equal the CPU path bit for bit.
@@ -385,14 +385,35 @@ void launch_mm_t(float *out, const float *add, const uint8_t *nib, const uint8_t
 
 }  // namespace
 
-// Every whole-group shape past 64 tokens: against the VALU kernel that the
-// shapes outside group 32 and K % 512 == 0 took before, whole calls measured
-// 14336x4096 at 512 tokens, group 128: 2084 -> 176 us; 4096x11008 at 301
-// tokens, group 32: 1630 -> 228 us (1.25 waves per SIMD: the 1280 waves leave
-// three quarters of the SIMDs with one); a small one, 35 -> 24 us.
-bool w4a8_mm_path(int rows, int cols, int m, int gs) {
-  return (gs == 32 || gs == 64 || gs == 128) && m > kMfmaMaxTokens && rows > 0 && cols % gs == 0 &&
+// Against the VALU kernel that the shapes outside group 32 and K % 512 == 0
+// took before, whole calls measured 14336x4096 at 512 tokens, group 128: 2084
+// -> 176 us; 4096x11008 at 301 tokens, group 32: 1630 -> 228 us (1.25 waves
+// per SIMD: the 1280 waves leave three quarters of the SIMDs with one).
+static bool mm_ok(int rows, int cols, int gs) {
+  return (gs == 32 || gs == 64 || gs == 128) && rows > 0 && cols > 0 && cols % gs == 0 &&
          (int64_t)rows * (cols / 2) < ((int64_t)1 << 31);
+}
+
+// Where the lines lie (device time, weights from HBM, K = 4096; the times of
+// all three grow alike with K):
+// - Up to 24 tokens the register-pipelined kernel, whose tiles are four
+//   tokens, where it applies: 28672 rows, 9 tokens 26.1 us (streamed 39.7), 24
+//   tokens 56.2 (68.4); 4096 rows, 32 tokens 19.2 (17.5).
+// - The streamed kernel has 16 x 16 tiles and splits a tile's chains over
+//   waves, so it wins until the GEMM's 32 x 32 tiles alone fill the chip, at
+//   about 4500 tiles of its own: group 32, 28672 rows, 32 tokens (3584 tiles)
+//   68.2 against 70.0, 64 tokens (7168) 120.5 against 97.5; 4096 rows, 96
+//   tokens (1536) 36 against 66.  Group 128, where the GEMM's two blocks per
+//   instruction count: 14336 rows, 33 tokens (2688) 38.4 against 41.1, 64
+//   (3584) 46.7 against 41.7.
+// - Up to 16 tokens half of the GEMM's tile would be padding at any size.
+W4Route w4a8_route(int rows, int cols, int m, int gs) {
+  if (!mm_ok(rows, cols, gs)) return W4Route::kValu;
+  if (m <= 24 && gemv_rp_path(rows, cols, m, gs)) return W4Route::kRp;
+  const int64_t tiles = (int64_t)((rows + 15) / 16) * ((m + 15) / 16);
+  if ((m <= 16 || tiles <= (gs == 128 ? 3000 : 4500)) && qa_bytes(m, cols, gs) < ((size_t)1 << 31))
+    return W4Route::kStream;
+  return W4Route::kMm;
 }
 
 // Records, flags and the bytes the last DMA piece may read past them.
@@ -418,7 +439,7 @@ void launch_w4a8_mm(float *out, const float *add, const uint8_t *nib, const uint
     go(launch_mm_t<128>);
 }
 
-bool moe_mm_path(int rows, int cols, int gs) { return w4a8_mm_path(rows, cols, kMfmaMaxTokens + 1, gs); }
+bool moe_mm_path(int rows, int cols, int gs) { return mm_ok(rows, cols, gs); }
 
 void launch_moe_mm(float *out, int ld, const MmMoe &moe, int max_tiles, const int8_t *q_split, const float *scales,
                    const float *sums, int rows, int cols, int gs, uint8_t *pack, hipStream_t s) {

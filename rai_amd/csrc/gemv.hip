@@ -506,13 +506,9 @@ void launch_params_tile16(const uint8_t *params, int rows, int cols, uint8_t *ti
                      reinterpret_cast<const u32x4 *>(params), rows, nq, reinterpret_cast<u32x4 *>(tiled));
 }
 
-// K as the register-pipelined kernel takes it (2..64 tokens at group 32).
-bool gemv_rp_cols(int cols, int gs) {
-  return gs == 32 && cols > 0 && cols % (128 * kRpRing) == 0 && cols <= kRpMaxColsOne;
-}
-
+// Group 32, K a multiple of 512 up to 14336, a matrix under 2 GiB.
 bool gemv_rp_path(int rows, int cols, int m, int gs) {
-  return gemv_rp_cols(cols, gs) && m >= 2 && m <= kMfmaMaxTokens && rows > 0 &&
+  return gs == 32 && cols > 0 && cols % (128 * kRpRing) == 0 && cols <= kRpMaxColsOne && m >= 2 && rows > 0 &&
          (int64_t)rows * (cols / 2) < ((int64_t)1 << 31);
 }
 

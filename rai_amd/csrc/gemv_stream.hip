@@ -1,4 +1,4 @@
-// W4A8 product for 2..64 tokens on the gfx950 matrix cores, groups of 32, 64
+// W4A8 product for small batches (w4a8_route) on the gfx950 matrix cores, groups of 32, 64
 // or 128 and any number of them: the same exact lane sums and the same f32
 // epilogue order as the other W4A8 kernels (gemm.rs:458-784), so the outputs
 // equal the CPU path bit for bit.
@@ -372,11 +372,6 @@ void launch_stream_t(float *out, const float *add, const uint8_t *nib, const uin
 }
 
 }  // namespace
-
-bool gemv_stream_path(int rows, int cols, int m, int gs) {
-  return (gs == 32 || gs == 64 || gs == 128) && m >= 2 && m <= kMfmaMaxTokens && rows > 0 && cols % gs == 0 &&
-         (int64_t)rows * (cols / 2) < ((int64_t)1 << 31) && qa_bytes(m, cols, gs) < ((size_t)1 << 31);
-}
 
 size_t qa_bytes(int m, int cols, int gs) {
   return (size_t)((m + 15) / 16) * ((cols / gs + 3) / 4) * qa_rec_bytes(gs);

@@ -21,10 +21,10 @@ void launch_quantize(const float *x, int m, int k, int gs, int8_t *q_nat, int8_t
 // `add` (may be null, may equal `out`): a residual [m][rows] added to each
 // output, out = add + matmul (the reference's vec_add after o_proj/down,
 // layers.rs:503-531, fused into the epilogue).
-// `qa` (may be null): the activations in the streamed kernel's lane order
-// (w4a8_wants_qa), which enables it for 2..kMfmaMaxTokens tokens.
+// `qa` (may be null): the activations in the streamed kernel's lane order,
+// which enables it where w4a8_route says so.
 // `mm` (may be null): mm_pack_bytes(m, cols, gs) bytes of scratch, which
-// enables the matrix-core GEMM for more than kMfmaMaxTokens tokens.
+// enables the matrix-core GEMM where w4a8_route says so.
 // `params_tiled` (may be null): launch_params_tile16's copy of `params`,
 // which the matrix-core GEMV then reads.
 void launch_w4a8(float *out, const float *add, const uint8_t *nib, const uint8_t *params, const float *x,
@@ -102,32 +102,28 @@ bool launch_w4a8_dec_moe(float *out, const DecMoe &moe, const int8_t *q_split, c
 bool launch_w4a8_dec_moe_glu(const DecMoe &moe, const int8_t *q_split, const float *scales, const float *sums,
                              int rows, int cols, int gs, int max_entries, hipStream_t s);
 
-// Matrix-core W4A8 for 2..64 tokens (past 64 the GEMM of gemm_mm.hip is faster
-// on every measured shape).  The register-pipelined kernel of gemv.hip:
-// group 32, K a multiple of 512 up to 14336; it builds its operands from the
-// block-split int8 activations.  `params_tiled` (may be null): the same
-// parameters in the layout of launch_params_tile16, read instead of `params`
-// where it applies.
-constexpr int kMfmaMaxTokens = 64;
+// Kernel of a W4A8 product of m >= 2 tokens over whole groups of 32, 64 or 128
+// (w4a8_route).  kRp: the register-pipelined kernel of gemv.hip, which builds
+// its operands from the block-split int8 activations; kStream: the streamed
+// kernel of gemv_stream.hip, with the activations in its lane order (`qa`,
+// qa_bytes of them, written by the quantizing kernels below; rows of tokens
+// past m are not read); kMm: the GEMM of gemm_mm.hip, which packs the
+// block-split activations into `mm` scratch; kValu: the VALU kernels (2 GiB
+// matrices).
+enum class W4Route { kRp, kStream, kMm, kValu };
+W4Route w4a8_route(int rows, int cols, int m, int gs);
+// `params_tiled` (may be null): the same parameters in the layout of
+// launch_params_tile16, read instead of `params` where it applies.
 bool gemv_rp_path(int rows, int cols, int m, int gs);
 void launch_gemv_rp(float *out, const float *add, const uint8_t *nib, const uint8_t *params, const int8_t *q_split,
                     const float *scales, const float *sums, int rows, int cols, int m, hipStream_t s,
                     const uint8_t *params_tiled);
-bool gemv_rp_cols(int cols, int gs);
-// The streamed kernel of gemv_stream.hip: whole groups of 32, 64 or 128, the
-// activations in its lane order (`qa`, qa_bytes of them, written by the
-// quantizing kernels below; rows of tokens past m are not read).
-bool gemv_stream_path(int rows, int cols, int m, int gs);
 // One step's activations: gs / 8 blocks of 64 lanes x 8 f16, then 64 scales
 // and 64 input sums.
 constexpr int qa_rec_bytes(int gs) { return gs * 128 + 512; }
 size_t qa_bytes(int m, int cols, int gs);
 void launch_gemv_stream(float *out, const float *add, const uint8_t *nib, const uint8_t *params, const _Float16 *qa,
                         int rows, int cols, int m, int gs, hipStream_t s);
-// True when a product over `cols` columns wants its activations as `qa`.
-inline bool w4a8_wants_qa(int cols, int m, int gs) {
-  return !gemv_rp_cols(cols, gs) && gemv_stream_path(1, cols, m, gs);
-}
 // The parameter array of a group-32 matrix (rows x cols/32 dwords, f16
 // scale and zero point per row and group) rearranged in 16-row tiles:
 // [rows / 16][cols / 128][16 rows][4 groups] dwords, the layout the
@@ -135,10 +131,9 @@ inline bool w4a8_wants_qa(int cols, int m, int gs) {
 // size as the input; requires params_tile16_ok.
 bool params_tile16_ok(int rows, int cols, int gs);
 void launch_params_tile16(const uint8_t *params, int rows, int cols, uint8_t *tiled, hipStream_t s);
-// Matrix-core W4A8 GEMM (gemm_mm.hip): whole groups of 32, 64 or 128,
-// more than kMfmaMaxTokens tokens.  Packs the block-split activations into
-// `pack` (mm_pack_bytes(m, cols, gs) bytes), then runs the GEMM.
-bool w4a8_mm_path(int rows, int cols, int m, int gs);
+// Matrix-core W4A8 GEMM (gemm_mm.hip): whole groups of 32, 64 or 128.  Packs
+// the block-split activations into `pack` (mm_pack_bytes(m, cols, gs) bytes),
+// then runs the GEMM.
 size_t mm_pack_bytes(int m, int cols, int gs);
 void launch_w4a8_mm(float *out, const float *add, const uint8_t *nib, const uint8_t *params, const int8_t *q_split,
                     const float *scales, const float *sums, int rows, int cols, int m, int gs, uint8_t *pack,

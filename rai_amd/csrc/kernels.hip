@@ -1451,17 +1451,20 @@ void launch_w4a8(float *out, const float *add, const uint8_t *nib, const uint8_t
                        sums, rows, cols, m, gs, groups);
     return;
   }
-  if (gemv_rp_path(rows, cols, m, gs)) {
-    launch_gemv_rp(out, add, nib, params, q_split, scales, sums, rows, cols, m, s, params_tiled);
-    return;
-  }
-  if (qa && gemv_stream_path(rows, cols, m, gs)) {
-    launch_gemv_stream(out, add, nib, params, qa, rows, cols, m, gs, s);
-    return;
-  }
-  if (mm && w4a8_mm_path(rows, cols, m, gs)) {
-    launch_w4a8_mm(out, add, nib, params, q_split, scales, sums, rows, cols, m, gs, mm, s);
-    return;
+  if (m > 1) {
+    const W4Route route = w4a8_route(rows, cols, m, gs);
+    if (route == W4Route::kRp) {
+      launch_gemv_rp(out, add, nib, params, q_split, scales, sums, rows, cols, m, s, params_tiled);
+      return;
+    }
+    if (qa && route == W4Route::kStream) {
+      launch_gemv_stream(out, add, nib, params, qa, rows, cols, m, gs, s);
+      return;
+    }
+    if (mm && route == W4Route::kMm) {
+      launch_w4a8_mm(out, add, nib, params, q_split, scales, sums, rows, cols, m, gs, mm, s);
+      return;
+    }
   }
   if (m == 1 &&
       launch_w4a8_dec(out, add, nib, params, q_split, scales, sums, rows, cols, gs, nullptr, nullptr, 0.0f, s))
@@ -1504,7 +1507,7 @@ void launch_w4a8(float *out, const float *add, const uint8_t *nib, const uint8_t
       launch_small_mt<128, 1>(out, add, nib, params, q_split, scales, sums, rows, cols, m, groups, s);
     return;
   }
-  // Several tokens and a matrix of 2 GiB or more.
+  // Several tokens and a matrix of 2 GiB or more (or no scratch for them).
   if (gs == 32)
     launch_fast_gs<32>(out, add, nib, params, q_split, scales, sums, rows, cols, m, groups, s);
   else if (gs == 64)

@@ -147,6 +147,9 @@ class CallScratch {
   bool done_ = false;
 };
 
+// Tokens up to which a sparse layer runs entry by entry.
+constexpr int kMoeEntryTokens = 64;
+
 struct DevBuf {
   void *p = nullptr;
   DevBuf() = default;
@@ -233,8 +236,8 @@ struct Workspace {
   DevBuf hid, normed, qb, kb, vb, att, ob, gb, ub, mo, logits, am;
   DevBuf qkvb, gub;  // fused q|k|v and gate|up outputs [m][rows]
   DevBuf q_nat, q_split, qscale, qsum, hq;
-  DevBuf qa;   // activations packed for the matrix-core W4A8 kernel (<= 64 tokens)
-  DevBuf qmm;  // activation records of the matrix-core W4A8 GEMM (> 64 tokens)
+  DevBuf qa;   // activations in the streamed W4A8 kernel's lane order
+  DevBuf qmm;  // activation records of the matrix-core W4A8 GEMM (> 16 tokens)
   DevBuf err;
   // Attention score/probability rows; grown to the largest KV capacity seen.
   DevBuf scores;
@@ -277,8 +280,8 @@ struct Workspace {
     am.alloc(sizeof(uint32_t) * maxm);
     q_nat.alloc(K * maxm);
     q_split.alloc(K * maxm);
-    qa.alloc(qa_bytes(std::min(maxm, kMfmaMaxTokens), (int)K, (int)c.group_size));
-    if (maxm > kMfmaMaxTokens) qmm.alloc(mm_pack_bytes(maxm, (int)K, (int)c.group_size));
+    qa.alloc(qa_bytes(maxm, (int)K, (int)c.group_size));
+    if (maxm > 16) qmm.alloc(mm_pack_bytes(maxm, (int)K, (int)c.group_size));
     hq.alloc(H * maxm);
     qscale.alloc(sizeof(float) * G * maxm);
     qsum.alloc(sizeof(float) * G * maxm);
@@ -297,7 +300,7 @@ struct Workspace {
       moff.alloc(sizeof(int) * (c.num_experts + 2));  // and the tile count
       const int nt = moe_max_tiles((int)ne, (int)c.num_experts);
       mtiles.alloc(sizeof(int4) * nt);
-      if (maxm > kMfmaMaxTokens && moe_device_path((int)H, (int)F, (int)c.group_size, (int)c.num_experts))
+      if (maxm > kMoeEntryTokens && moe_device_path((int)H, (int)F, (int)c.group_size, (int)c.num_experts))
         qmm.alloc(std::max(mm_pack_bytes(maxm, (int)K, (int)c.group_size),
                            mm_pack_tiles_bytes(nt, (int)std::max(H, F), (int)c.group_size)));
       ment_of.alloc(sizeof(int) * ne);
@@ -568,17 +571,20 @@ static void linear(const DLinear &L, const float *x, const Workspace &w, float *
               w.qa.as<_Float16>(), w.qmm.as<uint8_t>(), L.params_tiled);
 }
 
-// The matrix-core activation buffer for a fused quantizer to fill directly
-// (null when no product on these rows reads it).
-static _Float16 *mfma_acts(const rai_model &md, int m, int k, const Workspace &w) {
-  return w4a8_wants_qa(k, m, md.cfg.group_size) ? w.qa.as<_Float16>() : nullptr;
+// The lane-order activation buffer for a quantizer of m rows of k columns to
+// fill: null unless a product on them, of r0, r1 or r2 rows (0: none), takes the
+// streamed kernel.
+static _Float16 *stream_acts(const rai_model &md, int m, int k, const Workspace &w, int r0, int r1 = 0, int r2 = 0) {
+  auto wants = [&](int r) { return r > 0 && m > 1 && w4a8_route(r, k, m, md.cfg.group_size) == W4Route::kStream; };
+  return wants(r0) || wants(r1) || wants(r2) ? w.qa.as<_Float16>() : nullptr;
 }
 
+// For products of r0 and r1 (0: none) rows.
 static void quantize(const rai_model &md, const float *x, int m, int k, const Workspace &w,
-                     hipStream_t s) {
+                     hipStream_t s, int r0, int r1 = 0, int r2 = 0) {
   if (fused_quant_ok(k, md.cfg.group_size)) {
     launch_quant(x, m, k, md.cfg.group_size, w.q_split.as<int8_t>(), nullptr, w.qscale.as<float>(),
-                 w.qsum.as<float>(), s, mfma_acts(md, m, k, w));
+                 w.qsum.as<float>(), s, stream_acts(md, m, k, w, r0, r1, r2));
   } else {
     launch_quantize(x, m, k, md.cfg.group_size, w.q_nat.as<int8_t>(), w.q_split.as<int8_t>(),
                     w.qscale.as<float>(), w.qsum.as<float>(), s);
@@ -647,7 +653,7 @@ static void moe_block_device(const rai_model &md, int li, Workspace &w, int m, h
   launch_moe_combine(w.hid.as<float>(), w.eo.as<float>(), w.wts.as<float>(), w.ment_of.as<int>(), m, K, H, s);
 }
 
-// Prefill-sized batches (more than kMfmaMaxTokens tokens): the plan splits
+// Prefill-sized batches (more than kMoeEntryTokens tokens): the plan splits
 // every expert's entries into tiles of at most 32, and one GEMM launch per
 // projection runs all tiles of all experts (launch_moe_mm), so the chip is
 // filled whatever the counts are and the host waits for nothing.  Against one
@@ -712,11 +718,11 @@ static void moe_block(const rai_model &md, const DLayer &L, Workspace &w, int m,
       HIP_CHECK(hipMemcpyAsync(w.xg.as<float>() + (size_t)i * H, w.normed.as<float>() + (size_t)tok[e][i] * H,
                                sizeof(float) * H, hipMemcpyDeviceToDevice, s));
     const DLinear *ex = &L.experts[(size_t)e * 3];
-    quantize(md, w.xg.as<float>(), me, H, w, s);
+    quantize(md, w.xg.as<float>(), me, H, w, s, ex[0].rows, ex[1].rows);
     linear(ex[0], w.xg.as<float>(), w, w.gg.as<float>(), me, s);
     linear(ex[1], w.xg.as<float>(), w, w.ug.as<float>(), me, s);
     launch_silu_mul(w.gg.as<float>(), w.ug.as<float>(), me, F, s);
-    quantize(md, w.gg.as<float>(), me, F, w, s);
+    quantize(md, w.gg.as<float>(), me, F, w, s, ex[2].rows);
     linear(ex[2], w.gg.as<float>(), w, w.yg.as<float>(), me, s);
     for (int i = 0; i < me; ++i)
       HIP_CHECK(hipMemcpyAsync(eo + ((size_t)tok[e][i] * K + slot[e][i]) * H, w.yg.as<float>() + (size_t)i * H,
@@ -772,13 +778,13 @@ static void forward_enqueue(rai_model &md, rai_kv &kv, Workspace &w, int m, size
   // enter_block (model.rs:319-337): RMSNorm, then one quantization of the
   // normalised rows shared by the projections that read them (the
   // reference re-quantizes per projection; the result is identical).
-  auto norm_then_quant = [&](const float *wn) {
+  auto norm_then_quant = [&](const float *wn, int r0, int r1, int r2) {
     if (fused_quant_ok(H, gs)) {
       launch_norm_quant(hid, wn, normed, m, H, c.norm_eps, gs, w.q_split.as<int8_t>(), nullptr,
-                        w.qscale.as<float>(), w.qsum.as<float>(), s, mfma_acts(md, m, H, w));
+                        w.qscale.as<float>(), w.qsum.as<float>(), s, stream_acts(md, m, H, w, r0, r1, r2));
     } else {
       launch_rmsnorm(hid, wn, normed, nullptr, m, H, c.norm_eps, s);
-      quantize(md, normed, m, H, w, s);
+      quantize(md, normed, m, H, w, s, r0, r1, r2);
     }
   };
   // One token: the projections behind a norm normalise and quantize the
@@ -788,7 +794,12 @@ static void forward_enqueue(rai_model &md, rai_kv &kv, Workspace &w, int m, size
   for (int li = 0; li < (int)c.num_layers; ++li) {
     const DLayer &L = md.layers[li];
     const bool qkv1 = norm1 && L.qkv.rows && w4a8_norm1_path(L.qkv.rows, L.qkv.cols, L.qkv.gs);
-    if (!qkv1) norm_then_quant(L.in_norm);
+    if (!qkv1) {
+      if (L.qkv.rows)
+        norm_then_quant(L.in_norm, L.qkv.rows, 0, 0);
+      else
+        norm_then_quant(L.in_norm, L.lin[0].rows, L.lin[1].rows, L.lin[2].rows);
+    }
     float *qp, *kp, *vp;
     int q_ld, kv_ld;
     // One token: the qkv launch also rotates q and k and stores k and v
@@ -832,13 +843,15 @@ static void forward_enqueue(rai_model &md, rai_kv &kv, Workspace &w, int m, size
     const DLinear &O = L.lin[3];
     if (!(norm1 && launch_w4a8_dec(hid, hid, O.nib, O.params, nullptr, nullptr, nullptr, O.rows, O.cols, O.gs,
                                    w.att.as<float>(), nullptr, 0.0f, s))) {
-      quantize(md, w.att.as<float>(), m, qd, w, s);
+      quantize(md, w.att.as<float>(), m, qd, w, s, O.rows);
       linear(O, w.att.as<float>(), w, hid, m, s, hid);
     }
     const bool gu1 = norm1 && L.gate_up.rows && fused_quant_ok(F, gs) &&
                      w4a8_norm1_path(L.gate_up.rows, L.gate_up.cols, L.gate_up.gs);
-    if (!gu1) norm_then_quant(L.post_norm);
-    if (c.num_experts > 0 && moe_on_device(md) && m > kMfmaMaxTokens && moe_tiles_ok(c)) {
+    // gate|up as one product or two (a sparse layer's experts read the rows
+    // themselves).
+    if (!gu1) norm_then_quant(L.post_norm, c.num_experts ? 0 : L.gate_up.rows, c.num_experts ? 0 : F, 0);
+    if (c.num_experts > 0 && moe_on_device(md) && m > kMoeEntryTokens && moe_tiles_ok(c)) {
       moe_block_device_large(md, li, w, m, s);
     } else if (c.num_experts > 0 && moe_on_device(md)) {
       moe_block_device(md, li, w, m, s);
@@ -875,10 +888,10 @@ static void forward_enqueue(rai_model &md, rai_kv &kv, Workspace &w, int m, size
       }
       if (fused_quant_ok(F, gs)) {
         launch_silu_quant(gp, up, m, F, gu_ld, gs, w.q_split.as<int8_t>(), nullptr, w.qscale.as<float>(),
-                          w.qsum.as<float>(), s, mfma_acts(md, m, F, w));
+                          w.qsum.as<float>(), s, stream_acts(md, m, F, w, L.lin[6].rows));
       } else {
         launch_silu_mul(gp, up, m, F, s);
-        quantize(md, gp, m, F, w, s);
+        quantize(md, gp, m, F, w, s, L.lin[6].rows);
       }
       // down with the second residual add (model.rs:955-960) in its epilogue.
       linear(L.lin[6], gp, w, hid, m, s, hid);
@@ -906,10 +919,10 @@ static void logits(rai_model &md, Workspace &w, int m, hipStream_t s) {
     if (fused_quant_ok(H, c.group_size)) {
       launch_norm_quant(w.hid.as<float>(), md.final_norm, w.normed.as<float>(), m, H, c.norm_eps, c.group_size,
                         w.q_split.as<int8_t>(), nullptr, w.qscale.as<float>(), w.qsum.as<float>(), s,
-                        mfma_acts(md, m, H, w));
+                        stream_acts(md, m, H, w, md.lm_head.rows));
     } else {
       launch_rmsnorm(w.hid.as<float>(), md.final_norm, w.normed.as<float>(), nullptr, m, H, c.norm_eps, s);
-      quantize(md, w.normed.as<float>(), m, H, w, s);
+      quantize(md, w.normed.as<float>(), m, H, w, s, md.lm_head.rows);
     }
     linear(md.lm_head, w.normed.as<float>(), w, w.logits.as<float>(), m, s);
   } else {
@@ -1463,8 +1476,9 @@ int rai_w4a8_matmul_dev(float *out, const uint8_t *nib, const uint8_t *params, c
       return RAI_OK;
     }
     const bool fast = rai::w4a8_fast_path((int)cols, (int)gs, nib, params);
-    const bool wqa = fast && rai::w4a8_wants_qa((int)cols, (int)m, (int)gs);
-    const bool mm = fast && rai::w4a8_mm_path((int)rows, (int)cols, (int)m, (int)gs);
+    const rai::W4Route route = m > 1 && fast ? rai::w4a8_route((int)rows, (int)cols, (int)m, (int)gs)
+                                             : rai::W4Route::kValu;
+    const bool wqa = route == rai::W4Route::kStream, mm = route == rai::W4Route::kMm;
     const size_t nq = m * cols, ng = m * groups * 4;
     const size_t nqa = wqa ? rai::qa_bytes((int)m, (int)cols, (int)gs) : 0;
     const size_t nmm = mm ? rai::mm_pack_bytes((int)m, (int)cols, (int)gs) : 0;
@@ -1607,14 +1621,15 @@ int rai_w4a8_matmul_noalloc_dev(float *out, const uint8_t *nib, const uint8_t *p
                                  std::to_string(rai::kNaTokenCols) + " token columns and " +
                                  std::to_string(rai::kNaGroups) + " token groups)");
     const bool fast = rai::w4a8_fast_path((int)cols, (int)gs, nib, params);
-    // The streamed kernel's activations share the records' place; past its
-    // size (two tokens of more than 393216 columns) the product takes the
+    // The streamed kernel's activations and the GEMM's records share a place;
+    // what does not fit it (two tokens of more than 393216 columns) takes the
     // tiled VALU kernel.
-    const bool wqa = fast && rai::w4a8_wants_qa((int)cols, (int)m, (int)gs) &&
+    const rai::W4Route route = m > 1 && fast ? rai::w4a8_route((int)rows, (int)cols, (int)m, (int)gs)
+                                             : rai::W4Route::kValu;
+    const bool wqa = route == rai::W4Route::kStream &&
                      rai::qa_bytes((int)m, (int)cols, (int)gs) <= rai::kNaMmBytes;
-    const bool mm = fast && rai::w4a8_mm_path((int)rows, (int)cols, (int)m, (int)gs);
-    if (mm && rai::mm_pack_bytes((int)m, (int)cols, (int)gs) > rai::kNaMmBytes)
-      rai::fail(RAI_E_SHAPE, "activation records exceed the allocation-free scratch");
+    const bool mm = route == rai::W4Route::kMm &&
+                    rai::mm_pack_bytes((int)m, (int)cols, (int)gs) <= rai::kNaMmBytes;
     uint8_t *base = rai::noalloc_scratch();
     int8_t *qn = reinterpret_cast<int8_t *>(base);
     int8_t *qs = reinterpret_cast<int8_t *>(base + rai::kNaTokenCols);
@@ -1657,18 +1672,18 @@ int rai_w4a8_time_dev(float *out, const uint8_t *nib, const uint8_t *params, con
     HIP_CHECK(hipEventCreate(&e0));
     HIP_CHECK(hipEventCreate(&e1));
     const bool fast = rai::w4a8_fast_path((int)cols, (int)gs, nib, params);
-    const bool mfma = fast && rai::gemv_rp_path((int)rows, (int)cols, (int)m, (int)gs);
+    const rai::W4Route route = m > 1 && fast ? rai::w4a8_route((int)rows, (int)cols, (int)m, (int)gs)
+                                             : rai::W4Route::kValu;
     rai::DevBuf qa, mm;
-    if (fast && rai::w4a8_wants_qa((int)cols, (int)m, (int)gs)) qa.alloc(rai::qa_bytes((int)m, (int)cols, (int)gs));
+    if (route == rai::W4Route::kStream) qa.alloc(rai::qa_bytes((int)m, (int)cols, (int)gs));
     rai::quantize_call(x, (int)m, (int)cols, (int)gs, fast,
                        {qn.as<int8_t>(), qs.as<int8_t>(), sc.as<float>(), su.as<float>(), qa.as<_Float16>(), nullptr},
                        s);
-    if (fast && rai::w4a8_mm_path((int)rows, (int)cols, (int)m, (int)gs))
-      mm.alloc(rai::mm_pack_bytes((int)m, (int)cols, (int)gs));
+    if (route == rai::W4Route::kMm) mm.alloc(rai::mm_pack_bytes((int)m, (int)cols, (int)gs));
     const size_t nib_bytes = rows * cols / 2, par_bytes = rows * groups * 4;
     // The parameters' tile-layout copies, as a loaded model holds them.
     rai::DevBuf tiled;
-    if (mfma && rai::params_tile16_ok((int)rows, (int)cols, (int)gs)) {
+    if (route == rai::W4Route::kRp && rai::params_tile16_ok((int)rows, (int)cols, (int)gs)) {
       tiled.alloc(copies * par_bytes);
       for (size_t c = 0; c < copies; ++c)
         rai::launch_params_tile16(params + c * par_bytes, (int)rows, (int)cols, tiled.as<uint8_t>() + c * par_bytes,

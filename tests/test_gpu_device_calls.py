@@ -50,24 +50,44 @@ def _tokens(x, m, cols, gs, seed):
 
 # K: one group, fewer groups than a step or a stage of the kernel, one past a
 # stage, several stages with a remainder.
-MM = [(32, 32), (32, 96), (32, 544), (32, 1568), (32, 2048), (64, 64), (64, 320), (64, 576), (64, 1728),
+MM = [(32, 32), (32, 96), (32, 544), (32, 1568), (64, 64), (64, 320), (64, 576), (64, 1728),
       (128, 128), (128, 384), (128, 640), (128, 2176)]
+
+
+def _both_calls(rai, ora, rows, cols, m, gs, specials=(False, True)):
+    nib, params, x = gemv_operands(rows, cols, m, gs, seed=rows + cols + m)
+    dev = rai.DeviceArray.from_host
+    dn, dp, do = dev(nib), dev(params), rai.DeviceArray(4 * m * rows)
+    for special in specials:
+        if special:
+            x = _tokens(x, m, cols, gs, cols + m)
+        want = ora.w4a8_matmul(nib, params, x, rows, cols, m, gs)
+        xd = dev(np.ascontiguousarray(x, np.float32))
+        names = ["rai_w4a8_matmul_dev"]
+        if m * cols <= 1 << 20:
+            names.append("rai_w4a8_matmul_noalloc_dev")
+        for name in names:
+            got = _call(rai, name, do, dn, dp, xd, rows, cols, m, gs)
+            assert np.array_equal(_bits(got).reshape(-1), _bits(want).reshape(-1)), (name, special)
+
+
+@pytest.mark.parametrize("gs,cols", MM)
+def test_gemm_every_group_size(rai, ora, gs, cols):
+    """Enough row and token tiles for the matrix-core GEMM: a last row tile of
+    31 rows, a last token tile of one token."""
+    _both_calls(rai, ora, 2111, cols, 545, gs)
+
+
+@pytest.mark.parametrize("gs,cols", [(32, 96), (64, 192), (128, 128)])
+@pytest.mark.parametrize("rows,m", [(36097, 33), (72100, 25)])
+def test_gemm_many_rows_few_tokens(rai, ora, gs, cols, rows, m):
+    _both_calls(rai, ora, rows, cols, m, gs)
 
 
 @pytest.mark.parametrize("gs,cols", MM)
 @pytest.mark.parametrize("rows,m", [(1, 65), (127, 96), (130, 97), (300, 160)])
-def test_gemm_every_group_size(rai, ora, gs, cols, rows, m):
-    """More than 64 tokens: the matrix-core GEMM."""
-    nib, params, x = gemv_operands(rows, cols, m, gs, seed=rows + cols + m)
-    for special in (False, True):
-        if special:
-            x = _tokens(x, m, cols, gs, cols + m)
-        want = ora.w4a8_matmul(nib, params, x, rows, cols, m, gs)
-        dev = rai.DeviceArray.from_host
-        xd = dev(np.ascontiguousarray(x, np.float32))
-        for name in ("rai_w4a8_matmul_dev", "rai_w4a8_matmul_noalloc_dev"):
-            got = _call(rai, name, rai.DeviceArray(4 * m * rows), dev(nib), dev(params), xd, rows, cols, m, gs)
-            assert np.array_equal(_bits(got).reshape(-1), _bits(want).reshape(-1)), (name, special)
+def test_streamed_kernel_past_64_tokens(rai, ora, gs, cols, rows, m):
+    _both_calls(rai, ora, rows, cols, m, gs)
 
 
 @pytest.mark.parametrize("gs,experts,topk,m", [(32, 8, 3, 70), (64, 16, 2, 150), (128, 5, 5, 65), (32, 64, 8, 97)])
@@ -158,20 +178,11 @@ def test_decode_steps_every_group_size(rai, ora, gs, hidden, heads, kv, hd, ffn,
 def test_small_batches_every_group_size(rai, ora, gs, cols, rows, m):
     if rows > 1000 and cols > 700:
         cols = 4 * gs + gs  # the oracle's time
-    nib, params, x = gemv_operands(rows, cols, m, gs, seed=rows + cols + m)
-    for special in (False, True):
-        if special:
-            x = _tokens(x, m, cols, gs, cols + m)
-        want = ora.w4a8_matmul(nib, params, x, rows, cols, m, gs)
-        dev = rai.DeviceArray.from_host
-        xd = dev(np.ascontiguousarray(x, np.float32))
-        for name in ("rai_w4a8_matmul_dev", "rai_w4a8_matmul_noalloc_dev"):
-            got = _call(rai, name, rai.DeviceArray(4 * m * rows), dev(nib), dev(params), xd, rows, cols, m, gs)
-            assert np.array_equal(_bits(got).reshape(-1), _bits(want).reshape(-1)), (name, special)
+    _both_calls(rai, ora, rows, cols, m, gs)
 
 
-@pytest.mark.parametrize("gs", [64, 128])
-@pytest.mark.parametrize("m", [2, 9, 40])
+@pytest.mark.parametrize("gs", [32, 64, 128])
+@pytest.mark.parametrize("m", [2, 9, 40, 100])
 def test_small_batch_layers(rai, ora, gs, m):
     """The model path: norm, attention output, silu_mul and head activations
     in the streamed kernel's order."""
