@@ -177,6 +177,9 @@ int rai_forward_from_hidden(rai_model *model, rai_kv *kv, float *hidden, size_t 
  * positions strictly consecutive. */
 int rai_forward_batch(rai_model *model, rai_kv *kv, float *hiddens, const size_t *positions,
                       size_t batch);
+/* The same from `in` to `out` (which may be one buffer), `in` left as it is. */
+int rai_forward_batch_to(rai_model *model, rai_kv *kv, const float *in, float *out, const size_t *positions,
+                         size_t batch);
 /* RaiModel::hidden_to_logits_into (model.rs:504-548). */
 int rai_hidden_to_logits(rai_model *model, const float *hidden, float *logits);
 /* RaiModel::hidden_to_logits_batch (model.rs:966-1033). */

@@ -120,6 +120,7 @@ def lib():
         "rai_embed_token": (c_int, [P, S, P]),
         "rai_forward_from_hidden": (c_int, [P, P, P, S, c_int]),
         "rai_forward_batch": (c_int, [P, P, P, P, S]),
+        "rai_forward_batch_to": (c_int, [P, P, P, P, P, S]),
         "rai_hidden_to_logits": (c_int, [P, P, P]),
         "rai_hidden_to_logits_batch": (c_int, [P, P, P, S]),
         "rai_w4a8_matmul_dev": (c_int, [P, P, P, P, S, S, S, S, P]),
@@ -586,10 +587,11 @@ class RaiModel:
         return h
 
     def forward_batch(self, hiddens, positions, kv: "KVCache") -> np.ndarray:
-        h = _f32(hiddens).copy()
+        h = _f32(hiddens)
+        out = np.empty_like(h)
         p = np.ascontiguousarray(positions, np.uint64)
-        _check(lib().rai_forward_batch(self.h, kv.h, _ptr(h), _ptr(p), p.size))
-        return h
+        _check(lib().rai_forward_batch_to(self.h, kv.h, _ptr(h), _ptr(out), _ptr(p), p.size))
+        return out
 
     def hidden_to_logits(self, hidden) -> np.ndarray:
         out = np.zeros(self.config.vocab_size, np.float32)
@@ -598,7 +600,7 @@ class RaiModel:
         return out
 
     def hidden_to_logits_batch(self, hiddens, batch: int) -> np.ndarray:
-        out = np.zeros(batch * self.config.vocab_size, np.float32)
+        out = np.empty(batch * self.config.vocab_size, np.float32)
         h = _f32(hiddens)  # kept alive across the call
         _check(lib().rai_hidden_to_logits_batch(self.h, _ptr(h), _ptr(out), batch))
         return out.reshape(batch, self.config.vocab_size)

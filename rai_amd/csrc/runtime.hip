@@ -16,6 +16,7 @@
 
 #include "common.h"
 #include "format.h"
+#include "host_io.h"
 #include "kernels.h"
 
 namespace rai {
@@ -146,6 +147,159 @@ class CallScratch {
   size_t used_ = 0;
   bool done_ = false;
 };
+
+// dst[0..n) = src[0..n) in dwords; n16 of them in 16-byte units where both
+// are aligned for it.  Either side may be pinned host memory.
+__global__ __launch_bounds__(256) void k_host_copy(uint32_t *__restrict__ dst, const uint32_t *__restrict__ src,
+                                                   size_t n, size_t n16, uint32_t *__restrict__ dst2,
+                                                   const uint32_t *__restrict__ src2, int n2) {
+  const size_t i0 = (size_t)blockIdx.x * blockDim.x + threadIdx.x, step = (size_t)gridDim.x * blockDim.x;
+  if (i0 < (size_t)n2) dst2[i0] = src2[i0];
+  for (size_t i = i0; i < n16; i += step)
+    reinterpret_cast<uint4 *>(dst)[i] = reinterpret_cast<const uint4 *>(src)[i];
+  for (size_t i = 4 * n16 + i0; i < n; i += step) dst[i] = src[i];
+}
+
+// Copies n floats (and n2 dwords of src2) on stream s; device memory to pinned
+// or back.
+static void host_copy(void *dst, const void *src, size_t n, hipStream_t s, void *dst2 = nullptr,
+                      const void *src2 = nullptr, int n2 = 0) {
+  const size_t n16 = ((uintptr_t)dst | (uintptr_t)src) % 16 == 0 ? n / 4 : 0;
+  const size_t items = std::max<size_t>(n16 ? n16 : n, 1);
+  const int blocks = (int)std::min<size_t>((items + 255) / 256, 1024);
+  hipLaunchKernelGGL(k_host_copy, dim3(blocks), dim3(256), 0, s, static_cast<uint32_t *>(dst),
+                     static_cast<const uint32_t *>(src), n, n16, static_cast<uint32_t *>(dst2),
+                     static_cast<const uint32_t *>(src2), n2);
+}
+
+// A call's pinned staging, from a process-wide pool (pinning pages costs
+// milliseconds): a call holds its block alone until its stream is finished.
+// A transfer is cut into pieces of at most half of kStageMax; at most two
+// blocks are kept.
+class HostStage {
+ public:
+  static constexpr size_t kStageMax = size_t(32) << 20;
+  // For transfers of up to nin floats in and nout out at a time.
+  HostStage(hipStream_t s, size_t nin, size_t nout) : s_(s) {
+    take(bytes(std::min(nin, kPiece)) + bytes(std::min(nout, kPiece)));
+  }
+  HostStage(const HostStage &) = delete;
+  HostStage &operator=(const HostStage &) = delete;
+  ~HostStage() { give(hipStreamSynchronize(s_) == hipSuccess); }
+
+  // dst (device) = src (host), n floats, on the stream.  Returns with the
+  // source read and the block in use until the stream passes this point.
+  void in(float *dst, const float *src, size_t n) {
+    for (size_t o = 0; o < n; o += kPiece) {
+      const size_t k = std::min(kPiece, n - o);
+      if (o) HIP_CHECK(hipStreamSynchronize(s_));
+      float *pin = reinterpret_cast<float *>(b_.p);
+      const size_t part = part_floats(k);
+      for (size_t i = 0; i < k; i += part) {
+        const size_t kk = std::min(part, k - i);
+        CopyPool::get().copy(pin + i, src + o + i, kk * sizeof(float));
+        host_copy(dst + o + i, pin + i, kk, s_);
+      }
+    }
+  }
+  // dst (host) = src (device), n floats; and 2 words of err to e (host) when
+  // given.  Returns with the stream finished.
+  void out(float *dst, const float *src, size_t n, const int *err = nullptr, int *e = nullptr) {
+    for (size_t o = 0; o < n; o += kPiece) {
+      const size_t k = std::min(kPiece, n - o);
+      // At the end of the block, so that in()'s copy may still be under way.
+      float *pin = reinterpret_cast<float *>(b_.p + b_.n - 64 - bytes(k));
+      int *pe = reinterpret_cast<int *>(b_.p + b_.n - 64);
+      const size_t part = part_floats(k);
+      int np = 0;
+      for (size_t i = 0; i < k; i += part, ++np) {
+        const bool last = err && i + part >= k;
+        host_copy(pin + i, src + o + i, std::min(part, k - i), s_, pe, err, last ? 2 : 0);
+        HIP_CHECK(hipGetLastError());
+        if (part < k) HIP_CHECK(hipEventRecord(b_.ev[np], s_));
+      }
+      if (part >= k) {
+        HIP_CHECK(hipStreamSynchronize(s_));
+        CopyPool::get().copy(dst + o, pin, k * sizeof(float));
+      } else {
+        for (int p = 0; p < np; ++p) {
+          HIP_CHECK(hipEventSynchronize(b_.ev[p]));
+          CopyPool::get().copy(dst + o + p * part, pin + p * part, std::min(part, k - p * part) * sizeof(float));
+        }
+        HIP_CHECK(hipStreamSynchronize(s_));
+      }
+      if (e) e[0] = pe[0], e[1] = pe[1];
+    }
+  }
+
+ private:
+  static constexpr size_t kPiece = kStageMax / sizeof(float) / 2;
+  static size_t bytes(size_t n) { return (n * sizeof(float) + 63) & ~size_t(63); }
+  // A transfer's parts: up to eight of at least 2 MB, so that the host's copy
+  // of one overlaps the device's of the next.
+  static size_t part_floats(size_t k) {
+    const size_t least = (size_t(2) << 20) / sizeof(float);
+    return std::max(least, ((k + PinBlock::kEvents - 1) / PinBlock::kEvents + 15) & ~size_t(15));
+  }
+  void take(size_t n) {
+    n += 64;  // the error words
+    int dev = 0;
+    HIP_CHECK(hipGetDevice(&dev));
+    {
+      std::lock_guard<std::mutex> lk(g_m);
+      for (size_t i = 0; i < g_pins.size(); ++i)
+        if (g_pins[i].dev == dev && g_pins[i].n >= n) {
+          b_ = g_pins[i];
+          g_pins.erase(g_pins.begin() + i);
+          return;
+        }
+    }
+    size_t want = size_t(1) << 20;
+    while (want < n) want *= 2;
+    PinBlock b;
+    b.dev = dev;
+    HIP_CHECK(hipHostMalloc(reinterpret_cast<void **>(&b.p), want, hipHostMallocDefault));
+    b.n = want;
+    for (auto &ev : b.ev) {
+      const hipError_t r = hipEventCreateWithFlags(&ev, hipEventDisableTiming);
+      if (r != hipSuccess) {
+        drop(b);
+        HIP_CHECK(r);
+      }
+    }
+    b_ = b;
+  }
+  // Keeps the block for the next call (the larger ones first), or frees it.
+  void give(bool keep) {
+    if (!b_.p) return;
+    PinBlock out = b_;
+    b_ = PinBlock{};
+    if (keep) {
+      std::lock_guard<std::mutex> lk(g_m);
+      g_pins.push_back(out);
+      out.p = nullptr;
+      if (g_pins.size() > 2) {
+        size_t least = 0;
+        for (size_t i = 1; i < g_pins.size(); ++i)
+          if (g_pins[i].n < g_pins[least].n) least = i;
+        out = g_pins[least];
+        g_pins.erase(g_pins.begin() + least);
+      }
+    }
+    if (out.p) drop(out);
+  }
+  static void drop(PinBlock &b) {
+    for (auto ev : b.ev)
+      if (ev) (void)hipEventDestroy(ev);
+    (void)hipHostFree(b.p);
+  }
+  static std::mutex g_m;
+  static std::vector<PinBlock> g_pins;
+  hipStream_t s_;
+  PinBlock b_;
+};
+std::mutex HostStage::g_m;
+std::vector<PinBlock> HostStage::g_pins;
 
 // Tokens up to which a sparse layer runs entry by entry.
 constexpr int kMoeEntryTokens = 64;
@@ -1364,9 +1518,10 @@ int rai_embed_token(rai_model *m, size_t token, float *out) {
   });
 }
 
-int rai_forward_batch(rai_model *m, rai_kv *kv, float *hiddens, const size_t *positions, size_t batch) {
+int rai_forward_batch_to(rai_model *m, rai_kv *kv, const float *in, float *out, const size_t *positions,
+                         size_t batch) {
   RAI_API_BODY({
-    if (!m || !kv || !hiddens || !positions) rai::fail(RAI_E_ARG, "null argument");
+    if (!m || !kv || !in || !out || !positions) rai::fail(RAI_E_ARG, "null argument");
     if (kv->model != m) rai::fail(RAI_E_ARG, "KV cache belongs to another model");
     if (batch == 0) rai::fail(RAI_E_ARG, "batch must contain at least one token");
     for (size_t b = 0; b < batch; ++b) {
@@ -1377,19 +1532,26 @@ int rai_forward_batch(rai_model *m, rai_kv *kv, float *hiddens, const size_t *po
     rai::Workspace &w = rai::model_ws(*m);
     const size_t H = m->cfg.hidden_size;
     const std::vector<size_t> filled0 = kv->filled;
+    int err[2] = {0, 0};
+    const size_t most = H * std::min<size_t>(batch, rai::kChunk);
+    rai::HostStage io(m->stream, most, most);
     for (size_t b0 = 0; b0 < batch; b0 += rai::kChunk) {
       const int mm = (int)std::min<size_t>(rai::kChunk, batch - b0);
-      HIP_CHECK(hipMemcpyAsync(w.hid.p, hiddens + b0 * H, sizeof(float) * H * mm, hipMemcpyHostToDevice, m->stream));
+      io.in(w.hid.as<float>(), in + b0 * H, H * mm);
       rai::forward(*m, *kv, w, mm, positions[b0], m->stream);
-      HIP_CHECK(hipMemcpyAsync(hiddens + b0 * H, w.hid.p, sizeof(float) * H * mm, hipMemcpyDeviceToHost, m->stream));
+      io.out(out + b0 * H, w.hid.as<float>(), H * mm, w.err.as<int>(), err);
     }
     try {
-      rai::check_kernel_error(w, m->stream);
+      rai::raise_kernel_errors(w, m->stream, err);
     } catch (...) {
       kv->filled = filled0;  // the batch's KV rows are not trusted
       throw;
     }
   });
+}
+
+int rai_forward_batch(rai_model *m, rai_kv *kv, float *hiddens, const size_t *positions, size_t batch) {
+  return rai_forward_batch_to(m, kv, hiddens, hiddens, positions, batch);
 }
 
 int rai_forward_from_hidden(rai_model *m, rai_kv *kv, float *hidden, size_t pos, int store_kv) {
@@ -1406,13 +1568,14 @@ int rai_hidden_to_logits_batch(rai_model *m, const float *hiddens, float *out, s
     if (batch == 0) rai::fail(RAI_E_ARG, "batch must contain at least one token");
     rai::Workspace &w = rai::model_ws(*m);
     const size_t H = m->cfg.hidden_size, V = m->cfg.vocab_size;
+    const size_t most = std::min<size_t>(w.logit_rows, batch);
+    rai::HostStage io(m->stream, H * most, V * most);
     for (size_t b0 = 0; b0 < batch; b0 += (size_t)w.logit_rows) {
       const int mm = (int)std::min<size_t>(w.logit_rows, batch - b0);
-      HIP_CHECK(hipMemcpyAsync(w.hid.p, hiddens + b0 * H, sizeof(float) * H * mm, hipMemcpyHostToDevice, m->stream));
+      io.in(w.hid.as<float>(), hiddens + b0 * H, H * mm);
       rai::logits(*m, w, mm, m->stream);
-      HIP_CHECK(hipMemcpyAsync(out + b0 * V, w.logits.p, sizeof(float) * V * mm, hipMemcpyDeviceToHost, m->stream));
+      io.out(out + b0 * V, w.logits.as<float>(), V * mm);
     }
-    HIP_CHECK(hipStreamSynchronize(m->stream));
   });
 }
 

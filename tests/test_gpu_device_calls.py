@@ -194,3 +194,24 @@ def test_small_batch_layers(rai, ora, gs, m):
     assert np.array_equal(_bits(got).reshape(-1), _bits(want).reshape(-1))
     gl, ol = gm.hidden_to_logits_batch(got, m), om.hidden_to_logits_batch(want, m)
     assert np.array_equal(_bits(gl).reshape(-1), _bits(ol).reshape(-1))
+
+
+@pytest.mark.parametrize("m", [1, 3, 700, 1100])
+def test_host_buffers_of_every_size(rai, m):
+    """Hidden states through the pinned staging in one part, several parts and
+    several chunks: the batch equals its halves run one after the other, the
+    caller's array is left alone, and logits of a batch equal those of a row."""
+    H, V = 1024, 30001
+    img = rai.synth_model(H, 1, 8, 2, 128, 1024, V, 1200, group_size=64, seed=m)
+    gm = rai.RaiModel.from_bytes(img)
+    h = np.random.default_rng(m).normal(0.0, 1.0, (m, H)).astype(np.float32)
+    keep = h.copy()
+    got = gm.forward_batch(h, np.arange(m), gm.create_kv_cache(1200))
+    assert np.array_equal(h, keep)
+    kv, cut = gm.create_kv_cache(1200), max(1, m // 2)
+    parts = [gm.forward_batch(h[a:b], np.arange(a, b), kv) for a, b in ((0, cut), (cut, m)) if b > a]
+    assert np.array_equal(_bits(got), _bits(np.concatenate(parts)))
+    n = min(m, 130)
+    lg = gm.hidden_to_logits_batch(got[:n], n)
+    for i in (0, n // 2, n - 1):
+        assert np.array_equal(_bits(lg[i]), _bits(gm.hidden_to_logits(got[i])))
