@@ -24,12 +24,13 @@ ARCH = "gfx950"
 COMMON = ["-O3", "-std=c++17", "-fPIC", "-ffp-contract=off", "-Wall",
           "-I", os.path.join(ROOT, "include"), "-I", CSRC]
 DEVICE = [f"--offload-arch={ARCH}", "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"]
-SOURCES = ["kernels.hip", "fused.hip", "gemv.hip", "gemv_stream.hip", "gemm_mm.hip", "moe.hip", "sample.hip", "decode_gemv.hip", "tied_head.hip", "runtime.hip", "format.cpp", "synth.cpp"]
+SOURCES = ["kernels.hip", "fused.hip", "attn_mm.hip", "gemv.hip", "gemv_stream.hip", "gemm_mm.hip", "moe.hip", "sample.hip", "decode_gemv.hip", "tied_head.hip", "runtime.hip", "format.cpp", "synth.cpp"]
 # Per-source device flags: the matrix-core GEMV keeps MFMA results in
 # architectural VGPRs, which its epilogue reads directly (without it the
 # compiler routes them through AGPRs and one copy per value).
 EXTRA = {"gemv.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"], "gemm_mm.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
-         "gemv_stream.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"]}
+         "gemv_stream.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
+         "attn_mm.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"]}
 
 
 def _compile(src: str) -> str:

@@ -1716,8 +1716,14 @@ void launch_attention(const float *q, int q_ld, const float *kc, const float *vc
                       int vstride, int pos0, int m, int nh, int nkv, int hd, float scale,
                       float *out, float *scores, hipStream_t s, const int *st, int *err, int stages,
                       int span) {
-  for (int t0 = 0; t0 < m; t0 += kAttnTokens) {
-    const int mt = std::min(kAttnTokens, m - t0);
+  // Prefill batches: kAttnTokens per launch, so that the PV chains (one wave per
+  // 16 tokens, head and 64 dimensions) fill the chip; the streamed PV kernel
+  // keeps the 128 it was measured at.
+  const bool mm = !st && attn_mm_path(q, q_ld, kc, vc, vstride, m, nh, nkv, hd);
+  // A lowered poll limit asks for the kernel that waits.
+  const bool pv_mm = mm && g_pv_spin == kPvSpin;
+  for (int t0 = 0, mt; t0 < m; t0 += mt) {
+    mt = pv_mm && m - t0 > kPvMmTokens ? std::min(kAttnTokens, m - t0) : std::min(128, m - t0);
     const int p0 = pos0 + t0;
     // With a step record the position is on the device: the grids, the
     // score stride and the softmax kernel are those of the span of
@@ -1736,7 +1742,11 @@ void launch_attention(const float *q, int q_ld, const float *kc, const float *vc
                          st);
       continue;
     }
-    if (stages & 1) launch_scores(qt, q_ld, kc, cap, p0, mt, nh, nkv, hd, scale, scores, sstride, nmax, st, s);
+    if (!(stages & 1)) {
+    } else if (mm)
+      launch_scores_mm(qt, q_ld, kc, cap, p0, mt, nh, nkv, hd, scale, scores, sstride, s);
+    else
+      launch_scores(qt, q_ld, kc, cap, p0, mt, nh, nkv, hd, scale, scores, sstride, nmax, st, s);
     if (!(stages & 2)) {
     } else if (mt > 12 && nmax <= 4096) {
       // Many rows (prefill): one wave per row; per 4095-token Mistral-7B
@@ -1777,6 +1787,8 @@ void launch_attention(const float *q, int q_ld, const float *kc, const float *vc
     const bool stream = vstride > 0 && vstride % 64 == 0 &&
                         (G == 1 || G == 2 || G == 4 || G == 8 || G == 16) && hd % DL == 0;
     if (!(stages & 4)) {
+    } else if (pv_mm && mt > kPvMmTokens) {
+      launch_pv_mm(scores, vc, vstride, p0, mt, nh, nkv, hd, sstride, ot, s);
     } else if (stream) {
       // Tokens per block: one for one or two tokens (more blocks), three up
       // to twelve (the verify batch), four beyond; tile length and loader

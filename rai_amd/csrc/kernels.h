@@ -218,8 +218,19 @@ void launch_rope_store(float *q, float *k, const float *v, const float *cos_t, c
 // V cache d-major [nkv][hd][vstride] when vstride > 0, else [nkv][cap][hd].
 // `scores` is scratch of attention_scores_floats(m, nh, pos0 + m) floats;
 // tokens are processed in groups of kAttnTokens.
-constexpr int kAttnTokens = 128;
+constexpr int kAttnTokens = 256;
 size_t attention_scores_floats(int m, int nh, int ctx);
+// The scores and PV of attn_mm.hip (prefill batches of kAttnMmTokens and
+// more, PV past kPvMmTokens a launch); the softmax between them is
+// launch_attention's.  At 3072 to 4096 positions PV takes 143 us for up to 256
+// tokens there, 107 per 128 tokens in the streamed kernel.
+constexpr int kAttnMmTokens = 16, kPvMmTokens = 160;
+bool attn_mm_path(const float *q, int q_ld, const float *kc, const float *vc, int vstride, int m, int nh, int nkv,
+                  int hd);
+void launch_scores_mm(const float *q, int q_ld, const float *kc, int cap, int pos0, int m, int nh, int nkv, int hd,
+                      float scale, float *S, int sstride, hipStream_t s);
+void launch_pv_mm(const float *S, const float *vc, int vstride, int pos0, int m, int nh, int nkv, int hd, int sstride,
+                  float *out, hipStream_t s);
 // q rows are q_ld floats apart; out is [m][nh * hd].
 // With a step record `st` (m <= kAttnTokens), grids, the score stride and
 // the softmax kernel are sized for a span of positions, min(cap, span), so

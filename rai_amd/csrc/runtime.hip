@@ -1877,7 +1877,7 @@ int rai_attention_time_dev(const float *q, const float *kc, const float *vc, siz
                            size_t nh, size_t nkv, size_t hd, size_t copies, int iters, float *ms3) {
   RAI_API_BODY({
     if (!q || !kc || !vc || !ms3) rai::fail(RAI_E_ARG, "null argument");
-    if (m == 0 || m > (size_t)rai::kAttnTokens || nkv == 0 || nh % nkv || hd == 0 || hd % 8 || copies == 0 ||
+    if (m == 0 || m > 128 || nkv == 0 || nh % nkv || hd == 0 || hd % 8 || copies == 0 ||
         iters <= 0)
       rai::fail(RAI_E_SHAPE, "invalid attention shape");
     if (pos + m > cap) rai::fail(RAI_E_RANGE, "positions exceed the cache");

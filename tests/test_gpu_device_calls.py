@@ -215,3 +215,21 @@ def test_host_buffers_of_every_size(rai, m):
     lg = gm.hidden_to_logits_batch(got[:n], n)
     for i in (0, n // 2, n - 1):
         assert np.array_equal(_bits(lg[i]), _bits(gm.hidden_to_logits(got[i])))
+
+
+@pytest.mark.parametrize("heads,kv,hd", [(4, 1, 64), (3, 3, 128), (6, 3, 64), (8, 1, 128), (5, 1, 64)])
+@pytest.mark.parametrize("first,m", [(0, 16), (1, 17), (5, 33), (63, 64), (64, 161), (130, 300), (1, 530)])
+def test_prefill_attention(rai, ora, heads, kv, hd, first, m):
+    """Scores and PV on the matrix cores: token tiles of 16 with a remainder,
+    position tiles of 64 that tokens see whole, in part or not at all, launches
+    of 256 tokens, a cache filled before."""
+    H = heads * hd
+    img = rai.synth_model(H, 1, heads, kv, hd, 128, 64, 640, group_size=32, embed_group_size=32, seed=first + m)
+    gm, om = rai.RaiModel.from_bytes(img), ora.Model(img, 0)
+    h = np.random.default_rng(m).normal(0.0, 1.0, (first + m, H)).astype(np.float32)
+    gk, ok = gm.create_kv_cache(640), om.create_kv(640)
+    for a, b in ((0, first), (first, first + m)):
+        if b > a:
+            got = gm.forward_batch(h[a:b], np.arange(a, b), gk)
+            want = om.forward_batch(h[a:b], np.arange(a, b), ok)
+            assert np.array_equal(_bits(got).reshape(-1), _bits(want).reshape(-1)), (a, b)
