@@ -93,6 +93,15 @@ struct DecMoe {
   int8_t *qo = nullptr;
   float *so = nullptr, *uo = nullptr;
 };
+// The fused projections of one f32 row (K as w4a8_dec_fused_ok): up to three
+// matrices of the same columns and group in one launch, which quantizes the
+// row itself; false when one of them is outside the one-token kernel's shapes.
+struct DecMulti {
+  float *out[3];
+  const uint8_t *nib[3], *par[3];
+  int rows[3];
+};
+bool launch_w4a8_dec_multi(const DecMulti &mp, int n, int cols, int gs, const float *nx, hipStream_t s);
 bool launch_w4a8_dec_moe(float *out, const DecMoe &moe, const int8_t *q_split, const float *scales,
                          const float *sums, int rows, int cols, int gs, int max_entries, hipStream_t s);
 // The experts' gate|up (rows = 2 F, gate rows first) with silu_mul_inplace

@@ -1678,15 +1678,21 @@ static void fused_projections(float *const *outs, const rai_qlinear *const *lin,
   }
   hipStream_t s = (hipStream_t)stream;
   const size_t cols = lin[0]->cols, gs = lin[0]->group_size, groups = rai::ceil_div(cols, gs);
-  // Short rows: every GEMV launch quantizes the row itself.
-  bool self = true, fast = true;
-  for (int i = 0; i < n; ++i) fast = fast && rai::w4a8_fast_path((int)cols, (int)gs, lin[i]->nibbles, lin[i]->params);
-  for (int i = 0; i < n && self; ++i)
-    self = fast && rai::w4a8_dec_path((int)lin[i]->rows, (int)cols, (int)gs) && !rai::overlaps(outs[i], lin[i]->rows, x, cols);
-  if (self && rai::w4a8_dec_fused_ok((int)cols)) {
-    for (int i = 0; i < n; ++i)
-      rai::launch_w4a8_dec(outs[i], nullptr, lin[i]->nibbles, lin[i]->params, nullptr, nullptr, nullptr,
-                           (int)lin[i]->rows, (int)cols, (int)gs, x, nullptr, 0.0f, s);
+  // Short rows: one launch for all projections, which quantizes the row itself.
+  bool fast = true, self = true;
+  rai::DecMulti mp{};
+  for (int i = 0; i < n; ++i) {
+    fast = fast && rai::w4a8_fast_path((int)cols, (int)gs, lin[i]->nibbles, lin[i]->params);
+    self = self && !rai::overlaps(outs[i], lin[i]->rows, x, cols);
+    mp.out[i] = outs[i];
+    mp.nib[i] = lin[i]->nibbles;
+    mp.par[i] = lin[i]->params;
+    mp.rows[i] = (int)lin[i]->rows;
+  }
+  // Outputs that share memory are written in turn below, the last one last.
+  for (int i = 0; i < n; ++i)
+    for (int j = 0; j < i; ++j) self = self && !rai::overlaps(outs[i], lin[i]->rows, outs[j], lin[j]->rows);
+  if (fast && self && rai::launch_w4a8_dec_multi(mp, n, (int)cols, (int)gs, x, s)) {
     HIP_CHECK(hipGetLastError());
     HIP_CHECK(hipStreamSynchronize(s));
     return;

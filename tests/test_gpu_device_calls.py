@@ -233,3 +233,18 @@ def test_prefill_attention(rai, ora, heads, kv, hd, first, m):
             got = gm.forward_batch(h[a:b], np.arange(a, b), gk)
             want = om.forward_batch(h[a:b], np.arange(a, b), ok)
             assert np.array_equal(_bits(got).reshape(-1), _bits(want).reshape(-1)), (a, b)
+
+
+@pytest.mark.parametrize("gs", [32, 64, 128])
+@pytest.mark.parametrize("rows,cols", [((1, 3, 17), 256), ((16401, 40, 40), 256), ((100, 530), 1152), ((70, 70), 4096),
+                                       ((33, 34, 35), 4224)])
+def test_fused_projections_of_unequal_rows(rai, ora, gs, rows, cols):
+    """One launch for matrices of different heights (and K past it)."""
+    lin = []
+    for i, r in enumerate(rows):
+        nib, params, x = gemv_operands(r, cols, 1, gs, seed=r + i)
+        lin.append((nib, params, r, cols, gs))
+    x = np.ascontiguousarray(x, np.float32).reshape(-1)
+    got = rai.w4a8_fused_qkv(*lin, x) if len(rows) == 3 else rai.w4a8_fused_gate_up(*lin, x)
+    for g, p in zip(got, lin):
+        assert np.array_equal(_bits(g), _bits(ora.w4a8_matvec(p[0], p[1], x, p[2], p[3], p[4])))
