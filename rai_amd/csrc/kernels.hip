@@ -1265,6 +1265,64 @@ __global__ __launch_bounds__(64) void k_router_logits_r(const float *__restrict_
   if ((lane & 15) == 15 && (int)blockIdx.y * 4 + c < experts) logits[(size_t)t * experts + blockIdx.y * 4 + c] = acc;
 }
 
+// Router logits of many tokens: a tile of 16 tokens x 16 experts per block, the
+// products of 16 columns as four outer products on the matrix cores
+// (v_mfma_f32_16x16x1_4b_f32: one product and +0, one rounding; block b of
+// instruction u is column 4 b + u of the sixteen), then every lane adds its
+// chains' products in column order.  The two waves of a block multiply the same
+// tile and add half of its tokens each (wave w's at registers 0 and 1, by
+// loading token i ^ 2w at row i): the dependent adds, not the products, take the
+// time.  A -0 product enters as +0, which can only change the sign of a zero
+// logit.  Requires hidden % 16 == 0.
+__global__ __launch_bounds__(128) void k_router_logits_mm(const float *__restrict__ x,
+                                                          const float *__restrict__ router, int m, int hidden,
+                                                          int experts, float *__restrict__ logits) {
+  typedef float f16v __attribute__((ext_vector_type(16)));
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, col = lane & 15, h = lane >> 4;
+  const int t0 = blockIdx.x * 16, e = blockIdx.y * 16 + col;
+  const float4 *xp =
+      reinterpret_cast<const float4 *>(x + (size_t)min(t0 + (col ^ (2 * w)), m - 1) * hidden + 4 * h);
+  const float4 *rp = reinterpret_cast<const float4 *>(router + (size_t)min(e, experts - 1) * hidden + 4 * h);
+  const int nq = hidden / 16;
+  constexpr int D = 4;  // sixteens in flight
+  float4 xv[D], rv[D];
+#pragma unroll
+  for (int d = 0; d < D; ++d) {
+    xv[d] = xp[4 * min(d, nq - 1)];
+    rv[d] = rp[4 * min(d, nq - 1)];
+  }
+  float a0 = -0.0f, a1 = -0.0f;
+  const f16v zero = {};
+  for (int q0 = 0; q0 < nq; q0 += D) {
+#pragma unroll
+    for (int d = 0; d < D; ++d) {
+      if (q0 + d < nq) {
+        f16v p[4];
+        p[0] = __builtin_amdgcn_mfma_f32_16x16x1f32(xv[d].x, rv[d].x, zero, 0, 0, 0);
+        p[1] = __builtin_amdgcn_mfma_f32_16x16x1f32(xv[d].y, rv[d].y, zero, 0, 0, 0);
+        p[2] = __builtin_amdgcn_mfma_f32_16x16x1f32(xv[d].z, rv[d].z, zero, 0, 0, 0);
+        p[3] = __builtin_amdgcn_mfma_f32_16x16x1f32(xv[d].w, rv[d].w, zero, 0, 0, 0);
+#pragma unroll
+        for (int b = 0; b < 4; ++b)
+#pragma unroll
+          for (int u = 0; u < 4; ++u) {
+            a0 = a0 + p[u][4 * b];
+            a1 = a1 + p[u][4 * b + 1];
+          }
+      }
+      const int qn = min(q0 + d + D, nq - 1);
+      xv[d] = xp[4 * qn];
+      rv[d] = rp[4 * qn];
+    }
+  }
+  // Row 4 h + r of the tile is token (4 h + r) ^ 2w.
+  const int t = t0 + 4 * h + 2 * w;
+  if (e < experts) {
+    if (t < m) logits[(size_t)t * experts + e] = a0;
+    if (t + 1 < m) logits[(size_t)(t + 1) * experts + e] = a1;
+  }
+}
+
 // route_experts for at most 64 experts, one wave per token, expert e on
 // lane e: the maximum by DPP moves, glibc expf, the sum as one chain in
 // expert order (lane reads), the division; then each top-k pick is the
@@ -1590,7 +1648,13 @@ void launch_accept(const uint32_t *am, uint32_t *ctx, int len, int start, int nd
 void launch_router(const float *x, const float *router, int m, int hidden, int experts, int topk,
                    int norm_topk, int *sel, float *wts, float *logits, hipStream_t s) {
   const dim3 g4(m, (experts + 3) / 4);
-  if (hidden == 16 * 128)
+  // The tile kernel's chains take as long for one tile as for a hundred (32.6
+  // us at hidden 2048), the wave-per-token kernel's time grows with tokens x
+  // experts: 64 experts, 192 tokens 28.8 us, 256 tokens 39.5, 512 tokens 68.
+  if ((int64_t)m * experts >= 256 * 64 && hidden % 16 == 0 && (((uintptr_t)x | (uintptr_t)router) & 15) == 0)
+    hipLaunchKernelGGL(k_router_logits_mm, dim3((m + 15) / 16, (experts + 15) / 16), dim3(128), 0, s, x, router, m,
+                       hidden, experts, logits);
+  else if (hidden == 16 * 128)
     hipLaunchKernelGGL(k_router_logits_r<128>, g4, dim3(64), 0, s, x, router, experts, logits);
   else if (hidden == 16 * 64)
     hipLaunchKernelGGL(k_router_logits_r<64>, g4, dim3(64), 0, s, x, router, experts, logits);

@@ -104,6 +104,20 @@ def test_sparse_layer_prefill(rai, ora, gs, experts, topk, m):
     assert np.array_equal(_bits(got).reshape(-1), _bits(want).reshape(-1))
 
 
+@pytest.mark.parametrize("experts,topk,m", [(64, 8, 257), (70, 4, 239), (17, 16, 964)])
+@pytest.mark.parametrize("hidden", [128, 288])
+def test_router_tiles(rai, ora, hidden, experts, topk, m):
+    """Router logits in tiles of 16 tokens x 16 experts: whole and ragged tiles
+    of both, column chunks that fill the loads in flight and that do not."""
+    img = rai.synth_model(hidden, 1, 2, 2, 64, 64, 300, 1024, group_size=32, num_experts=experts,
+                          experts_per_token=topk, seed=experts + m)
+    gm, om = rai.RaiModel.from_bytes(img), ora.Model(img, 256)
+    h = np.random.default_rng(m).normal(0.0, 1.0, (m, hidden)).astype(np.float32)
+    got = gm.forward_batch(h, np.arange(m), gm.create_kv_cache(1024))
+    want = om.forward_batch(h, np.arange(m), om.create_kv(1024))
+    assert np.array_equal(_bits(got).reshape(-1), _bits(want).reshape(-1))
+
+
 def _table(vocab, hidden, gs, seed):
     r = np.random.default_rng(seed)
     codes = r.integers(0, 256, vocab * hidden, dtype=np.uint8)
