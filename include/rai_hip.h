@@ -134,7 +134,7 @@ int rai_device_info(char *name, size_t name_len, int *compute_units);
  * 128, or a larger bound for group-32 models with K > 4096.  Device memory:
  * the file's bytes, RoPE tables, and for group-32 dense matrices a second
  * copy of their scale/zero parameters in 16-row tiles (about a fifth of the
- * quantized weight bytes), which the 2..64-token GEMVs read. */
+ * quantized weight bytes), which the 2..24-token GEMVs read. */
 int rai_model_open(const char *path, int max_groups, rai_model **out);
 /* Same, from a caller-owned in-memory .raimodel image (copied). */
 int rai_model_from_buffer(const void *data, size_t len, int max_groups, rai_model **out);
@@ -218,7 +218,7 @@ int rai_w4a8_fused_gate_up_dev(float *gate_out, float *up_out, const rai_qlinear
  * reference: it is for callers that cannot allocate device memory (code under
  * HIP graph capture, tight serving loops, harnesses that forbid hipMalloc).
  * Same arguments, arithmetic and results; the quantized activations live in
- * a fixed per-GPU scratch array held until the process ends (8 MiB),
+ * a fixed per-GPU scratch array held until the process ends (14.5 MiB),
  * so the call is asynchronous on `stream` and calls no allocator.  Limits:
  * m * cols <= 1048576 and m * ceil(cols / group_size) <= 65536, else
  * RAI_E_SHAPE.  Every call on one GPU shares that GPU's scratch: calls that
