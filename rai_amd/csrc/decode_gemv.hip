@@ -285,9 +285,9 @@ __global__ __launch_bounds__(256) void k_w4a8_dec(float *out, const float *add, 
     uint32_t vp = ((uint32_t)row * groups + un / LPG) * 4;
     // Past the last iteration, and on the lanes past the units of a
     // partial last chunk: zeros without a memory access.  Zero codes and
-    // parameters give +0 or -0 products, which leave a chain unchanged (a
-    // chain starts at +0 and a sum of floats is -0 only when both terms
-    // are).
+    // parameters, with the zero scale and sum of read_act, give +0 or -0
+    // products, which leave a chain unchanged (a chain starts at +0 and a sum
+    // of floats is -0 only when both terms are).
     if (lt >= tiles_per_wave || un >= units) {
       vc = 0x80000000u;  // past num_records
       vp = 0x80000000u;
@@ -340,15 +340,17 @@ __global__ __launch_bounds__(256) void k_w4a8_dec(float *out, const float *add, 
   const int cbase = min(lane, NC * R - 1) * STR;
   // Group of the lane's unit in the chunk, and the unit's place in it.
   const int kg = k / LPG, ku = k % LPG;
-  // Activations of the iteration's chunk (read one iteration ahead).
+  // Activations of the iteration's chunk (read one iteration ahead).  Units
+  // past the row's: the last one's codes, with a zero scale and sum, so that
+  // their zero parameters meet no infinite or NaN factor.
   uint4 q0, q1;
   float as, xsum;
   auto read_act = [&](int ch) {
-    const int un = min(ch * kDecChunk + k, units - 1);
+    const int uq = ch * kDecChunk + k, un = min(uq, units - 1);
     q0 = *reinterpret_cast<const uint4 *>(qsh + un * 32);
     q1 = *reinterpret_cast<const uint4 *>(qsh + un * 32 + 16);
-    as = ash[un / LPG];
-    xsum = ssh[un / LPG];
+    as = uq < units ? ash[un / LPG] : 0.0f;
+    xsum = uq < units ? ssh[un / LPG] : 0.0f;
   };
   // End of tile t: the row sums from the chain values in acc.
   auto finish = [&](int t) {

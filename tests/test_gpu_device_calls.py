@@ -164,6 +164,33 @@ def test_one_token_every_group_size(rai, ora, gs, cols, rows):
             assert np.array_equal(_bits(got), _bits(want).reshape(-1)), (name, scale)
 
 
+# Every one-token kernel, K ending inside a chunk of 1024 columns (for group 32,
+# also one group past it) and on its edge.
+@pytest.mark.parametrize("gs,cols", [(32, 1056), (32, 1184), (32, 2048), (32, 4128), (64, 320), (64, 1088), (64, 4160),
+                                     (128, 384), (128, 1152), (128, 4224)])
+@pytest.mark.parametrize("last", ["sum", "element"])
+def test_one_token_infinite_last_group(rai, ora, gs, cols, last):
+    """The last group's input sum overflows (finite values), or one of its
+    elements is infinite: nothing but that group's own terms sees it."""
+    rows = 37
+    nib, params, x = gemv_operands(rows, cols, 1, gs, seed=cols + gs)
+    x = np.ascontiguousarray(x, np.float32).reshape(-1)
+    if last == "sum":
+        x[-gs:] = 2e37
+    else:
+        x[-gs // 2] = np.inf
+    want = ora.w4a8_matmul(nib, params, x, rows, cols, 1, gs).reshape(-1)
+    if last == "sum":
+        assert np.isneginf(want).all()  # every zero point is negative
+    dev = rai.DeviceArray.from_host
+    for name in ("rai_w4a8_matmul_dev", "rai_w4a8_matmul_noalloc_dev"):
+        got = _call(rai, name, rai.DeviceArray(4 * rows), dev(nib), dev(params), dev(x), rows, cols, 1, gs)
+        assert np.array_equal(got, want, equal_nan=True), name
+    lin = (nib, params, rows, cols, gs)
+    for got in rai.w4a8_fused_gate_up(lin, lin, x):
+        assert np.array_equal(got, want, equal_nan=True)
+
+
 @pytest.mark.parametrize("gs", [32, 64, 128])
 @pytest.mark.parametrize("hidden,heads,kv,hd,ffn,experts", [(256, 4, 2, 64, 384, 0), (1152, 9, 3, 128, 1280, 0),
                                                             (512, 8, 8, 64, 256, 8)])
