@@ -28,7 +28,8 @@
 // the row so that the 16 rows' reads fall on different banks).  One barrier a
 // stage.  Lanes of tokens past the tile's last read that last token's data,
 // and lanes of groups past the row's last read that group's codes with zero
-// parameters and scales, so nothing outside the inputs enters.
+// parameters and scales, so nothing outside the inputs enters; no load leaves
+// the arrays (stream_addr.h).
 //
 // CW: the eight (four at group 32) lane chains of a row are independent until
 // the final sum, so CW waves may share a row tile, NL / CW chains each, where
@@ -46,6 +47,7 @@
 #include <type_traits>
 
 #include "kernels.h"
+#include "stream_addr.h"
 
 namespace rai {
 
@@ -124,14 +126,15 @@ __global__ __launch_bounds__(256, 2) void k_gemv_stream(float *out, const float 
 #pragma unroll
   for (int c = 0; c < NC; ++c) {
     const int r = (64 * c + lane) / U, u = ((64 * c + lane) % U) ^ swz(r);
-    const int base = min(row0 + r, rows - 1) * (cols / 2) + (u % NC) * 16;
-    vc[c] = base + (u / NC) * (GS / 2);
-    vcl[c] = base + min(u / NC, groups - 1 - 4 * (nq - 1)) * (GS / 2);
+    const int rr = min(row0 + r, rows - 1);
+    vc[c] = stream_code_off(rr, cols, GS, 0, u / NC, u % NC).v;
+    vcl[c] = stream_code_off(rr, cols, GS, nq - 1, u / NC, u % NC).v;
   }
   // Parameters of stage S: lane i moves 16 bytes (one step) of row
-  // i / 4.  Past the row's groups they are some other row's, never used.
+  // i / 4.  Past the row's groups they are the next row's, or past the array
+  // (zeros, which the range check of the VGPR offset answers); never used.
   const int pr = lane >> 2, ps = (lane & 3) ^ ((pr >> 2) & 3);
-  const int vp = (min(row0 + pr, rows - 1) * groups + 4 * ps) * 4;
+  const int prow = min(row0 + pr, rows - 1);
   const int jt = min(j, mt - 1);
   const int va = (h * 16 + jt) * 16, vs = (h * 16 + jt) * 4;
   // Groups past the row's have no activations: the last step's lanes read
@@ -154,7 +157,8 @@ __global__ __launch_bounds__(256, 2) void k_gemv_stream(float *out, const float 
       for (int c = 0; c < NC; ++c)
         rc[d][i * NC + c] = __builtin_amdgcn_raw_buffer_load_b128(rcs, last ? vcl[c] : vc[c], qc * (2 * GS), 0);
     }
-    rp[d] = __builtin_amdgcn_raw_buffer_load_b128(rps, vp, min(S, nst - 1) * 64, 0);
+    const BufOff po = stream_param_off(prow, groups, S, ps);
+    rp[d] = __builtin_amdgcn_raw_buffer_load_b128(rps, po.v, po.s, 0);
   };
   // Step q's scales and activations.
   auto load_a = [&](int s, int q) __attribute__((always_inline)) {

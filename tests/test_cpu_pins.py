@@ -220,6 +220,19 @@ def test_expf_restatement_matches_host_libm(tmp_path):
     assert int(bad) == 0, f"first mismatch at {first}"
 
 
+def test_streamed_weight_loads_stay_inside_their_arrays(tmp_path):
+    """Every code and parameter load of the streamed W4A8 kernel, any rows and
+    group count (multiples of a stage's 16 groups and not): no dword outside the
+    caller's arrays, and every real group's dwords at their place."""
+    exe = tmp_path / "stream_addr_check"
+    subprocess.run(["g++", "-O2", "-std=c++17", "-I", os.path.join(ROOT, "rai_amd", "csrc"),
+                    os.path.join(ROOT, "tests", "stream_addr_check.cpp"), "-o", str(exe)], check=True)
+    out = subprocess.run([str(exe)], check=True, capture_output=True, text=True).stdout
+    loads, outside, wrong = (int(v) for v in out.split())
+    assert loads > 1_000_000
+    assert (outside, wrong) == (0, 0)
+
+
 # The PCG32 reference implementation's demo (pcg32_srandom_r(42, 54), then
 # pcg32_random_r): its published first outputs.
 _PCG_DEMO_42_54 = [0xA15C02B7, 0x7B47F409, 0xBA1D3330, 0x83D2F293, 0xBFA4784B, 0xCBED606E]
