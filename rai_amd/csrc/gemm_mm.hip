@@ -394,22 +394,39 @@ static bool mm_ok(int rows, int cols, int gs) {
          (int64_t)rows * (cols / 2) < ((int64_t)1 << 31);
 }
 
-// Where the lines lie (device time, weights from HBM, K = 4096; the times of
-// all three grow alike with K):
-// - Up to 24 tokens the register-pipelined kernel, whose tiles are four
-//   tokens, where it applies: 28672 rows, 9 tokens 26.1 us (streamed 39.7), 24
-//   tokens 56.2 (68.4); 4096 rows, 32 tokens 19.2 (17.5).
+// Two to four tokens on the tiled VALU kernel, whose time grows with the tokens
+// where the streamed kernel's (16 token slots) does not (device time, weights
+// from HBM, us, VALU / streamed):
+// - Two tokens: 28672x4096 group 64 26.2 / 36.1, group 128 26.1 / 29.7;
+//   11008x4128 group 32 14.9 / 21.4; 256x2048 group 64 5.7 / 6.7.  One to four
+//   groups of 64 or 128 in few rows: 4096x256 group 128 5.1 / 4.7.
+// - Three, where the streamed kernel's blocks leave much of their last round
+//   empty (5000 to 12288 rows: 384 or 344 blocks on 256 CUs) or K is short:
+//   11008x4096 group 64 16.0 / 19.4, group 128 13.5 / 15.9; 6144x2048 group 64
+//   8.1 / 9.2, 6144x14336 38.0 / 34.2; 28672x2048 group 64 19.1 / 22.3, group 128
+//   18.3 / 19.0; 4096x2048 group 64 7.2 / 7.4; 14336x4096 23.6 / 20.5.
+// - Four: 11008x2048 group 64 11.1 / 12.2, 11008x4096 27.1 / 19.5.
+static bool small_path(int rows, int cols, int m, int gs) {
+  if (m == 2) return gs == 32 || cols >= 1024 || rows > 5000;
+  if (m == 3) return rows > 5000 && (rows <= 12288 ? cols <= 4096 || rows > 8192 : gs < 128 && cols < 4096);
+  return m == 4 && rows > 8192 && rows <= 12288 && cols <= 2048;
+}
+
+// Where the lines lie (device time, weights from HBM):
+// - The register-pipelined kernel, whose tiles are four tokens, where
+//   gemv_rp_path says so; the VALU kernel for small_path's few tokens.
 // - The streamed kernel has 16 x 16 tiles and splits a tile's chains over
 //   waves, so it wins until the GEMM's 32 x 32 tiles alone fill the chip, at
-//   about 4500 tiles of its own: group 32, 28672 rows, 32 tokens (3584 tiles)
-//   68.2 against 70.0, 64 tokens (7168) 120.5 against 97.5; 4096 rows, 96
+//   about 4500 tiles of its own: group 32, K = 4096, 28672 rows, 32 tokens (3584
+//   tiles) 68.2 against 70.0, 64 tokens (7168) 120.5 against 97.5; 4096 rows, 96
 //   tokens (1536) 36 against 66.  Group 128, where the GEMM's two blocks per
 //   instruction count: 14336 rows, 33 tokens (2688) 38.4 against 41.1, 64
 //   (3584) 46.7 against 41.7.
 // - Up to 16 tokens half of the GEMM's tile would be padding at any size.
-W4Route w4a8_route(int rows, int cols, int m, int gs) {
+W4Route w4a8_route(int rows, int cols, int m, int gs, bool tiled) {
   if (!mm_ok(rows, cols, gs)) return W4Route::kValu;
-  if (m <= 24 && gemv_rp_path(rows, cols, m, gs)) return W4Route::kRp;
+  if (gemv_rp_path(rows, cols, m, gs, tiled)) return W4Route::kRp;
+  if (small_path(rows, cols, m, gs)) return W4Route::kSmall;
   const int64_t tiles = (int64_t)((rows + 15) / 16) * ((m + 15) / 16);
   if ((m <= 16 || tiles <= (gs == 128 ? 3000 : 4500)) && qa_bytes(m, cols, gs) < ((size_t)1 << 31))
     return W4Route::kStream;

@@ -453,36 +453,50 @@ void launch_rp(float *out, const float *add, const uint8_t *nib, const uint8_t *
                      q_split, scales, sums, rows, cols, m, ntg);
 }
 
+// Token groups (of four) per block.  K <= 4096: three for 3, 5 or 6 and more
+// groups (the duplicates past an odd count cost less than a third pass over
+// the weights) from 16384 rows or where that still gives at least 192 blocks of
+// 64 rows, else two where they do; one up to 8192 rows and five token groups
+// with the tiled parameters (qkv 6144x4096 at 9 tokens 14.3 -> 13.5 us, at 17
+// tokens 19.3 -> 14.3; o_proj 4096x4096 at 17 tokens 14.3 -> 13.5).  Longer K:
+// one (the block's activations must fit in LDS).
+int rp_groups(int rows, int cols, int ntg, bool tiled) {
+  const int rb = (rows + 63) / 64;
+  const bool three = ntg >= 3 && ntg != 4;
+  if (cols > kRpMaxCols || (tiled && rows <= 8192 && ntg <= 5)) return 1;
+  if (three && (rows >= 16384 || rb * ((ntg + 2) / 3) >= 192)) return 3;
+  return ntg >= 2 && rb * ((ntg + 1) / 2) >= 192 ? 2 : 1;
+}
+
 template <bool TMP>
 void launch_rp_shape(float *out, const float *add, const uint8_t *nib, const uint8_t *params, const int8_t *q_split,
                      const float *scales, const float *sums, int rows, int cols, int m, int ntg, hipStream_t s) {
   constexpr int Q = kRpMaxCols / 128, Q1 = kRpMaxColsOne / 128;
-  const int rb = (rows + 63) / 64;
-  auto blocks = [&](int tgw) { return rb * ((ntg + tgw - 1) / tgw); };
-  // Three token groups per wave for 3, 5 or 6 and more groups (the
-  // duplicates past an odd count cost less than a third pass over the
-  // weights), two for four.  Up to 8192 rows and five token groups, one
-  // token group per block with the tiled parameters (qkv 6144x4096 at 9
-  // tokens 14.3 -> 13.5 us, at 17 tokens 19.3 -> 14.3; o_proj 4096x4096 at
-  // 17 tokens 14.3 -> 13.5).
-  const bool three = ntg >= 3 && ntg != 4;
-  // Past K = 4096 (one token group per block, 3.5 x the steps) a ring of
-  // eight steps where K / 128 allows (down 4096x14336 at 9 tokens 26.9 ->
-  // 26.2 us; shorter K is slower with it).
-  if (cols > kRpMaxCols && (cols / 128) % 8 == 0)
-    launch_rp<1, 4, Q1, TMP, 8>(out, add, nib, params, q_split, scales, sums, rows, cols, m, ntg, s);
-  else if (cols > kRpMaxCols)
-    launch_rp<1, 4, Q1, TMP>(out, add, nib, params, q_split, scales, sums, rows, cols, m, ntg, s);
-  else if (TMP && rows <= 8192 && ntg <= 5)
-    launch_rp<1, 4, Q, TMP>(out, add, nib, params, q_split, scales, sums, rows, cols, m, ntg, s);
-  else if (three && rows >= 16384)
-    launch_rp<3, 8, Q, TMP>(out, add, nib, params, q_split, scales, sums, rows, cols, m, ntg, s);
-  else if (three && blocks(3) >= 192)
-    launch_rp<3, 4, Q, TMP>(out, add, nib, params, q_split, scales, sums, rows, cols, m, ntg, s);
-  else if (ntg >= 2 && blocks(2) >= 192)
-    launch_rp<2, 4, Q, TMP>(out, add, nib, params, q_split, scales, sums, rows, cols, m, ntg, s);
+  const int g = rp_groups(rows, cols, ntg, TMP);
+  // Steps in flight: four, two where K / 128 is no multiple of four, and past K
+  // = 4096 (3.5 x the steps) eight where it allows (down 4096x14336 at 9 tokens
+  // 26.9 -> 26.2 us; shorter K is slower with eight).
+  auto go = [&](auto nq) {
+    constexpr int NQ = decltype(nq)::value;
+    if (cols > kRpMaxCols)
+      launch_rp<1, 4, Q1, TMP, NQ>(out, add, nib, params, q_split, scales, sums, rows, cols, m, ntg, s);
+    else if constexpr (NQ <= kRpRing) {
+      if (g == 3 && rows >= 16384)
+        launch_rp<3, 8, Q, TMP, NQ>(out, add, nib, params, q_split, scales, sums, rows, cols, m, ntg, s);
+      else if (g == 3)
+        launch_rp<3, 4, Q, TMP, NQ>(out, add, nib, params, q_split, scales, sums, rows, cols, m, ntg, s);
+      else if (g == 2)
+        launch_rp<2, 4, Q, TMP, NQ>(out, add, nib, params, q_split, scales, sums, rows, cols, m, ntg, s);
+      else
+        launch_rp<1, 4, Q, TMP, NQ>(out, add, nib, params, q_split, scales, sums, rows, cols, m, ntg, s);
+    }
+  };
+  if (cols > kRpMaxCols && cols / 128 % 8 == 0)
+    go(std::integral_constant<int, 8>{});
+  else if (cols / 128 % kRpRing == 0)
+    go(std::integral_constant<int, kRpRing>{});
   else
-    launch_rp<1, 4, Q, TMP>(out, add, nib, params, q_split, scales, sums, rows, cols, m, ntg, s);
+    go(std::integral_constant<int, 2>{});
 }
 
 // One thread per 16 bytes (four groups' parameters of one row).
@@ -506,21 +520,42 @@ void launch_params_tile16(const uint8_t *params, int rows, int cols, uint8_t *ti
                      reinterpret_cast<const u32x4 *>(params), rows, nq, reinterpret_cast<u32x4 *>(tiled));
 }
 
-// Group 32, K a multiple of 512 up to 14336, a matrix under 2 GiB.
-bool gemv_rp_path(int rows, int cols, int m, int gs) {
-  return gs == 32 && cols > 0 && cols % (128 * kRpRing) == 0 && cols <= kRpMaxColsOne && m >= 2 && rows > 0 &&
-         (int64_t)rows * (cols / 2) < ((int64_t)1 << 31);
+// Group 32, K a multiple of 256 up to 14336, a matrix under 2 GiB, 2..64 tokens,
+// where it is faster than the streamed kernel (device time, weights from HBM,
+// us, this kernel / streamed; `tiled`: the parameters in 16-row tiles):
+// - Whole rings of four (K a multiple of 512): up to 24 tokens 28672x4096 at 9
+//   26.1 / 39.7, at 24 56.2 / 68.4.
+// - More tokens: while its blocks run in one round, up to two token groups
+//   each: 1024x2048 at 64 tokens 6.9 / 8.5, 1024x14336 27.8 / 38.5, 2048x4096 at
+//   32 10.2 / 13.4, 2560x4096 at 48 (two groups, 240 blocks) 15.0 / 16.7; with
+//   three groups 3072x4096 at 48 19.6 / 19.2, 4096x4096 at 25 19.7 / 16.9.  One
+//   round is 256 blocks, and with the tiled parameters, whose loads leave a
+//   second block of a CU something to do, 384, past K = 4096 512 while two
+//   blocks' activations fit the LDS: 2048x4096 at 40 (320 blocks) 13.8 / 15.9
+//   tiled, 18.9 / 16.0 not; 3072x5632 at 40 (480) 20.5 / 24.4; 4096x14336 at 25
+//   (448) 53.1 / 48.6.
+// - Rings of two: many rows and few tokens, 11008x2816 at 4 tokens 11.4 / 16.0,
+//   at 8 13.3 / 15.9, at 12 17.4 / 16.8; 28672x2816 at 9 21.1 / 28.4, at 16 34.4 /
+//   28.8; 4096x2816 at 8 10.7 / 10.7, 4096x5376 19.2 / 16.9; 11008x5376 at 4 20.2 /
+//   25.1, 28672x5376 at 5 50.5 / 44.7.  Short K in one round of one
+//   token group each: 1024x1280 at 48 6.4 / 6.7, 4096x768 at 24 (two groups) 6.8 /
+//   6.5.
+bool gemv_rp_path(int rows, int cols, int m, int gs, bool tiled) {
+  if (gs != 32 || cols <= 0 || cols % 256 != 0 || cols > kRpMaxColsOne || m < 2 || m > 64 || rows <= 0 ||
+      (int64_t)rows * (cols / 2) >= ((int64_t)1 << 31))
+    return false;
+  const int ntg = (m + 3) / 4, g = rp_groups(rows, cols, ntg, tiled);
+  const int64_t blocks = (int64_t)((rows + 63) / 64) * ((ntg + g - 1) / g);
+  if (cols % (128 * kRpRing) != 0) {
+    if (cols <= 1280 && g == 1 && blocks <= 256) return true;
+    return rows > 5000 && ntg <= (cols > kRpMaxCols ? 1 : rows >= 16384 ? 3 : 2);
+  }
+  if (m <= 24) return true;
+  if (cols <= kRpMaxCols) return g < 3 && blocks <= (tiled ? 384 : 256);
+  return blocks <= (tiled && cols <= 8192 ? 512 : 256);
 }
 
-// Kernel shape per matrix shape, measured on 4096..32000 x 2048..14336 and
-// M = 2..64 with the weights streamed from HBM: for K <= 4096 three token
-// groups per wave, or two, when that
-// still gives at least 192 blocks of four waves (64 rows), else one (a
-// count of token groups that the wave's groups do not divide runs the
-// last block with clamped duplicate groups whose outputs are not stored);
-// eight waves per block for three groups from 16384 rows.  For longer K (at
-// most 14336) one token group per block.  With the
-// parameters also in the 16-row tile layout, that copy is read instead
+// With the parameters also in the 16-row tile layout, that copy is read instead
 // (o_proj 4096x4096 at 9 tokens 10.9 -> 9.3 us, down 4096x14336 31.8 ->
 // 26.6, gate|up 28672x4096 27.5 -> 26.6).
 void launch_gemv_rp(float *out, const float *add, const uint8_t *nib, const uint8_t *params, const int8_t *q_split,

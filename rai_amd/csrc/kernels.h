@@ -112,18 +112,19 @@ bool launch_w4a8_dec_moe_glu(const DecMoe &moe, const int8_t *q_split, const flo
                              int rows, int cols, int gs, int max_entries, hipStream_t s);
 
 // Kernel of a W4A8 product of m >= 2 tokens over whole groups of 32, 64 or 128
-// (w4a8_route).  kRp: the register-pipelined kernel of gemv.hip, which builds
-// its operands from the block-split int8 activations; kStream: the streamed
-// kernel of gemv_stream.hip, with the activations in its lane order (`qa`,
-// qa_bytes of them, written by the quantizing kernels below; rows of tokens
-// past m are not read); kMm: the GEMM of gemm_mm.hip, which packs the
-// block-split activations into `mm` scratch; kValu: the VALU kernels (2 GiB
-// matrices).
-enum class W4Route { kRp, kStream, kMm, kValu };
-W4Route w4a8_route(int rows, int cols, int m, int gs);
+// (w4a8_route; `tiled`: the parameters are there in 16-row tiles as well).
+// kRp: the register-pipelined kernel of gemv.hip, which builds its operands from
+// the block-split int8 activations; kSmall: the tiled VALU kernel of two to four
+// tokens; kStream: the streamed kernel of gemv_stream.hip, with the activations
+// in its lane order (`qa`, qa_bytes of them, written by the quantizing kernels
+// below; rows of tokens past m are not read); kMm: the GEMM of gemm_mm.hip, which
+// packs the block-split activations into `mm` scratch; kValu: the VALU kernels
+// (2 GiB matrices).
+enum class W4Route { kRp, kSmall, kStream, kMm, kValu };
+W4Route w4a8_route(int rows, int cols, int m, int gs, bool tiled);
+bool gemv_rp_path(int rows, int cols, int m, int gs, bool tiled);
 // `params_tiled` (may be null): the same parameters in the layout of
 // launch_params_tile16, read instead of `params` where it applies.
-bool gemv_rp_path(int rows, int cols, int m, int gs);
 void launch_gemv_rp(float *out, const float *add, const uint8_t *nib, const uint8_t *params, const int8_t *q_split,
                     const float *scales, const float *sums, int rows, int cols, int m, hipStream_t s,
                     const uint8_t *params_tiled);

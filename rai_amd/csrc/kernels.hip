@@ -1510,7 +1510,24 @@ void launch_w4a8(float *out, const float *add, const uint8_t *nib, const uint8_t
     return;
   }
   if (m > 1) {
-    const W4Route route = w4a8_route(rows, cols, m, gs);
+    const W4Route route =
+        w4a8_route(rows, cols, m, gs, params_tiled && params_tile16_ok(rows, cols, gs));
+    if (route == W4Route::kSmall) {
+      auto go = [&](auto g) {
+        constexpr int GS = decltype(g)::value;
+        if (m == 2)
+          launch_small_mt<GS, 2>(out, add, nib, params, q_split, scales, sums, rows, cols, m, groups, s);
+        else
+          launch_small_mt<GS, 4>(out, add, nib, params, q_split, scales, sums, rows, cols, m, groups, s);
+      };
+      if (gs == 32)
+        go(std::integral_constant<int, 32>{});
+      else if (gs == 64)
+        go(std::integral_constant<int, 64>{});
+      else
+        go(std::integral_constant<int, 128>{});
+      return;
+    }
     if (route == W4Route::kRp) {
       launch_gemv_rp(out, add, nib, params, q_split, scales, sums, rows, cols, m, s, params_tiled);
       return;

@@ -725,20 +725,24 @@ static void linear(const DLinear &L, const float *x, const Workspace &w, float *
               w.qa.as<_Float16>(), w.qmm.as<uint8_t>(), L.params_tiled);
 }
 
-// The lane-order activation buffer for a quantizer of m rows of k columns to
-// fill: null unless a product on them, of r0, r1 or r2 rows (0: none), takes the
-// streamed kernel.
-static _Float16 *stream_acts(const rai_model &md, int m, int k, const Workspace &w, int r0, int r1 = 0, int r2 = 0) {
-  auto wants = [&](int r) { return r > 0 && m > 1 && w4a8_route(r, k, m, md.cfg.group_size) == W4Route::kStream; };
-  return wants(r0) || wants(r1) || wants(r2) ? w.qa.as<_Float16>() : nullptr;
+// The products that read a quantized input (null or without rows: none).
+using Readers = std::initializer_list<const DLinear *>;
+
+// The lane-order activation buffer for a quantizer of m rows to fill: null
+// unless a product that reads them takes the streamed kernel.
+static _Float16 *stream_acts(const Workspace &w, int m, Readers readers) {
+  for (const DLinear *L : readers)
+    if (L && L->rows > 0 && m > 1 &&
+        w4a8_route(L->rows, L->cols, m, L->gs, L->params_tiled != nullptr) == W4Route::kStream)
+      return w.qa.as<_Float16>();
+  return nullptr;
 }
 
-// For products of r0 and r1 (0: none) rows.
 static void quantize(const rai_model &md, const float *x, int m, int k, const Workspace &w,
-                     hipStream_t s, int r0, int r1 = 0, int r2 = 0) {
+                     hipStream_t s, Readers readers) {
   if (fused_quant_ok(k, md.cfg.group_size)) {
     launch_quant(x, m, k, md.cfg.group_size, w.q_split.as<int8_t>(), nullptr, w.qscale.as<float>(),
-                 w.qsum.as<float>(), s, stream_acts(md, m, k, w, r0, r1, r2));
+                 w.qsum.as<float>(), s, stream_acts(w, m, readers));
   } else {
     launch_quantize(x, m, k, md.cfg.group_size, w.q_nat.as<int8_t>(), w.q_split.as<int8_t>(),
                     w.qscale.as<float>(), w.qsum.as<float>(), s);
@@ -872,11 +876,11 @@ static void moe_block(const rai_model &md, const DLayer &L, Workspace &w, int m,
       HIP_CHECK(hipMemcpyAsync(w.xg.as<float>() + (size_t)i * H, w.normed.as<float>() + (size_t)tok[e][i] * H,
                                sizeof(float) * H, hipMemcpyDeviceToDevice, s));
     const DLinear *ex = &L.experts[(size_t)e * 3];
-    quantize(md, w.xg.as<float>(), me, H, w, s, ex[0].rows, ex[1].rows);
+    quantize(md, w.xg.as<float>(), me, H, w, s, {&ex[0], &ex[1]});
     linear(ex[0], w.xg.as<float>(), w, w.gg.as<float>(), me, s);
     linear(ex[1], w.xg.as<float>(), w, w.ug.as<float>(), me, s);
     launch_silu_mul(w.gg.as<float>(), w.ug.as<float>(), me, F, s);
-    quantize(md, w.gg.as<float>(), me, F, w, s, ex[2].rows);
+    quantize(md, w.gg.as<float>(), me, F, w, s, {&ex[2]});
     linear(ex[2], w.gg.as<float>(), w, w.yg.as<float>(), me, s);
     for (int i = 0; i < me; ++i)
       HIP_CHECK(hipMemcpyAsync(eo + ((size_t)tok[e][i] * K + slot[e][i]) * H, w.yg.as<float>() + (size_t)i * H,
@@ -932,13 +936,13 @@ static void forward_enqueue(rai_model &md, rai_kv &kv, Workspace &w, int m, size
   // enter_block (model.rs:319-337): RMSNorm, then one quantization of the
   // normalised rows shared by the projections that read them (the
   // reference re-quantizes per projection; the result is identical).
-  auto norm_then_quant = [&](const float *wn, int r0, int r1, int r2) {
+  auto norm_then_quant = [&](const float *wn, Readers readers) {
     if (fused_quant_ok(H, gs)) {
       launch_norm_quant(hid, wn, normed, m, H, c.norm_eps, gs, w.q_split.as<int8_t>(), nullptr,
-                        w.qscale.as<float>(), w.qsum.as<float>(), s, stream_acts(md, m, H, w, r0, r1, r2));
+                        w.qscale.as<float>(), w.qsum.as<float>(), s, stream_acts(w, m, readers));
     } else {
       launch_rmsnorm(hid, wn, normed, nullptr, m, H, c.norm_eps, s);
-      quantize(md, normed, m, H, w, s, r0, r1, r2);
+      quantize(md, normed, m, H, w, s, readers);
     }
   };
   // One token: the projections behind a norm normalise and quantize the
@@ -950,9 +954,9 @@ static void forward_enqueue(rai_model &md, rai_kv &kv, Workspace &w, int m, size
     const bool qkv1 = norm1 && L.qkv.rows && w4a8_norm1_path(L.qkv.rows, L.qkv.cols, L.qkv.gs);
     if (!qkv1) {
       if (L.qkv.rows)
-        norm_then_quant(L.in_norm, L.qkv.rows, 0, 0);
+        norm_then_quant(L.in_norm, {&L.qkv});
       else
-        norm_then_quant(L.in_norm, L.lin[0].rows, L.lin[1].rows, L.lin[2].rows);
+        norm_then_quant(L.in_norm, {&L.lin[0], &L.lin[1], &L.lin[2]});
     }
     float *qp, *kp, *vp;
     int q_ld, kv_ld;
@@ -997,14 +1001,21 @@ static void forward_enqueue(rai_model &md, rai_kv &kv, Workspace &w, int m, size
     const DLinear &O = L.lin[3];
     if (!(norm1 && launch_w4a8_dec(hid, hid, O.nib, O.params, nullptr, nullptr, nullptr, O.rows, O.cols, O.gs,
                                    w.att.as<float>(), nullptr, 0.0f, s))) {
-      quantize(md, w.att.as<float>(), m, qd, w, s, O.rows);
+      quantize(md, w.att.as<float>(), m, qd, w, s, {&O});
       linear(O, w.att.as<float>(), w, hid, m, s, hid);
     }
     const bool gu1 = norm1 && L.gate_up.rows && fused_quant_ok(F, gs) &&
                      w4a8_norm1_path(L.gate_up.rows, L.gate_up.cols, L.gate_up.gs);
     // gate|up as one product or two (a sparse layer's experts read the rows
     // themselves).
-    if (!gu1) norm_then_quant(L.post_norm, c.num_experts ? 0 : L.gate_up.rows, c.num_experts ? 0 : F, 0);
+    if (!gu1) {
+      if (c.num_experts)
+        norm_then_quant(L.post_norm, {});
+      else if (L.gate_up.rows)
+        norm_then_quant(L.post_norm, {&L.gate_up});
+      else
+        norm_then_quant(L.post_norm, {&L.lin[4], &L.lin[5]});
+    }
     if (c.num_experts > 0 && moe_on_device(md) && m > kMoeEntryTokens && moe_tiles_ok(c)) {
       moe_block_device_large(md, li, w, m, s);
     } else if (c.num_experts > 0 && moe_on_device(md)) {
@@ -1042,10 +1053,10 @@ static void forward_enqueue(rai_model &md, rai_kv &kv, Workspace &w, int m, size
       }
       if (fused_quant_ok(F, gs)) {
         launch_silu_quant(gp, up, m, F, gu_ld, gs, w.q_split.as<int8_t>(), nullptr, w.qscale.as<float>(),
-                          w.qsum.as<float>(), s, stream_acts(md, m, F, w, L.lin[6].rows));
+                          w.qsum.as<float>(), s, stream_acts(w, m, {&L.lin[6]}));
       } else {
         launch_silu_mul(gp, up, m, F, s);
-        quantize(md, gp, m, F, w, s, L.lin[6].rows);
+        quantize(md, gp, m, F, w, s, {&L.lin[6]});
       }
       // down with the second residual add (model.rs:955-960) in its epilogue.
       linear(L.lin[6], gp, w, hid, m, s, hid);
@@ -1073,10 +1084,10 @@ static void logits(rai_model &md, Workspace &w, int m, hipStream_t s) {
     if (fused_quant_ok(H, c.group_size)) {
       launch_norm_quant(w.hid.as<float>(), md.final_norm, w.normed.as<float>(), m, H, c.norm_eps, c.group_size,
                         w.q_split.as<int8_t>(), nullptr, w.qscale.as<float>(), w.qsum.as<float>(), s,
-                        stream_acts(md, m, H, w, md.lm_head.rows));
+                        stream_acts(w, m, {&md.lm_head}));
     } else {
       launch_rmsnorm(w.hid.as<float>(), md.final_norm, w.normed.as<float>(), nullptr, m, H, c.norm_eps, s);
-      quantize(md, w.normed.as<float>(), m, H, w, s, md.lm_head.rows);
+      quantize(md, w.normed.as<float>(), m, H, w, s, {&md.lm_head});
     }
     linear(md.lm_head, w.normed.as<float>(), w, w.logits.as<float>(), m, s);
   } else {
@@ -1639,7 +1650,7 @@ int rai_w4a8_matmul_dev(float *out, const uint8_t *nib, const uint8_t *params, c
       return RAI_OK;
     }
     const bool fast = rai::w4a8_fast_path((int)cols, (int)gs, nib, params);
-    const rai::W4Route route = m > 1 && fast ? rai::w4a8_route((int)rows, (int)cols, (int)m, (int)gs)
+    const rai::W4Route route = m > 1 && fast ? rai::w4a8_route((int)rows, (int)cols, (int)m, (int)gs, false)
                                              : rai::W4Route::kValu;
     const bool wqa = route == rai::W4Route::kStream, mm = route == rai::W4Route::kMm;
     const size_t nq = m * cols, ng = m * groups * 4;
@@ -1793,7 +1804,7 @@ int rai_w4a8_matmul_noalloc_dev(float *out, const uint8_t *nib, const uint8_t *p
     // The streamed kernel's activations and the GEMM's records share a place;
     // what does not fit it (two tokens of more than 393216 columns) takes the
     // tiled VALU kernel.
-    const rai::W4Route route = m > 1 && fast ? rai::w4a8_route((int)rows, (int)cols, (int)m, (int)gs)
+    const rai::W4Route route = m > 1 && fast ? rai::w4a8_route((int)rows, (int)cols, (int)m, (int)gs, false)
                                              : rai::W4Route::kValu;
     const bool wqa = route == rai::W4Route::kStream &&
                      rai::qa_bytes((int)m, (int)cols, (int)gs) <= rai::kNaMmBytes;
@@ -1841,7 +1852,8 @@ int rai_w4a8_time_dev(float *out, const uint8_t *nib, const uint8_t *params, con
     HIP_CHECK(hipEventCreate(&e0));
     HIP_CHECK(hipEventCreate(&e1));
     const bool fast = rai::w4a8_fast_path((int)cols, (int)gs, nib, params);
-    const rai::W4Route route = m > 1 && fast ? rai::w4a8_route((int)rows, (int)cols, (int)m, (int)gs)
+    const bool tl = rai::params_tile16_ok((int)rows, (int)cols, (int)gs);
+    const rai::W4Route route = m > 1 && fast ? rai::w4a8_route((int)rows, (int)cols, (int)m, (int)gs, tl)
                                              : rai::W4Route::kValu;
     rai::DevBuf qa, mm;
     if (route == rai::W4Route::kStream) qa.alloc(rai::qa_bytes((int)m, (int)cols, (int)gs));
@@ -1852,7 +1864,7 @@ int rai_w4a8_time_dev(float *out, const uint8_t *nib, const uint8_t *params, con
     const size_t nib_bytes = rows * cols / 2, par_bytes = rows * groups * 4;
     // The parameters' tile-layout copies, as a loaded model holds them.
     rai::DevBuf tiled;
-    if (route == rai::W4Route::kRp && rai::params_tile16_ok((int)rows, (int)cols, (int)gs)) {
+    if (route == rai::W4Route::kRp && tl) {
       tiled.alloc(copies * par_bytes);
       for (size_t c = 0; c < copies; ++c)
         rai::launch_params_tile16(params + c * par_bytes, (int)rows, (int)cols, tiled.as<uint8_t>() + c * par_bytes,

@@ -222,6 +222,34 @@ def test_small_batches_every_group_size(rai, ora, gs, cols, rows, m):
     _both_calls(rai, ora, rows, cols, m, gs)
 
 
+# Both sides of the lines between the kernels of 2..64 tokens: the register-
+# pipelined one with its ring of two (K an odd multiple of 256) and past 24 tokens,
+# the VALU one at two to four tokens.
+@pytest.mark.parametrize("gs,rows,cols,m", [
+    (32, 70, 256, 12), (32, 70, 768, 64), (32, 1100, 1280, 65), (32, 4097, 1280, 17), (32, 5009, 2816, 2),
+    (32, 5009, 2816, 8), (32, 5009, 2816, 9), (32, 16401, 768, 12), (32, 16401, 2816, 11), (32, 16401, 1280, 13),
+    (32, 5009, 5376, 4), (32, 5009, 5376, 5), (32, 4999, 5376, 3), (32, 130, 13056, 4),
+    (32, 513, 512, 25), (32, 1024, 2048, 64), (32, 2561, 1024, 47), (32, 3073, 512, 64), (32, 200, 4608, 40),
+    (32, 1025, 4608, 64), (32, 60, 14336, 33),
+    (32, 300, 1056, 2), (32, 5009, 1056, 3), (32, 8209, 96, 4), (64, 200, 192, 2), (64, 200, 1088, 2),
+    (64, 5009, 192, 2), (64, 5009, 576, 3), (64, 8209, 2048, 4), (64, 12289, 320, 3), (64, 12305, 4160, 3),
+    (128, 200, 2176, 2), (128, 8209, 4224, 3), (128, 8209, 640, 4), (128, 12305, 640, 3)])
+def test_small_batch_kernel_lines(rai, ora, gs, rows, cols, m):
+    _both_calls(rai, ora, rows, cols, m, gs)
+
+
+@pytest.mark.parametrize("hidden,ffn", [(1024, 2816), (1280, 1536), (2560, 5376)])
+@pytest.mark.parametrize("m", [2, 3, 9, 24, 25, 40, 64])
+def test_small_batch_layers_with_tiled_parameters(rai, ora, hidden, ffn, m):
+    """Group 32, where a model also holds its parameters in 16-row tiles."""
+    img = rai.synth_model(hidden, 1, hidden // 64, 2, 64, ffn, 400, 128, group_size=32, seed=m)
+    gm, om = rai.RaiModel.from_bytes(img, max_groups=1024), ora.Model(img, 0)
+    h = np.random.default_rng(m).normal(0.0, 1.0, (m, hidden)).astype(np.float32)
+    got = gm.forward_batch(h, np.arange(m), gm.create_kv_cache(128))
+    want = om.forward_batch(h, np.arange(m), om.create_kv(128))
+    assert np.array_equal(_bits(got).reshape(-1), _bits(want).reshape(-1))
+
+
 @pytest.mark.parametrize("gs", [32, 64, 128])
 @pytest.mark.parametrize("m", [2, 9, 40, 100])
 def test_small_batch_layers(rai, ora, gs, m):
