@@ -1712,18 +1712,102 @@ static int g_pv_spin = kPvSpin;
 
 void set_attention_spin(int polls) { g_pv_spin = polls > 0 ? polls : kPvSpin; }
 
+// PV of m tokens from position p0 on (out [m][nh * hd]): the streamed kernel of
+// the head layout, or the general one.
+static void launch_pv(const float *S, const float *vc, int cap, int vstride, int p0, int m, int nh, int nkv, int hd,
+                      int sstride, float *out, const int *st, int *err, hipStream_t s) {
+  const size_t total = (size_t)m * nh * hd;
+  const int G = nh / nkv;
+  const int DL = (G == 2) ? 32 : 16;
+  const bool stream = vstride > 0 && vstride % 64 == 0 &&
+                      (G == 1 || G == 2 || G == 4 || G == 8 || G == 16) && hd % DL == 0;
+  if (stream) {
+    // Tokens per block: one for one or two tokens (more blocks), three up
+    // to twelve (the verify batch), four beyond; tile length and loader
+    // waves measured on 4.1K-4.35K positions with V streamed from HBM (one
+    // token: 512-position tiles and two loaders, 21.0 -> 20.0 us against
+    // 256 and four; the loaders' registers spill from 640 positions or four
+    // loaders at 512; three tokens: 256 and three).
+    if (G == 4 && m > 12 && hd % 32 == 0)
+      // Prefill batches (128 tokens per launch): 32-dim slices, eight
+      // tokens per block, four per compute lane (each V read feeds four
+      // chains; a kv head's probability rows are read by four slice
+      // blocks instead of eight), 64-position tiles and two loaders, whose
+      // registers (126 per lane) let two blocks share a CU: 0.483 s per
+      // 4095-token Mistral-7B prefill against 0.491 with 128-position
+      // tiles (236 registers, one block per CU) and 0.506 with 64-token
+      // launches.
+      launch_pv_flag<32, 4, 64, 8, 2, 4>(S, vc, vstride, p0, m, nh, nkv, hd, sstride, out, st, err, g_pv_spin,
+                                         s);
+    else if (G == 4 && m > 12)
+      launch_pv_flag<16, 4, 128, 8, 4, 2>(S, vc, vstride, p0, m, nh, nkv, hd, sstride, out, st, err, g_pv_spin,
+                                          s);
+    else if (G == 4 && m > 2)
+      launch_pv_flag<16, 4, 256, 3, 3>(S, vc, vstride, p0, m, nh, nkv, hd, sstride, out, st, err, g_pv_spin, s);
+    else if (G == 4)
+      launch_pv_flag<16, 4, 512, 1, 2>(S, vc, vstride, p0, m, nh, nkv, hd, sstride, out, st, err, g_pv_spin, s);
+    else if (G == 8 && m == 1)
+      // One token, eight query heads per kv head (TinyLlama-shaped): 8-dim
+      // slices (one compute wave of 8 heads x 8 dims) with 512-position
+      // tiles and two loaders: 11.97 us at 2048 positions, head_dim 64,
+      // against 14.06 with 16-dim slices, 256-position tiles and six
+      // loaders (12.3-14.0 for the four other shapes measured).
+      launch_pv_flag<8, 8, 512, 1, 2>(S, vc, vstride, p0, m, nh, nkv, hd, sstride, out, st, err, g_pv_spin, s);
+    else if (G == 8)
+      launch_pv_flag<16, 8, 256, 1, 6>(S, vc, vstride, p0, m, nh, nkv, hd, sstride, out, st, err, g_pv_spin, s);
+    else if (G == 16)
+      launch_pv_flag<16, 16, 256, 1, 4>(S, vc, vstride, p0, m, nh, nkv, hd, sstride, out, st, err, g_pv_spin, s);
+    else if (G == 2)
+      launch_pv_flag<32, 2, 128, 1, 7>(S, vc, vstride, p0, m, nh, nkv, hd, sstride, out, st, err, g_pv_spin, s);
+    else if (m > 4)
+      // One query head per kv head: 16-d slices, so a wave's four lane
+      // rows take four tokens of one head (eight tokens in two compute
+      // waves here) and a 256-position tile fits the loaders' registers
+      // (64-d slices needed 64-position tiles: 22.5 -> 15.1 us at nine
+      // tokens and 2100 positions, 19.1 -> 13.4 us at one).
+      launch_pv_flag<16, 1, 256, 8, 3>(S, vc, vstride, p0, m, nh, nkv, hd, sstride, out, st, err, g_pv_spin, s);
+    else
+      launch_pv_flag<16, 1, 256, 4, 2>(S, vc, vstride, p0, m, nh, nkv, hd, sstride, out, st, err, g_pv_spin, s);
+  } else if (vstride > 0) {
+    hipLaunchKernelGGL(k_pv_any<true>, dim3((unsigned)((total + 63) / 64)), dim3(64), 0, s, S,
+                       vc, cap, vstride, p0, m, nh, nkv, hd, sstride, out, st);
+  } else {
+    hipLaunchKernelGGL(k_pv_any<false>, dim3((unsigned)((total + 63) / 64)), dim3(64), 0, s, S,
+                       vc, cap, 0, p0, m, nh, nkv, hd, sstride, out, st);
+  }
+}
+
+// Whether the matrix-core PV takes a launch of m > kPvMmTokens tokens.  It runs
+// one chain over the positions per wave, 35 ns a position however few waves
+// there are, until 1024 of them fill the chip (43 ns); the streamed kernels' time
+// grows with their blocks, about 20 ns a position per 1000 (three times that
+// with four query heads per kv head, whose blocks take eight tokens of four
+// heads, 1.4 times with sixteen), from a floor of 10 to 17 ns per 128 tokens.
+// 256 tokens at 3840 positions, head size 128 and (64), streamed / matrix cores
+// (us): 32 heads on 8 251 / 173, 16 on 4 146 / 145, 8 on 2 131 / 140, 8 on 8 157 /
+// 141, 16 on 16 320 / 146, 8 on 4 317 / 142, (32 on 4 336 / 151), (8 on 1 89 /
+// 138), (6 on 6 79 / 139), (32 on 2 235 / 145); 176 tokens: 8 on 8 117 / 138, 32
+// on 8 199 / 162.
+static bool pv_mm_best(int m, int nh, int nkv, int hd) {
+  const int64_t d16 = (int64_t)nkv * (hd / 16), t8 = (m + 7) / 8;  // blocks per token row, token tiles of eight
+  switch (nh / nkv) {
+    case 1: return d16 * t8 >= 1800;
+    case 2: return d16 / 2 * m >= 1800;
+    case 4: return d16 / 2 * t8 * 3 >= 1800;
+    case 8: return d16 * m >= 1800;
+    case 16: return d16 * m * 7 / 5 >= 1800;
+    default: return true;  // no streamed kernel
+  }
+}
+
 void launch_attention(const float *q, int q_ld, const float *kc, const float *vc, int cap,
                       int vstride, int pos0, int m, int nh, int nkv, int hd, float scale,
                       float *out, float *scores, hipStream_t s, const int *st, int *err, int stages,
                       int span) {
-  // Prefill batches: kAttnTokens per launch, so that the PV chains (one wave per
-  // 16 tokens, head and 64 dimensions) fill the chip; the streamed PV kernel
-  // keeps the 128 it was measured at.
+  // Prefill batches: kAttnTokens per launch; without a matrix-core path 128.
   const bool mm = !st && attn_mm_path(q, q_ld, kc, vc, vstride, m, nh, nkv, hd);
-  // A lowered poll limit asks for the kernel that waits.
-  const bool pv_mm = mm && g_pv_spin == kPvSpin;
   for (int t0 = 0, mt; t0 < m; t0 += mt) {
-    mt = pv_mm && m - t0 > kPvMmTokens ? std::min(kAttnTokens, m - t0) : std::min(128, m - t0);
+    mt = mm && m - t0 > kPvMmTokens ? std::min(kAttnTokens, m - t0) : std::min(128, m - t0);
     const int p0 = pos0 + t0;
     // With a step record the position is on the device: the grids, the
     // score stride and the softmax kernel are those of the span of
@@ -1781,67 +1865,15 @@ void launch_attention(const float *q, int q_ld, const float *kc, const float *vc
     } else {
       hipLaunchKernelGGL(k_softmax_l, dim3(nh, mt), dim3(512), 0, s, scores, p0, nh, sstride, st);
     }
-    const size_t total = (size_t)mt * nh * hd;
-    const int G = nh / nkv;
-    const int DL = (G == 2) ? 32 : 16;
-    const bool stream = vstride > 0 && vstride % 64 == 0 &&
-                        (G == 1 || G == 2 || G == 4 || G == 8 || G == 16) && hd % DL == 0;
     if (!(stages & 4)) {
-    } else if (pv_mm && mt > kPvMmTokens) {
+    } else if (mm && mt > kPvMmTokens && pv_mm_best(mt, nh, nkv, hd)) {
       launch_pv_mm(scores, vc, vstride, p0, mt, nh, nkv, hd, sstride, ot, s);
-    } else if (stream) {
-      // Tokens per block: one for one or two tokens (more blocks), three up
-      // to twelve (the verify batch), four beyond; tile length and loader
-      // waves measured on 4.1K-4.35K positions with V streamed from HBM (one
-      // token: 512-position tiles and two loaders, 21.0 -> 20.0 us against
-      // 256 and four; the loaders' registers spill from 640 positions or four
-      // loaders at 512; three tokens: 256 and three).
-      if (G == 4 && mt > 12 && hd % 32 == 0)
-        // Prefill batches (128 tokens per launch): 32-dim slices, eight
-        // tokens per block, four per compute lane (each V read feeds four
-        // chains; a kv head's probability rows are read by four slice
-        // blocks instead of eight), 64-position tiles and two loaders, whose
-        // registers (126 per lane) let two blocks share a CU: 0.483 s per
-        // 4095-token Mistral-7B prefill against 0.491 with 128-position
-        // tiles (236 registers, one block per CU) and 0.506 with 64-token
-        // launches.
-        launch_pv_flag<32, 4, 64, 8, 2, 4>(scores, vc, vstride, p0, mt, nh, nkv, hd, sstride, ot, st, err, g_pv_spin,
-                                           s);
-      else if (G == 4 && mt > 12)
-        launch_pv_flag<16, 4, 128, 8, 4, 2>(scores, vc, vstride, p0, mt, nh, nkv, hd, sstride, ot, st, err, g_pv_spin,
-                                            s);
-      else if (G == 4 && mt > 2)
-        launch_pv_flag<16, 4, 256, 3, 3>(scores, vc, vstride, p0, mt, nh, nkv, hd, sstride, ot, st, err, g_pv_spin, s);
-      else if (G == 4)
-        launch_pv_flag<16, 4, 512, 1, 2>(scores, vc, vstride, p0, mt, nh, nkv, hd, sstride, ot, st, err, g_pv_spin, s);
-      else if (G == 8 && mt == 1)
-        // One token, eight query heads per kv head (TinyLlama-shaped): 8-dim
-        // slices (one compute wave of 8 heads x 8 dims) with 512-position
-        // tiles and two loaders: 11.97 us at 2048 positions, head_dim 64,
-        // against 14.06 with 16-dim slices, 256-position tiles and six
-        // loaders (12.3-14.0 for the four other shapes measured).
-        launch_pv_flag<8, 8, 512, 1, 2>(scores, vc, vstride, p0, mt, nh, nkv, hd, sstride, ot, st, err, g_pv_spin, s);
-      else if (G == 8)
-        launch_pv_flag<16, 8, 256, 1, 6>(scores, vc, vstride, p0, mt, nh, nkv, hd, sstride, ot, st, err, g_pv_spin, s);
-      else if (G == 16)
-        launch_pv_flag<16, 16, 256, 1, 4>(scores, vc, vstride, p0, mt, nh, nkv, hd, sstride, ot, st, err, g_pv_spin, s);
-      else if (G == 2)
-        launch_pv_flag<32, 2, 128, 1, 7>(scores, vc, vstride, p0, mt, nh, nkv, hd, sstride, ot, st, err, g_pv_spin, s);
-      else if (mt > 4)
-        // One query head per kv head: 16-d slices, so a wave's four lane
-        // rows take four tokens of one head (eight tokens in two compute
-        // waves here) and a 256-position tile fits the loaders' registers
-        // (64-d slices needed 64-position tiles: 22.5 -> 15.1 us at nine
-        // tokens and 2100 positions, 19.1 -> 13.4 us at one).
-        launch_pv_flag<16, 1, 256, 8, 3>(scores, vc, vstride, p0, mt, nh, nkv, hd, sstride, ot, st, err, g_pv_spin, s);
-      else
-        launch_pv_flag<16, 1, 256, 4, 2>(scores, vc, vstride, p0, mt, nh, nkv, hd, sstride, ot, st, err, g_pv_spin, s);
-    } else if (vstride > 0) {
-      hipLaunchKernelGGL(k_pv_any<true>, dim3((unsigned)((total + 63) / 64)), dim3(64), 0, s, scores,
-                         vc, cap, vstride, p0, mt, nh, nkv, hd, sstride, ot, st);
     } else {
-      hipLaunchKernelGGL(k_pv_any<false>, dim3((unsigned)((total + 63) / 64)), dim3(64), 0, s, scores,
-                         vc, cap, 0, p0, mt, nh, nkv, hd, sstride, ot, st);
+      // The streamed kernels at the 128 tokens a launch that they are shaped
+      // for.
+      for (int u = 0; u < mt; u += 128)
+        launch_pv(scores + (size_t)u * nh * sstride, vc, cap, vstride, p0 + u, std::min(128, mt - u), nh, nkv, hd,
+                  sstride, ot + (size_t)u * nh * hd, st, err, s);
     }
   }
 }

@@ -230,10 +230,12 @@ void launch_rope_store(float *q, float *k, const float *v, const float *cos_t, c
 // tokens are processed in groups of kAttnTokens.
 constexpr int kAttnTokens = 256;
 size_t attention_scores_floats(int m, int nh, int ctx);
-// The scores and PV of attn_mm.hip (prefill batches of kAttnMmTokens and
-// more, PV past kPvMmTokens a launch); the softmax between them is
-// launch_attention's.  At 3072 to 4096 positions PV takes 143 us for up to 256
-// tokens there, 107 per 128 tokens in the streamed kernel.
+// The scores and PV of attn_mm.hip: the scores of prefill batches of
+// kAttnMmTokens and more (never slower than the DPP-FMA kernel from there on over
+// ten head layouts from 4 heads on 1 of 64 to 64 on 8 of 128 at 0 to 8000
+// positions: 16 tokens at 3072 17.1 -> 11.2 us at 32 heads on 8, 6.5 -> 5.5 at 4 on
+// 1), PV past kPvMmTokens a launch where the head layout gives it enough work
+// (pv_mm_best, fused.hip); the softmax between them is launch_attention's.
 constexpr int kAttnMmTokens = 16, kPvMmTokens = 160;
 bool attn_mm_path(const float *q, int q_ld, const float *kc, const float *vc, int vstride, int m, int nh, int nkv,
                   int hd);

@@ -304,6 +304,32 @@ def test_prefill_attention(rai, ora, heads, kv, hd, first, m):
             assert np.array_equal(_bits(got).reshape(-1), _bits(want).reshape(-1)), (a, b)
 
 
+# Query heads per kv head on both sides of the rule between the two PV kernels
+# past 160 tokens (5, 6 / 2: matrix cores; 4, 8, 1: streamed in parts of 128),
+# behind each softmax of long rows.
+@pytest.mark.parametrize("heads,kv,hd", [(5, 1, 64), (6, 2, 128), (4, 1, 64), (8, 1, 64), (3, 3, 64)])
+@pytest.mark.parametrize("first", [4101, 8300, 16500])
+def test_prefill_attention_of_long_contexts(rai, ora, heads, kv, hd, first):
+    H, m = heads * hd, 203
+    cap = first + 2 * m
+    img = rai.synth_model(H, 1, heads, kv, hd, 128, 64, cap, group_size=32, embed_group_size=32, seed=first)
+    gm = rai.RaiModel.from_bytes(img)
+    h = np.random.default_rng(first).normal(0.0, 1.0, (first + m, H)).astype(np.float32)
+    whole, parts = gm.create_kv_cache(cap), gm.create_kv_cache(cap)
+    for kvc in (whole, parts):
+        gm.forward_batch(h[:first], np.arange(first), kvc)
+    got = gm.forward_batch(h[first:], np.arange(first, first + m), whole)
+    cuts = [(first, first + 101), (first + 101, first + m)]
+    want = np.concatenate([gm.forward_batch(h[a:b], np.arange(a, b), parts) for a, b in cuts])
+    assert np.array_equal(_bits(got), _bits(want))
+    if first == 4101 and heads == 5:
+        om = ora.Model(img, 0)
+        ok = om.create_kv(cap)
+        om.forward_batch(h[:first], np.arange(first), ok)
+        want = om.forward_batch(h[first:], np.arange(first, first + m), ok)
+        assert np.array_equal(_bits(got).reshape(-1), _bits(want).reshape(-1))
+
+
 @pytest.mark.parametrize("gs", [32, 64, 128])
 @pytest.mark.parametrize("rows,cols", [((1, 3, 17), 256), ((16401, 40, 40), 256), ((100, 530), 1152), ((70, 70), 4096),
                                        ((33, 34, 35), 4224)])
