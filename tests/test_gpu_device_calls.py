@@ -286,6 +286,17 @@ def test_host_buffers_of_every_size(rai, m):
         assert np.array_equal(_bits(lg[i]), _bits(gm.hidden_to_logits(got[i])))
 
 
+def test_rows_past_the_positions_come_back_unchanged(rai):
+    """forward_batch of more rows than positions: the others are the input's."""
+    gm = rai.RaiModel.from_bytes(rai.synth_model(256, 1, 4, 4, 64, 512, 100, 64, group_size=32, seed=3))
+    h = np.random.default_rng(0).normal(0.0, 1.0, (5, 256)).astype(np.float32)
+    want = gm.forward_batch(h[:3], np.arange(3), gm.create_kv_cache(64))
+    for _ in range(8):  # so that fresh memory of this size is not the input by chance
+        np.full_like(h, 7.0)
+    got = gm.forward_batch(h, np.arange(3), gm.create_kv_cache(64))
+    assert np.array_equal(_bits(got[:3]), _bits(want)) and np.array_equal(_bits(got[3:]), _bits(h[3:]))
+
+
 @pytest.mark.parametrize("heads,kv,hd", [(4, 1, 64), (3, 3, 128), (6, 3, 64), (8, 1, 128), (5, 1, 64)])
 @pytest.mark.parametrize("first,m", [(0, 16), (1, 17), (5, 33), (63, 64), (64, 161), (130, 300), (1, 530)])
 def test_prefill_attention(rai, ora, heads, kv, hd, first, m):
