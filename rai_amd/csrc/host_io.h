@@ -1,5 +1,6 @@
-// Host buffers of the model calls: pageable memory to and from the device
-// through pinned staging blocks and a few copy threads.
+// Host side of the model calls' transfers between pageable memory and the
+// device: a few copy threads, and the bookkeeping of the pinned staging blocks
+// (no HIP here, so that the host can test it alone).
 //
 // hipMemcpyAsync on pageable memory moved 16.8 MB of hidden states at 12 to 15
 // GB/s and took 30 to 70 us for a few kilobytes, each with a wait of its own
@@ -10,8 +11,6 @@
 #ifndef RAI_HOST_IO_H
 #define RAI_HOST_IO_H
 
-#include <hip/hip_runtime.h>
-
 #include <algorithm>
 #include <atomic>
 #include <condition_variable>
@@ -19,7 +18,6 @@
 #include <cstring>
 #include <mutex>
 #include <thread>
-#include <vector>
 
 namespace rai {
 
@@ -109,13 +107,54 @@ class CopyPool {
   int workers_ = 0;
 };
 
-// A pinned block and the events of its pieces.
-struct PinBlock {
-  static constexpr int kEvents = 8;
-  uint8_t *p = nullptr;
-  size_t n = 0;
-  int dev = 0;
-  hipEvent_t ev[kEvents] = {};
+// At most Max blocks per device, in use and free together, for blocks that cost
+// milliseconds to make.  Block has n (bytes) and dev.  Nothing here allocates or
+// throws; making and freeing a block is the caller's.
+enum class PoolTake {
+  kBlock,    // b is a free block of n bytes or more
+  kMake,     // none, but one more may be made: then give() it, or gone()
+  kReplace,  // b is a smaller free block to drop for a new one: as kMake
+  kNone      // Max are in use
+};
+template <class Block, int Max, int Devices = 64>
+class BoundedPool {
+ public:
+  PoolTake take(size_t n, int dev, Block &b) noexcept {
+    if (dev < 0 || dev >= Devices) return PoolTake::kNone;
+    std::lock_guard<std::mutex> lk(m_);
+    Slots &s = d_[dev];
+    int best = -1;  // the smallest that fits
+    for (int i = 0; i < s.nfree; ++i)
+      if (s.free[i].n >= n && (best < 0 || s.free[i].n < s.free[best].n)) best = i;
+    if (best < 0 && s.total < Max) {
+      ++s.total;
+      return PoolTake::kMake;
+    }
+    if (s.nfree == 0) return PoolTake::kNone;
+    const int i = best < 0 ? 0 : best;
+    b = s.free[i];
+    s.free[i] = s.free[--s.nfree];
+    return best < 0 ? PoolTake::kReplace : PoolTake::kBlock;
+  }
+  // The caller's block is free again.
+  void give(const Block &b) noexcept {
+    std::lock_guard<std::mutex> lk(m_);
+    Slots &s = d_[b.dev];
+    s.free[s.nfree++] = b;
+  }
+  // A block of the device was dropped, or not made after kMake or kReplace.
+  void gone(int dev) noexcept {
+    std::lock_guard<std::mutex> lk(m_);
+    --d_[dev].total;
+  }
+
+ private:
+  struct Slots {
+    Block free[Max];
+    int nfree = 0, total = 0;
+  };
+  std::mutex m_;
+  Slots d_[Devices];
 };
 
 }  // namespace rai

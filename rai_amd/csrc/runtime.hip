@@ -172,24 +172,56 @@ static void host_copy(void *dst, const void *src, size_t n, hipStream_t s, void 
                      static_cast<const uint32_t *>(src2), n2);
 }
 
+// A pinned block and the events of its pieces.
+struct PinBlock {
+  static constexpr int kEvents = 8;
+  uint8_t *p = nullptr;
+  size_t n = 0;
+  int dev = 0;
+  hipEvent_t ev[kEvents] = {};
+};
+
 // A call's pinned staging, from a process-wide pool (pinning pages costs
-// milliseconds): a call holds its block alone until its stream is finished.
-// A transfer is cut into pieces of at most half of kStageMax; at most two
-// blocks are kept.
+// milliseconds): a call holds its block alone until its stream is finished.  A
+// transfer is cut into pieces of at most 16 MiB, and a block holds one in each
+// direction.  A device has at most eight blocks of up to 2 MiB and two of up to
+// 33 MiB, in use and kept together.  A call that finds all of its size in use,
+// or that cannot pin, copies directly between the caller's memory and the
+// device.
 class HostStage {
+  static inline BoundedPool<PinBlock, 8> g_small;
+  static inline BoundedPool<PinBlock, 2> g_large;
+  // f on the pool of blocks of n bytes.
+  template <class F>
+  static auto pool_of(size_t n, F f) {
+    return n <= (size_t(2) << 20) ? f(g_small) : f(g_large);
+  }
+
  public:
-  static constexpr size_t kStageMax = size_t(32) << 20;
   // For transfers of up to nin floats in and nout out at a time.
   HostStage(hipStream_t s, size_t nin, size_t nout) : s_(s) {
-    take(bytes(std::min(nin, kPiece)) + bytes(std::min(nout, kPiece)));
+    take(bytes(std::min(nin, kPiece)) + bytes(std::min(nout, kPiece)) + 64);  // and the error words
   }
   HostStage(const HostStage &) = delete;
   HostStage &operator=(const HostStage &) = delete;
-  ~HostStage() { give(hipStreamSynchronize(s_) == hipSuccess); }
+  ~HostStage() {
+    const bool done = hipStreamSynchronize(s_) == hipSuccess;
+    if (!b_.p) return;
+    if (done) {
+      pool_of(b_.n, [&](auto &pool) { pool.give(b_); });
+    } else {  // the work's state is unknown: never reused
+      drop(b_);
+      pool_of(b_.n, [&](auto &pool) { pool.gone(b_.dev); });
+    }
+  }
 
-  // dst (device) = src (host), n floats, on the stream.  Returns with the
-  // source read and the block in use until the stream passes this point.
+  // dst (device) = src (host), n floats, on the stream; src stays as it is
+  // until out() has returned.
   void in(float *dst, const float *src, size_t n) {
+    if (!b_.p) {
+      HIP_CHECK(hipMemcpyAsync(dst, src, n * sizeof(float), hipMemcpyHostToDevice, s_));
+      return;
+    }
     for (size_t o = 0; o < n; o += kPiece) {
       const size_t k = std::min(kPiece, n - o);
       if (o) HIP_CHECK(hipStreamSynchronize(s_));
@@ -205,6 +237,13 @@ class HostStage {
   // dst (host) = src (device), n floats; and 2 words of err to e (host) when
   // given.  Returns with the stream finished.
   void out(float *dst, const float *src, size_t n, const int *err = nullptr, int *e = nullptr) {
+    if (!b_.p) {
+      HIP_CHECK(hipGetLastError());
+      HIP_CHECK(hipMemcpyAsync(dst, src, n * sizeof(float), hipMemcpyDeviceToHost, s_));
+      if (e) HIP_CHECK(hipMemcpyAsync(e, err, 2 * sizeof(int), hipMemcpyDeviceToHost, s_));
+      HIP_CHECK(hipStreamSynchronize(s_));
+      return;
+    }
     for (size_t o = 0; o < n; o += kPiece) {
       const size_t k = std::min(kPiece, n - o);
       // At the end of the block, so that in()'s copy may still be under way.
@@ -233,7 +272,7 @@ class HostStage {
   }
 
  private:
-  static constexpr size_t kPiece = kStageMax / sizeof(float) / 2;
+  static constexpr size_t kPiece = (size_t(16) << 20) / sizeof(float);
   static size_t bytes(size_t n) { return (n * sizeof(float) + 63) & ~size_t(63); }
   // A transfer's parts: up to eight of at least 2 MB, so that the host's copy
   // of one overlaps the device's of the next.
@@ -241,65 +280,47 @@ class HostStage {
     const size_t least = (size_t(2) << 20) / sizeof(float);
     return std::max(least, ((k + PinBlock::kEvents - 1) / PinBlock::kEvents + 15) & ~size_t(15));
   }
+  // Leaves b_ without memory when there is no block for the call.
   void take(size_t n) {
-    n += 64;  // the error words
-    int dev = 0;
-    HIP_CHECK(hipGetDevice(&dev));
-    {
-      std::lock_guard<std::mutex> lk(g_m);
-      for (size_t i = 0; i < g_pins.size(); ++i)
-        if (g_pins[i].dev == dev && g_pins[i].n >= n) {
-          b_ = g_pins[i];
-          g_pins.erase(g_pins.begin() + i);
-          return;
-        }
-    }
-    size_t want = size_t(1) << 20;
-    while (want < n) want *= 2;
+    hipDevice_t dev = 0;  // the stream's, which the events must be of
+    HIP_CHECK(hipStreamGetDevice(s_, &dev));
+    n = (n + (size_t(1) << 20) - 1) & ~((size_t(1) << 20) - 1);  // nearby sizes share a block
     PinBlock b;
-    b.dev = dev;
-    HIP_CHECK(hipHostMalloc(reinterpret_cast<void **>(&b.p), want, hipHostMallocDefault));
-    b.n = want;
-    for (auto &ev : b.ev) {
-      const hipError_t r = hipEventCreateWithFlags(&ev, hipEventDisableTiming);
-      if (r != hipSuccess) {
-        drop(b);
-        HIP_CHECK(r);
-      }
+    switch (pool_of(n, [&](auto &pool) { return pool.take(n, dev, b); })) {
+      case PoolTake::kBlock: b_ = b; return;
+      case PoolTake::kNone: return;
+      case PoolTake::kReplace: drop(b); break;
+      case PoolTake::kMake: break;
     }
-    b_ = b;
-  }
-  // Keeps the block for the next call (the larger ones first), or frees it.
-  void give(bool keep) {
-    if (!b_.p) return;
-    PinBlock out = b_;
-    b_ = PinBlock{};
-    if (keep) {
-      std::lock_guard<std::mutex> lk(g_m);
-      g_pins.push_back(out);
-      out.p = nullptr;
-      if (g_pins.size() > 2) {
-        size_t least = 0;
-        for (size_t i = 1; i < g_pins.size(); ++i)
-          if (g_pins[i].n < g_pins[least].n) least = i;
-        out = g_pins[least];
-        g_pins.erase(g_pins.begin() + least);
-      }
+    PinBlock made;
+    made.dev = dev;
+    made.n = n;
+    int cur = dev;
+    bool ok = hipGetDevice(&cur) == hipSuccess && (cur == dev || hipSetDevice(dev) == hipSuccess) &&
+              hipHostMalloc(reinterpret_cast<void **>(&made.p), made.n, hipHostMallocDefault) == hipSuccess;
+    if (!ok) made.p = nullptr;
+    for (auto &ev : made.ev) {
+      if (!ok) break;
+      ok = hipEventCreateWithFlags(&ev, hipEventDisableTiming) == hipSuccess;
+      if (!ok) ev = nullptr;
     }
-    if (out.p) drop(out);
+    if (cur != dev) (void)hipSetDevice(cur);
+    if (ok) {
+      b_ = made;
+      return;
+    }
+    (void)hipGetLastError();
+    drop(made);
+    pool_of(n, [&](auto &pool) { pool.gone(dev); });
   }
   static void drop(PinBlock &b) {
     for (auto ev : b.ev)
       if (ev) (void)hipEventDestroy(ev);
-    (void)hipHostFree(b.p);
+    if (b.p) (void)hipHostFree(b.p);
   }
-  static std::mutex g_m;
-  static std::vector<PinBlock> g_pins;
   hipStream_t s_;
   PinBlock b_;
 };
-std::mutex HostStage::g_m;
-std::vector<PinBlock> HostStage::g_pins;
 
 // Tokens up to which a sparse layer runs entry by entry.
 constexpr int kMoeEntryTokens = 64;

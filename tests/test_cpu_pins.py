@@ -233,6 +233,17 @@ def test_streamed_weight_loads_stay_inside_their_arrays(tmp_path):
     assert (outside, wrong) == (0, 0)
 
 
+@pytest.mark.parametrize("flags", [[], ["-fsanitize=thread", "-g"]])
+def test_copy_threads_and_block_pool(tmp_path, flags):
+    """rai_amd/csrc/host_io.h: copies by several callers at once, and a pool that
+    never has more than its bound of blocks, also when one cannot be made."""
+    exe = tmp_path / "host_io_check"
+    subprocess.run(["g++", "-O1", "-std=c++17", "-pthread", *flags, "-I", os.path.join(ROOT, "rai_amd", "csrc"),
+                    os.path.join(ROOT, "tests", "host_io_check.cpp"), "-o", str(exe)], check=True)
+    r = subprocess.run([str(exe)], capture_output=True, text=True, timeout=120)
+    assert (r.returncode, r.stdout) == (0, "ok\n"), r.stdout + r.stderr
+
+
 # The PCG32 reference implementation's demo (pcg32_srandom_r(42, 54), then
 # pcg32_random_r): its published first outputs.
 _PCG_DEMO_42_54 = [0xA15C02B7, 0x7B47F409, 0xBA1D3330, 0x83D2F293, 0xBFA4784B, 0xCBED606E]

@@ -1,6 +1,8 @@
 """The device-pointer calls against the CPU oracle: every group size, token
 counts on both sides of each kernel's range, rows that leave partial tiles,
 and K that leaves partial tiles of groups.  Bar: bit-exact."""
+import concurrent.futures
+
 import numpy as np
 import pytest
 
@@ -284,6 +286,48 @@ def test_host_buffers_of_every_size(rai, m):
     lg = gm.hidden_to_logits_batch(got[:n], n)
     for i in (0, n // 2, n - 1):
         assert np.array_equal(_bits(lg[i]), _bits(gm.hidden_to_logits(got[i])))
+
+
+def test_logits_past_one_staging_piece(rai):
+    """More than 16 MiB of logits in one call: several pieces through one block."""
+    n, V = 64, 70001
+    gm = rai.RaiModel.from_bytes(rai.synth_model(64, 1, 1, 1, 64, 64, V, 64, group_size=32, seed=1))
+    h = np.random.default_rng(1).normal(0.0, 1.0, (n, 64)).astype(np.float32)
+    lg = gm.hidden_to_logits_batch(h, n)
+    for i in range(n):
+        assert np.array_equal(_bits(lg[i]), _bits(gm.hidden_to_logits(h[i]))), i
+
+
+def test_calls_on_several_threads(rai):
+    """Five threads, each with its own model and cache, at once: forward_batch and
+    logits through the two staging blocks, the copy threads and the direct
+    copies, device-pointer products through the shared scratch blocks."""
+    H, m, V = 1024, 600, 3001
+    img = rai.synth_model(H, 1, 8, 2, 128, 1024, V, 1200, group_size=64, seed=9)
+
+    def work(seed, models):
+        gm = models[seed]
+        r = np.random.default_rng(seed)
+        h = r.normal(0.0, 1.0, (m, H)).astype(np.float32)
+        out = []
+        for it in range(4):
+            n = m if it % 2 else 40
+            y = gm.forward_batch(h[:n], np.arange(n), gm.create_kv_cache(1200))
+            out += [y, gm.hidden_to_logits_batch(y[:33], 33)]
+            for mm, gs, rows in ((1, 32, 300), (9, 64, 500), (70, 128, 900)):
+                nib, params, x = gemv_operands(rows, 640, mm, gs, seed=seed + it)
+                dev = rai.DeviceArray.from_host
+                out.append(_call(rai, "rai_w4a8_matmul_dev", rai.DeviceArray(4 * mm * rows), dev(nib), dev(params),
+                                 dev(x), rows, 640, mm, gs))
+        return out
+
+    n = 5
+    models = [rai.RaiModel.from_bytes(img) for _ in range(n)]
+    want = [work(i, models) for i in range(n)]
+    with concurrent.futures.ThreadPoolExecutor(n) as ex:
+        got = list(ex.map(lambda i: work(i, models), range(n)))
+    for g, w in zip(got, want):
+        assert all(np.array_equal(_bits(a), _bits(b)) for a, b in zip(g, w))
 
 
 def test_rows_past_the_positions_come_back_unchanged(rai):
