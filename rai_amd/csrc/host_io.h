@@ -157,6 +157,46 @@ class BoundedPool {
   Slots d_[Devices];
 };
 
+// At most Max free blocks kept for later calls, of any device; a block in use is
+// its caller's alone.  Nothing here allocates or throws.
+template <class Block, int Max>
+class KeptBlocks {
+ public:
+  // The smallest kept block of dev with n bytes or more.
+  bool take(size_t n, int dev, Block &b) noexcept {
+    std::lock_guard<std::mutex> lk(m_);
+    int best = -1;
+    for (int i = 0; i < n_; ++i)
+      if (k_[i].dev == dev && k_[i].n >= n && (best < 0 || k_[i].n < k_[best].n)) best = i;
+    return best >= 0 && leave(best, b);
+  }
+  // Keeps b.  True when one is too many: the oldest leaves in `out`.
+  bool keep(const Block &b, Block &out) noexcept {
+    std::lock_guard<std::mutex> lk(m_);
+    const bool full = n_ == Max && leave(0, out);
+    k_[n_++] = b;
+    return full;
+  }
+  // Any kept block of dev leaves.
+  bool drop(int dev, Block &out) noexcept {
+    std::lock_guard<std::mutex> lk(m_);
+    for (int i = 0; i < n_; ++i)
+      if (k_[i].dev == dev) return leave(i, out);
+    return false;
+  }
+
+ private:
+  bool leave(int i, Block &out) noexcept {
+    out = k_[i];
+    --n_;
+    for (; i < n_; ++i) k_[i] = k_[i + 1];
+    return true;
+  }
+  std::mutex m_;
+  Block k_[Max];
+  int n_ = 0;
+};
+
 }  // namespace rai
 
 #endif

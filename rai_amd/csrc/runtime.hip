@@ -48,28 +48,23 @@ constexpr int kPoolBlocks = 4;
 constexpr size_t kPoolBlockBytes = size_t(32) << 20;
 
 struct PoolBlock {
-  void *p;
-  size_t n;
-  int dev;
+  void *p = nullptr;
+  size_t n = 0;
+  int dev = 0;
 };
-static std::mutex g_pool_mutex;
-static std::vector<PoolBlock> g_pool;
+static KeptBlocks<PoolBlock, kPoolBlocks> g_pool;
 
 // Frees the kept blocks of the current device; true when there were any.
 static bool pool_trim() {
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess) return false;
-  std::vector<void *> drop;
-  {
-    std::lock_guard<std::mutex> lk(g_pool_mutex);
-    for (size_t i = g_pool.size(); i-- > 0;)
-      if (g_pool[i].dev == dev) {
-        drop.push_back(g_pool[i].p);
-        g_pool.erase(g_pool.begin() + i);
-      }
+  PoolBlock b;
+  bool any = false;
+  while (g_pool.drop(dev, b)) {
+    (void)hipFree(b.p);
+    any = true;
   }
-  for (void *p : drop) (void)hipFree(p);
-  return !drop.empty();
+  return any;
 }
 
 static void *device_alloc(size_t n) {
@@ -92,18 +87,10 @@ class CallScratch {
     hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
     HIP_CHECK(hipStreamIsCapturing(s, &st));
     if (st != hipStreamCaptureStatusNone) HIP_CHECK(hipErrorStreamCaptureUnsupported);
-    HIP_CHECK(hipGetDevice(&b_.dev));
-    {
-      std::lock_guard<std::mutex> lk(g_pool_mutex);
-      int best = -1;  // the smallest kept block that fits
-      for (int i = 0; i < (int)g_pool.size(); ++i)
-        if (g_pool[i].dev == b_.dev && g_pool[i].n >= n && (best < 0 || g_pool[i].n < g_pool[best].n)) best = i;
-      if (best >= 0) {
-        b_ = g_pool[best];
-        g_pool.erase(g_pool.begin() + best);
-        return;
-      }
-    }
+    int dev = 0;
+    HIP_CHECK(hipGetDevice(&dev));
+    if (g_pool.take(n, dev, b_)) return;
+    b_.dev = dev;
     // Rounded up so that nearby sizes share a block.
     b_.n = std::max<size_t>((n + (size_t(1) << 20) - 1) & ~((size_t(1) << 20) - 1), size_t(1) << 20);
     b_.p = device_alloc(b_.n);
@@ -128,21 +115,15 @@ class CallScratch {
       (void)hipFree(b_.p);  // the work's state is unknown: never reused
       return;
     }
-    PoolBlock drop = b_;
-    if (b_.n <= kPoolBlockBytes) {
-      std::lock_guard<std::mutex> lk(g_pool_mutex);
-      g_pool.push_back(b_);
-      drop.p = nullptr;
-      if ((int)g_pool.size() > kPoolBlocks) {
-        drop = g_pool.front();
-        g_pool.erase(g_pool.begin());
-      }
-    }
-    if (drop.p) (void)hipFree(drop.p);
+    PoolBlock old;
+    if (b_.n > kPoolBlockBytes)
+      (void)hipFree(b_.p);
+    else if (g_pool.keep(b_, old))
+      (void)hipFree(old.p);
   }
 
  private:
-  PoolBlock b_{nullptr, 0, 0};
+  PoolBlock b_;
   hipStream_t s_;
   size_t used_ = 0;
   bool done_ = false;

@@ -73,6 +73,20 @@ void bounds() {
   expect(p.take(1, 0, b) == Take::kMake, "none is left");
 }
 
+void kept() {
+  static rai::KeptBlocks<Block, 3> k;
+  Block b, out;
+  static_assert(noexcept(k.keep(b, out)), "called from a destructor");
+  expect(!k.take(1, 0, b) && !k.drop(0, b), "nothing kept");
+  for (size_t n : {30, 10, 20}) expect(!k.keep(Block{nullptr, n, n == 20}, out), "room");
+  expect(k.take(5, 0, b) && b.n == 10, "the smallest that fits, of the device");
+  expect(!k.keep(b, out), "back");
+  expect(k.keep(Block{nullptr, 40, 0}, out) && out.n == 30, "the oldest leaves");
+  expect(!k.take(41, 0, b) && !k.take(1, 2, b), "none fits");
+  expect(k.take(11, 0, b) && b.n == 40 && k.drop(0, b) && b.n == 10 && !k.drop(0, b), "of the device only");
+  expect(k.take(20, 1, b) && b.n == 20 && !k.take(0, 1, b), "the other device's");
+}
+
 // Takers on several threads: a block is never two takers', and there are never
 // more than two.
 void threads() {
@@ -114,6 +128,7 @@ void threads() {
 int main() {
   copies();
   bounds();
+  kept();
   threads();
   if (!bad) std::printf("ok\n");
   return bad != 0;

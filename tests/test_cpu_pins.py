@@ -236,7 +236,8 @@ def test_streamed_weight_loads_stay_inside_their_arrays(tmp_path):
 @pytest.mark.parametrize("flags", [[], ["-fsanitize=thread", "-g"]])
 def test_copy_threads_and_block_pool(tmp_path, flags):
     """rai_amd/csrc/host_io.h: copies by several callers at once, and a pool that
-    never has more than its bound of blocks, also when one cannot be made."""
+    never has more than its bound of blocks, also when one cannot be made; the
+    calls made from destructors neither allocate nor throw."""
     exe = tmp_path / "host_io_check"
     subprocess.run(["g++", "-O1", "-std=c++17", "-pthread", *flags, "-I", os.path.join(ROOT, "rai_amd", "csrc"),
                     os.path.join(ROOT, "tests", "host_io_check.cpp"), "-o", str(exe)], check=True)
