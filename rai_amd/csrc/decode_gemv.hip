@@ -84,7 +84,7 @@ struct DecCfg {
 // LDS bytes of a block: activations (codes, scales, sums) and the waves'
 // product areas; with the fused RMSNorm the product areas double as the
 // norm's chain-major row scratch.
-__host__ __device__ inline int dec_act_bytes(int cols) { return (cols + 8 * (cols / 32) + 15) & ~15; }
+__host__ __device__ inline int dec_act_bytes(int cols) { return (cols + 8 * ((cols + 1023) / 1024 * 32) + 15) & ~15; }
 
 template <int GS, int R>
 size_t dec_smem(int cols, bool fused) {
@@ -192,10 +192,10 @@ __global__ __launch_bounds__(256) void k_w4a8_dec(float *out, const float *add, 
   const int nchunks = (units + kDecChunk - 1) / kDecChunk;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int h = lane >> 5, k = lane & 31;
-  // LDS: q [cols] bytes | scales [groups] | sums [groups] | waves' areas.
+  // LDS: q [cols] bytes | scales, sums [groups of whole chunks] | waves' areas.
   int8_t *qsh = reinterpret_cast<int8_t *>(smem);
   float *ash = reinterpret_cast<float *>(smem + cols);
-  float *ssh = ash + groups;
+  float *ssh = ash + nchunks * GPC;
   float *wbase = reinterpret_cast<float *>(smem + dec_act_bytes(cols));
   float *pw_lds = wbase + wave * C::WAVE_FLOATS;
   float *fin = pw_lds + 2 * C::BUF;
@@ -285,7 +285,7 @@ __global__ __launch_bounds__(256) void k_w4a8_dec(float *out, const float *add, 
     uint32_t vp = ((uint32_t)row * groups + un / LPG) * 4;
     // Past the last iteration, and on the lanes past the units of a
     // partial last chunk: zeros without a memory access.  Zero codes and
-    // parameters, with the zero scale and sum of read_act, give +0 or -0
+    // parameters, with the zero scale and sum staged for them, give +0 or -0
     // products, which leave a chain unchanged (a chain starts at +0 and a sum
     // of floats is -0 only when both terms are).
     if (lt >= tiles_per_wave || un >= units) {
@@ -331,6 +331,9 @@ __global__ __launch_bounds__(256) void k_w4a8_dec(float *out, const float *add, 
       ssh[min(tid + u * 256, groups - 1)] = sv[u];
     }
   }
+  // Groups past the row's, to the end of its last chunk: a zero scale and sum, so
+  // that their zero parameters meet no infinite or NaN factor.
+  if (tid < nchunks * GPC - groups) ash[groups + tid] = ssh[groups + tid] = 0.0f;
   __syncthreads();
 
   float acc = 0.0f, gate_v = 0.0f, up_v = 0.0f;
@@ -340,17 +343,16 @@ __global__ __launch_bounds__(256) void k_w4a8_dec(float *out, const float *add, 
   const int cbase = min(lane, NC * R - 1) * STR;
   // Group of the lane's unit in the chunk, and the unit's place in it.
   const int kg = k / LPG, ku = k % LPG;
-  // Activations of the iteration's chunk (read one iteration ahead).  Units
-  // past the row's: the last one's codes, with a zero scale and sum, so that
-  // their zero parameters meet no infinite or NaN factor.
+  // Activations of the iteration's chunk (read one iteration ahead); units past
+  // the row's take the last one's codes.
   uint4 q0, q1;
   float as, xsum;
   auto read_act = [&](int ch) {
-    const int uq = ch * kDecChunk + k, un = min(uq, units - 1);
+    const int un = min(ch * kDecChunk + k, units - 1);
     q0 = *reinterpret_cast<const uint4 *>(qsh + un * 32);
     q1 = *reinterpret_cast<const uint4 *>(qsh + un * 32 + 16);
-    as = uq < units ? ash[un / LPG] : 0.0f;
-    xsum = uq < units ? ssh[un / LPG] : 0.0f;
+    as = ash[ch * GPC + kg];
+    xsum = ssh[ch * GPC + kg];
   };
   // End of tile t: the row sums from the chain values in acc.
   auto finish = [&](int t) {
