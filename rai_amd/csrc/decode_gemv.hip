@@ -580,55 +580,28 @@ bool w4a8_dec_path(int rows, int cols, int gs) {
 
 bool w4a8_dec_fused_ok(int cols) { return cols / 32 <= 128; }
 
-// Tile height, ring depth and grid per shape, measured on the 7B decode
-// shapes (4096..32000 rows, K 4096 / 14336) with the weights streamed from
-// HBM: 4-row tiles with a 4-chunk ring, or 8-row tiles with a 3-chunk ring
-// where the fused RMSNorm prologue needs fewer blocks; a 512-block grid for
-// many rows, one tile per wave otherwise.
-static void dec_choice(int rows, bool fused, int &variant, int &blocks) {
-  if (!fused) {
-    variant = 4;
-    blocks = rows >= 16384 ? 512 : 0;
-  } else if (rows >= 16384) {
-    variant = 2;
-    blocks = 512;
-  } else if (rows >= 8192) {
-    variant = 4;
-    blocks = 512;
-  } else {
-    variant = rows > 4096 ? 2 : 4;
-    blocks = 0;
-  }
-}
-
 bool launch_w4a8_dec(float *out, const float *add, const uint8_t *nib, const uint8_t *params, const int8_t *q_split,
                      const float *scales, const float *sums, int rows, int cols, int gs, const float *nx,
-                     const float *nw, float eps, hipStream_t s, int variant, int blocks) {
+                     const float *nw, float eps, hipStream_t s) {
   if (!w4a8_dec_path(rows, cols, gs)) return false;
   if (nx && !w4a8_dec_fused_ok(cols)) return false;
-  // Groups of 64 and 128 (nine chains a row): four-row tiles, a ring of four
-  // chunks, one tile per wave up to 16384 rows.  Against the tiled VALU
+  // Four-row tiles with a ring of four chunks, one tile per wave (blocks = 0) up to
+  // 16384 rows and 512 blocks from there on.  Group 32 with the fused norm, whose
+  // prologue every block repeats: 512 blocks from 8192 rows, and eight-row tiles
+  // with a ring of three between 4096 and 8192 rows and from 16384.  Measured on
+  // the 7B decode shapes (4096..32000 rows, K 4096 / 14336) with the weights
+  // streamed from HBM.  Groups of 64 and 128 (nine chains a row) against the tiled VALU
   // kernel they took before (with the norm and quantization launches of their
-  // own): a 4096-wide layer and head at group 128, 1000 positions, 211 -> 170
-  // us.
-  if (gs != 32) {
-    if (blocks == 0 && rows >= 16384) blocks = 512;
-    if (gs == 64)
-      launch_dec_rd<64, 4, 4>(out, add, nib, params, q_split, scales, sums, rows, cols, nx, nw, eps, blocks, s);
-    else
-      launch_dec_rd<128, 4, 4>(out, add, nib, params, q_split, scales, sums, rows, cols, nx, nw, eps, blocks, s);
-    return true;
-  }
-  if (variant == 0) dec_choice(rows, nw != nullptr, variant, blocks);
-  switch (variant) {
-    case 1: launch_dec_rd<32, 4, 6>(out, add, nib, params, q_split, scales, sums, rows, cols, nx, nw, eps, blocks, s); break;
-    case 2: launch_dec_rd<32, 8, 3>(out, add, nib, params, q_split, scales, sums, rows, cols, nx, nw, eps, blocks, s); break;
-    case 3: launch_dec_rd<32, 12, 2>(out, add, nib, params, q_split, scales, sums, rows, cols, nx, nw, eps, blocks, s); break;
-    case 4: launch_dec_rd<32, 4, 4>(out, add, nib, params, q_split, scales, sums, rows, cols, nx, nw, eps, blocks, s); break;
-    case 5: launch_dec_rd<32, 8, 4>(out, add, nib, params, q_split, scales, sums, rows, cols, nx, nw, eps, blocks, s); break;
-    case 6: launch_dec_rd<32, 12, 3>(out, add, nib, params, q_split, scales, sums, rows, cols, nx, nw, eps, blocks, s); break;
-    default: launch_dec_rd<32, 8, 3>(out, add, nib, params, q_split, scales, sums, rows, cols, nx, nw, eps, blocks, s); break;
-  }
+  // own): a 4096-wide layer and head at group 128, 1000 positions, 211 -> 170 us.
+  const int blocks = rows >= (gs == 32 && nw ? 8192 : 16384) ? 512 : 0;
+  if (gs == 64)
+    launch_dec_rd<64, 4, 4>(out, add, nib, params, q_split, scales, sums, rows, cols, nx, nw, eps, blocks, s);
+  else if (gs == 128)
+    launch_dec_rd<128, 4, 4>(out, add, nib, params, q_split, scales, sums, rows, cols, nx, nw, eps, blocks, s);
+  else if (nw && (rows >= 16384 || (rows > 4096 && rows < 8192)))
+    launch_dec_t<32, 8, 3, 0>(out, add, nib, params, q_split, scales, sums, rows, cols, nx, nw, eps, blocks, s);
+  else
+    launch_dec_rd<32, 4, 4>(out, add, nib, params, q_split, scales, sums, rows, cols, nx, nw, eps, blocks, s);
   return true;
 }
 
