@@ -518,12 +518,7 @@ void launch_dec_t(float *out, const float *add, const uint8_t *nib, const uint8_
                   const float *scales, const float *sums, int rows, int cols, const float *nx, const float *nw,
                   float eps, int blocks, hipStream_t s) {
   const size_t smem = dec_smem<GS, R>(cols, ST == 0);  // the norm's row scratch
-  static size_t configured = 0;
-  if (smem > configured) {
-    (void)hipFuncSetAttribute(reinterpret_cast<const void *>(&k_w4a8_dec<GS, R, D, ST, kEpiPlain>),
-                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
-    configured = smem;
-  }
+  dynamic_lds<&k_w4a8_dec<GS, R, D, ST, kEpiPlain>>(smem);
   const int tiles = (rows + R - 1) / R;
   if (blocks <= 0) blocks = (tiles + kDecWaves - 1) / kDecWaves;
   blocks = std::max(1, std::min(blocks, 1024));
@@ -553,12 +548,7 @@ template <int GS, int R, int D, int ST>
 void launch_dec_moe_t(float *out, const DecMoe &moe, const int8_t *q_split, const float *scales, const float *sums,
                       int rows, int cols, int blocks, int entries, hipStream_t s) {
   const size_t smem = dec_smem<GS, R>(cols, false);
-  static size_t configured = 0;
-  if (smem > configured) {
-    (void)hipFuncSetAttribute(reinterpret_cast<const void *>(&k_w4a8_dec<GS, R, D, ST, kEpiMoe>),
-                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
-    configured = smem;
-  }
+  dynamic_lds<&k_w4a8_dec<GS, R, D, ST, kEpiMoe>>(smem);
   const int tiles = (rows + R - 1) / R, waves = blocks * kDecWaves;
   const int per_wave = (tiles + waves - 1) / waves;
   hipLaunchKernelGGL((k_w4a8_dec<GS, R, D, ST, kEpiMoe>), dim3(blocks, entries), dim3(256), smem, s, out, nullptr,
@@ -618,12 +608,7 @@ bool launch_w4a8_dec_multi(const DecMulti &mp, int n, int cols, int gs, const fl
   auto go = [&](auto g) {
     constexpr int GS = decltype(g)::value, R = 4;
     const size_t smem = dec_smem<GS, R>(cols, false);
-    static size_t configured = 0;
-    if (smem > configured) {
-      (void)hipFuncSetAttribute(reinterpret_cast<const void *>(&k_w4a8_dec<GS, R, 4, 8, kEpiMulti>),
-                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
-      configured = smem;
-    }
+    dynamic_lds<&k_w4a8_dec<GS, R, 4, 8, kEpiMulti>>(smem);
     const int tiles = (rows + R - 1) / R;
     const int full = (tiles + kDecWaves - 1) / kDecWaves, blocks = rows >= 16384 ? 512 : std::min(full, 1024);
     const int per_wave = (tiles + blocks * kDecWaves - 1) / (blocks * kDecWaves);
@@ -685,12 +670,7 @@ bool launch_w4a8_dec_moe_glu(const DecMoe &moe, const int8_t *q_split, const flo
   const size_t smem = dec_smem<32, 8>(cols, false);
   auto go = [&](auto st) {
     constexpr int ST = decltype(st)::value;
-    static size_t configured = 0;
-    if (smem > configured) {
-      (void)hipFuncSetAttribute(reinterpret_cast<const void *>(&k_w4a8_dec<32, 8, 2, ST, kEpiMoeGlu>),
-                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
-      configured = smem;
-    }
+    dynamic_lds<&k_w4a8_dec<32, 8, 2, ST, kEpiMoeGlu>>(smem);
     hipLaunchKernelGGL((k_w4a8_dec<32, 8, 2, ST, kEpiMoeGlu>), dim3(rows / 64, max_entries), dim3(256), smem, s,
                        nullptr, nullptr, nullptr, nullptr, q_split, scales, sums, rows, cols, 2, nullptr, nullptr,
                        0.0f, DecNone{}, moe, DecNone{});
@@ -712,12 +692,7 @@ bool launch_w4a8_glu1(const uint8_t *nib, const uint8_t *params, const float *x,
                       int rows, int cols, int gs, int8_t *q_out, float *scale_out, float *sum_out, hipStream_t s) {
   if (gs != 32 || !w4a8_dec_path(rows, cols, gs) || !w4a8_dec_fused_ok(cols) || rows % 64 != 0) return false;
   const size_t smem = dec_smem<32, 8>(cols, true);
-  static size_t configured = 0;
-  if (smem > configured) {
-    (void)hipFuncSetAttribute(reinterpret_cast<const void *>(&k_w4a8_dec<32, 8, 2, 0, kEpiGlu>),
-                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
-    configured = smem;
-  }
+  dynamic_lds<&k_w4a8_dec<32, 8, 2, 0, kEpiGlu>>(smem);
   hipLaunchKernelGGL((k_w4a8_dec<32, 8, 2, 0, kEpiGlu>), dim3(rows / 64), dim3(256), smem, s, nullptr, nullptr, nib,
                      params, q_out, scale_out, sum_out, rows, cols, 2, x, norm_w, eps, DecNone{}, DecNone{}, DecNone{});
   return true;
@@ -731,12 +706,7 @@ bool launch_w4a8_qkv_rope1(float *out, const uint8_t *nib, const uint8_t *params
   auto go = [&](auto g, auto r) {
     constexpr int GS = decltype(g)::value, R = decltype(r)::value;
     const size_t smem = dec_smem<GS, R>(cols, true);
-    static size_t configured = 0;
-    if (smem > configured) {
-      (void)hipFuncSetAttribute(reinterpret_cast<const void *>(&k_w4a8_dec<GS, R, 2, 0, kEpiRope>),
-                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
-      configured = smem;
-    }
+    dynamic_lds<&k_w4a8_dec<GS, R, 2, 0, kEpiRope>>(smem);
     const int tiles = rows / R, blocks = (tiles + kDecWaves - 1) / kDecWaves;
     hipLaunchKernelGGL((k_w4a8_dec<GS, R, 2, 0, kEpiRope>), dim3(blocks), dim3(256), smem, s, out, nullptr, nib,
                        params, nullptr, nullptr, nullptr, rows, cols, 1, x, norm_w, eps, rope, DecNone{}, DecNone{});

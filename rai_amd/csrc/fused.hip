@@ -523,12 +523,7 @@ void launch_scores_mt(hipStream_t s, const float *q, int q_ld, const float *kc, 
   const int ntiles = (nmax + kScoreTile - 1) / kScoreTile;
   const int ns = std::max(1, std::min(ntiles, 256 / (nkv * nz)));
   const size_t smem = sizeof(float) * (2 * (size_t)kScoreTile * (HD + 4) + (size_t)G * mb * HD);
-  static bool configured = false;
-  if (!configured) {
-    (void)hipFuncSetAttribute(reinterpret_cast<const void *>(&k_scores_mt<HD, 8>),
-                              hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
-    configured = true;
-  }
+  dynamic_lds<&k_scores_mt<HD, 8>>(160 * 1024);
   hipLaunchKernelGGL((k_scores_mt<HD, 8>), dim3(ns, nkv, nz), dim3(512), smem, s, q, q_ld, kc, cap, p0, m, nh, nkv,
                      scale, scores, sstride, st, mb, ns);
 }
@@ -537,13 +532,7 @@ template <int HD, int PB>
 void launch_scores_t(dim3 sg, size_t ksm, hipStream_t s, const float *q, int q_ld, const float *kc, int cap, int p0,
                      int m, int nh, int nkv, float scale, float *scores, int sstride, const int *st, int toff,
                      int mb) {
-  static bool configured = false;
-  if (!configured) {
-    (void)hipFuncSetAttribute(reinterpret_cast<const void *>(&k_scores<HD, PB>),
-                              hipFuncAttributeMaxDynamicSharedMemorySize,
-                              (int)(sizeof(float) * ((size_t)kScoreTile * (HD + 4) + 16384)));
-    configured = true;
-  }
+  dynamic_lds<&k_scores<HD, PB>>(sizeof(float) * ((size_t)kScoreTile * (HD + 4) + 16384));
   hipLaunchKernelGGL((k_scores<HD, PB>), sg, dim3(256), ksm, s, q, q_ld, kc, cap, p0, m, nh, nkv, HD, scale, scores,
                      sstride, st, toff, mb);
 }
@@ -574,7 +563,6 @@ void launch_scores_hd(dim3 sg, size_t ksm, int npw, hipStream_t s, const float *
 // whose query rows fit next to the keys in LDS (at most 64 KB of them).
 void launch_scores(const float *q, int q_ld, const float *kc, int cap, int p0, int m, int nh, int nkv, int hd,
                    float scale, float *scores, int sstride, int nmax, const int *st, hipStream_t s) {
-  static size_t sc_configured = 0;
   const int G = nh / nkv;
   if (hd == 128 || hd == 64) {
     // Groups of mb tokens (their query rows next to the keys in LDS, at
@@ -604,11 +592,7 @@ void launch_scores(const float *q, int q_ld, const float *kc, int cap, int p0, i
   }
   const dim3 sg((nmax + kScoreTile - 1) / kScoreTile, nkv);
   const size_t ksm = sizeof(float) * (size_t)kScoreTile * (hd + 1);
-  if (ksm > 48 * 1024 && ksm > sc_configured) {
-    (void)hipFuncSetAttribute(reinterpret_cast<const void *>(&k_scores<0, 1>),
-                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)ksm);
-    sc_configured = ksm;
-  }
+  if (ksm > 48 * 1024) dynamic_lds<&k_scores<0, 1>>(ksm);
   hipLaunchKernelGGL((k_scores<0, 1>), sg, dim3(256), ksm, s, q, q_ld, kc, cap, p0, m, nh, nkv, hd, scale, scores,
                      sstride, st, 0, m);
 }
@@ -1005,12 +989,7 @@ __global__ __launch_bounds__(64 * RPB) void k_softmax_w(float *__restrict__ S, i
 template <int NBW, int RPB>
 void launch_softmax_w(float *scores, int p0, int m, int nh, int sstride, const int *st, hipStream_t s) {
   constexpr size_t smem = sizeof(float) * RPB * 8 * (8 * kSoftSeg + 4);
-  static bool configured = false;
-  if (!configured) {
-    (void)hipFuncSetAttribute(reinterpret_cast<const void *>(&k_softmax_w<NBW, RPB>),
-                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
-    configured = true;
-  }
+  dynamic_lds<&k_softmax_w<NBW, RPB>>(smem);
   hipLaunchKernelGGL((k_softmax_w<NBW, RPB>), dim3((m * nh + RPB - 1) / RPB), dim3(64 * RPB), smem, s, scores, p0, m,
                      nh, sstride, st);
 }
@@ -1636,12 +1615,7 @@ void launch_norm_quant_t(const float *x, const float *w, float *normed, int m, i
     }
   }
   const size_t smem = (GS > 0 ? 1 : 2) * sizeof(float) * (size_t)n;
-  static size_t configured = 0;
-  if (smem > 48 * 1024 && smem > configured) {
-    (void)hipFuncSetAttribute(reinterpret_cast<const void *>(&k_norm_quant<GS>),
-                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
-    configured = smem;
-  }
+  if (smem > 48 * 1024) dynamic_lds<&k_norm_quant<GS>>(smem);
   hipLaunchKernelGGL(k_norm_quant<GS>, dim3(m), dim3(256), smem, s, x, w, normed, q_split, q_nat,
                      scales, sums, n, eps, qa);
 }

@@ -441,12 +441,7 @@ template <int TGW, int WPB, int MAXQ, bool TMP, int NQ = kRpRing>
 void launch_rp(float *out, const float *add, const uint8_t *nib, const uint8_t *params, const int8_t *q_split,
                const float *scales, const float *sums, int rows, int cols, int m, int ntg, hipStream_t s) {
   constexpr size_t kStepBytes = 68 * 16 + 2 * 4 * 16;  // A blocks, scales, sums of one (group, step)
-  static bool configured = false;
-  if (!configured) {
-    (void)hipFuncSetAttribute(reinterpret_cast<const void *>(&k_gemv_rp<TGW, NQ, WPB, MAXQ, TMP>),
-                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)(TGW * MAXQ * kStepBytes));
-    configured = true;
-  }
+  dynamic_lds<&k_gemv_rp<TGW, NQ, WPB, MAXQ, TMP>>(TGW * MAXQ * kStepBytes);
   const size_t smem = TGW * (size_t)(cols / 128) * kStepBytes;
   const dim3 grid((rows + 16 * WPB - 1) / (16 * WPB), (ntg + TGW - 1) / TGW);
   hipLaunchKernelGGL((k_gemv_rp<TGW, NQ, WPB, MAXQ, TMP>), grid, dim3(64 * WPB), smem, s, out, add, nib, params,

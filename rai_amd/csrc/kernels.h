@@ -8,7 +8,18 @@
 #include <cstddef>
 #include <cstdint>
 
+#include "raised_limit.h"
+
 namespace rai {
+
+// Lets kernel K be launched with n bytes of dynamic LDS.
+template <auto K>
+inline void dynamic_lds(size_t n) {
+  static RaisedLimit limit;
+  limit.raise(n, [](size_t b) {
+    (void)hipFuncSetAttribute(reinterpret_cast<const void *>(K), hipFuncAttributeMaxDynamicSharedMemorySize, (int)b);
+  });
+}
 
 // Per-token activation quantization of gemm.rs:147-374 for K-column rows:
 // q_nat [m][K] int8 in natural column order; q_split [m][K] int8 in

@@ -317,12 +317,7 @@ void launch_fast_t(float *out, const float *add, const uint8_t *nib, const uint8
                    const float *scales, const float *sums, int rows, int cols, int m, int groups,
                    hipStream_t s) {
   const size_t smem = fast_smem<GS, MT>();
-  static bool configured = false;
-  if (!configured) {
-    (void)hipFuncSetAttribute(reinterpret_cast<const void *>(&k_w4a8_fast<GS, MT>),
-                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
-    configured = true;
-  }
+  dynamic_lds<&k_w4a8_fast<GS, MT>>(smem);
   dim3 grid((rows + kRows - 1) / kRows, (m + MT - 1) / MT);
   hipLaunchKernelGGL((k_w4a8_fast<GS, MT>), grid, dim3(kThreads), smem, s, out, add, nib, params,
                      q_split, scales, sums, rows, cols, m, groups);
@@ -586,12 +581,7 @@ void launch_small_t(float *out, const float *add, const uint8_t *nib, const uint
                     const float *scales, const float *sums, int rows, int cols, int m, int groups,
                     hipStream_t s, const float *nx = nullptr, const float *nw = nullptr, float eps = 0.0f) {
   const size_t smem = small_smem<GS, MT, R, PD, WHOLE>(groups, std::min(m, MT), nx ? cols : 0);
-  static size_t configured = 0;
-  if (smem > configured) {
-    (void)hipFuncSetAttribute(reinterpret_cast<const void *>(&k_w4a8_small<GS, MT, R, PD, WHOLE>),
-                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
-    configured = smem;
-  }
+  dynamic_lds<&k_w4a8_small<GS, MT, R, PD, WHOLE>>(smem);
   dim3 grid((rows + R - 1) / R, (m + MT - 1) / MT);
   hipLaunchKernelGGL((k_w4a8_small<GS, MT, R, PD, WHOLE>), grid, dim3(kThreads), smem, s, out, add,
                      nib, params, q_split, scales, sums, rows, cols, m, groups, nx, nw, eps);
@@ -719,12 +709,7 @@ void launch_m1_t(float *out, const float *add, const uint8_t *nib, const uint8_t
   // With a fused RMSNorm the products area doubles as the row scratch.
   const size_t prod = std::max(4 * (size_t)NC * R * (groups + 1), nx ? 4 * (size_t)rms_scratch_floats(cols) : 0);
   const size_t smem = (size_t)((cols + 15) & ~15) + 4 * (size_t)((2 * groups + 3) & ~3) + prod;
-  static size_t configured = 0;
-  if (smem > configured) {
-    (void)hipFuncSetAttribute(reinterpret_cast<const void *>(&k_w4a8_m1<GS, R, IPT>),
-                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
-    configured = smem;
-  }
+  dynamic_lds<&k_w4a8_m1<GS, R, IPT>>(smem);
   hipLaunchKernelGGL((k_w4a8_m1<GS, R, IPT>), dim3((rows + R - 1) / R), dim3(kThreads), smem, s,
                      out, add, nib, params, q_split, scales, sums, rows, cols, groups, nx, nw, eps);
 }

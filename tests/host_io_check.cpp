@@ -1,9 +1,10 @@
 // Host check of rai_amd/csrc/host_io.h: the copy threads (several callers at
 // once, sizes around their blocks) and the bounded block pool (takers past its
-// bound, blocks that could not be made, blocks that grow).  Prints "ok", or what
-// is wrong.  Built (also under a thread sanitizer) and run by
+// bound, blocks that could not be made, blocks that grow); and of
+// raised_limit.h.  Prints "ok", or what is wrong.  Built (also under a thread sanitizer) and run by
 // tests/test_cpu_pins.py (test infrastructure only).
 #include "host_io.h"
+#include "raised_limit.h"
 
 #include <cstdio>
 #include <cstdlib>
@@ -123,6 +124,29 @@ void threads() {
   expect(most <= 2, "blocks at once");
 }
 
+// Callers that raise a limit past each other: it never falls, and holds for each
+// when its call returns.
+void limits() {
+  for (int it = 0; it < 200; ++it) {
+    rai::RaisedLimit l;
+    std::atomic<size_t> set{0};
+    std::atomic<int> low{0}, fell{0};
+    std::vector<std::thread> ts;
+    for (size_t t = 0; t < 4; ++t)
+      ts.emplace_back([&, t] {
+        for (size_t i = 0; i < 8; ++i) {
+          const size_t n = 1 + (3 * i + 5 * t) % 16;
+          l.raise(n, [&](size_t b) {
+            if (set.exchange(b) >= b) ++fell;
+          });
+          if (set < n) ++low;
+        }
+      });
+    for (auto &t : ts) t.join();
+    expect(low == 0 && fell == 0, "a limit raised on several threads");
+  }
+}
+
 }  // namespace
 
 int main() {
@@ -130,6 +154,7 @@ int main() {
   bounds();
   kept();
   threads();
+  limits();
   if (!bad) std::printf("ok\n");
   return bad != 0;
 }

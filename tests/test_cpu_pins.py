@@ -237,7 +237,8 @@ def test_streamed_weight_loads_stay_inside_their_arrays(tmp_path):
 def test_copy_threads_and_block_pool(tmp_path, flags):
     """rai_amd/csrc/host_io.h: copies by several callers at once, and a pool that
     never has more than its bound of blocks, also when one cannot be made; the
-    calls made from destructors neither allocate nor throw."""
+    calls made from destructors neither allocate nor throw.  raised_limit.h: a
+    limit that several callers raise at once."""
     exe = tmp_path / "host_io_check"
     subprocess.run(["g++", "-O1", "-std=c++17", "-pthread", *flags, "-I", os.path.join(ROOT, "rai_amd", "csrc"),
                     os.path.join(ROOT, "tests", "host_io_check.cpp"), "-o", str(exe)], check=True)
