@@ -61,6 +61,7 @@
 #include <type_traits>
 
 #include "kernels.h"
+#include "quant_dev.h"
 
 namespace rai {
 
@@ -68,7 +69,6 @@ namespace {
 
 typedef _Float16 h8 __attribute__((ext_vector_type(8)));
 typedef _Float16 h4 __attribute__((ext_vector_type(4)));
-typedef _Float16 h2 __attribute__((ext_vector_type(2)));
 typedef float f16v __attribute__((ext_vector_type(16)));
 typedef float f32v __attribute__((ext_vector_type(32)));
 typedef uint32_t u4v __attribute__((ext_vector_type(4)));
@@ -175,27 +175,6 @@ __global__ __launch_bounds__(256) void k_mm_pack(const int8_t *__restrict__ q_sp
   }
 }
 
-// The B operand of block dword w for half h (sh = 8 h): the codes as f16
-// subnormals (SUB), or as 1024 + n minus 1024.
-template <bool SUB>
-__device__ __forceinline__ h4 unpack_half(uint32_t w, uint32_t sh) {
-  const uint32_t t = w >> sh;
-  if constexpr (SUB) {
-    typedef uint32_t u2 __attribute__((ext_vector_type(2)));
-    const u2 d = {t & 0x000F000Fu, t & 0x00F000F0u};
-    return __builtin_bit_cast(h4, d);
-  }
-  const h2 bias = {(_Float16)1024.0f, (_Float16)1024.0f};
-  const h2 e0 = __builtin_bit_cast(h2, (t & 0x000F000Fu) | 0x64006400u) - bias;
-  const h2 e1 = __builtin_bit_cast(h2, (t & 0x00F000F0u) | 0x64006400u) - bias;
-  h4 r;
-  r[0] = e0[0];
-  r[1] = e0[1];
-  r[2] = e1[0];
-  r[3] = e1[1];
-  return r;
-}
-
 // The reference lanes' sums D = A_l x B_l of one group.
 template <int GS, bool SUB>
 __device__ __forceinline__ f16v mm_lane_sums(const uint8_t *rc, const u4v (&wq)[MmCfg<GS>::NU], int b, uint32_t sh,
@@ -203,13 +182,13 @@ __device__ __forceinline__ f16v mm_lane_sums(const uint8_t *rc, const u4v (&wq)[
   const f16v zero = {};
   if constexpr (GS == 128) {
     const uint32_t w = wq[b >> 2][b & 3];
-    const h4 lo = unpack_half<SUB>(w, 0), hi = unpack_half<SUB>(w, 8);
+    const h4 lo = codes_half<SUB>(w), hi = codes_half<SUB>(w >> 8);
     const h8 bq = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
     return __builtin_amdgcn_mfma_f32_32x32x16_f16(*reinterpret_cast<const h8 *>(rc + b * 1024 + lane * 16), bq, zero,
                                                   0, 0, 0);
   } else {
     return __builtin_amdgcn_mfma_f32_32x32x8f16(*reinterpret_cast<const h4 *>(rc + b * 512 + lane * 8),
-                                                unpack_half<SUB>(wq[b >> 2][b & 3], sh), zero, 0, 0, 0);
+                                                codes_half<SUB>(wq[b >> 2][b & 3] >> sh), zero, 0, 0, 0);
   }
 }
 

@@ -47,6 +47,7 @@
 #include <type_traits>
 
 #include "kernels.h"
+#include "quant_dev.h"
 #include "stream_addr.h"
 
 namespace rai {
@@ -55,7 +56,6 @@ namespace {
 
 typedef _Float16 h8 __attribute__((ext_vector_type(8)));
 typedef _Float16 h4 __attribute__((ext_vector_type(4)));
-typedef _Float16 h2 __attribute__((ext_vector_type(2)));
 typedef float f16v __attribute__((ext_vector_type(16)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
@@ -79,20 +79,6 @@ struct StreamCfg {
   static_assert(4 * D % NQ == 0, "static ring slots");
   static constexpr int TILE_UNITS = 64 * U;          // LDS units of a row tile's stage
 };
-
-// A block dword's codes, columns (0, 4, 1, 5) and (2, 6, 3, 7), the odd ones
-// at 16 times their value: f16 subnormals (SUB) or exact integers.
-template <bool SUB>
-__device__ __forceinline__ h4 codes_half(uint32_t t) {
-  if constexpr (SUB) {
-    const u32x2 d = {t & 0x000F000Fu, t & 0x00F000F0u};
-    return __builtin_bit_cast(h4, d);
-  }
-  const h2 bias = {(_Float16)1024.0f, (_Float16)1024.0f};
-  const h2 e0 = __builtin_bit_cast(h2, (t & 0x000F000Fu) | 0x64006400u) - bias;
-  const h2 e1 = __builtin_bit_cast(h2, (t & 0x00F000F0u) | 0x64006400u) - bias;
-  return h4{e0[0], e0[1], e1[0], e1[1]};
-}
 
 template <int GS, int CW>
 __global__ __launch_bounds__(256, 2) void k_gemv_stream(float *out, const float *add, const uint8_t *__restrict__ nib,

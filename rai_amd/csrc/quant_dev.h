@@ -19,16 +19,24 @@ __device__ __forceinline__ int split_col(int c) {
   return (c & ~7) + ((j & 1) ? 4 + (j >> 1) : (j >> 1));
 }
 
-// Quantize one group held by 8 consecutive lanes (lane j owns the columns
-// 8c + j, c = 0..NB-1, of the group) exactly as quantize_input_split_avx2
-// and compute_input_sums do (gemm.rs:182-212, 280-374):
-//   sum   = ((a0+a4)+(a1+a5))+((a2+a6)+(a3+a7)), a_j = sequential sum of the
-//           lane's values in column order;
-//   scale = absmax/127 (1 when absmax <= 1e-10); q = clamp(rne(v/scale)).
-// qs_grp / qn_grp point at the group's first byte in the block-split and
-// natural layouts (qn_grp may be null; either may be in LDS).
-// All 64 lanes of the wave must call this together.
-// Lanes with ok == false take part in the shuffles and store nothing.
+// The B operand of a block dword's codes in columns (0, 4, 1, 5) - of the dword
+// shifted by 8: (2, 6, 3, 7) - the odd ones at 16 times their value: f16 subnormals
+// (SUB: one mask a pair), or exact integers as 1024 + n minus 1024.
+typedef _Float16 codes4 __attribute__((ext_vector_type(4)));
+template <bool SUB>
+__device__ __forceinline__ codes4 codes_half(uint32_t t) {
+  if constexpr (SUB) {
+    typedef uint32_t u2 __attribute__((ext_vector_type(2)));
+    const u2 d = {t & 0x000F000Fu, t & 0x00F000F0u};
+    return __builtin_bit_cast(codes4, d);
+  }
+  typedef _Float16 h2 __attribute__((ext_vector_type(2)));
+  const h2 bias = {(_Float16)1024.0f, (_Float16)1024.0f};
+  const h2 e0 = __builtin_bit_cast(h2, (t & 0x000F000Fu) | 0x64006400u) - bias;
+  const h2 e1 = __builtin_bit_cast(h2, (t & 0x00F000F0u) | 0x64006400u) - bias;
+  return codes4{e0[0], e0[1], e1[0], e1[1]};
+}
+
 // Place of (token t, group g) in the activations of k_gemv_stream
 // (gemv_stream.hip): record [t / 16][g / 4] holds, in lane order
 // 16 (g % 4) + t % 16, GS / 8 blocks of eight f16, then the scale and the
@@ -60,6 +68,16 @@ __device__ __forceinline__ float dpp_mov(float v) {
 constexpr int kDppShl1 = 0x101, kDppShl2 = 0x102, kDppShl4 = 0x104, kDppHalfMirror = 0x141, kDppXor1 = 0xB1,
               kDppXor2 = 0x4E;
 
+// Quantize one group held by 8 consecutive lanes (lane j owns the columns
+// 8c + j, c = 0..NB-1, of the group) exactly as quantize_input_split_avx2
+// and compute_input_sums do (gemm.rs:182-212, 280-374):
+//   sum   = ((a0+a4)+(a1+a5))+((a2+a6)+(a3+a7)), a_j = sequential sum of the
+//           lane's values in column order;
+//   scale = absmax/127 (1 when absmax <= 1e-10); q = clamp(rne(v/scale)).
+// qs_grp / qn_grp point at the group's first byte in the block-split and
+// natural layouts (qn_grp may be null; either may be in LDS).
+// All 64 lanes of the wave must call this together.
+// Lanes with ok == false take part in the shuffles and store nothing.
 template <int NB>
 __device__ __forceinline__ void quantize_group8_to(const float (&v)[NB], int j, bool ok, int8_t *qs_grp,
                                                    int8_t *qn_grp, float *scale_out, float *sum_out,
