@@ -134,7 +134,7 @@ int rai_device_info(char *name, size_t name_len, int *compute_units);
  * 128, or a larger bound for group-32 models with K > 4096.  Device memory:
  * the file's bytes, RoPE tables, and for group-32 dense matrices a second
  * copy of their scale/zero parameters in 16-row tiles (about a fifth of the
- * quantized weight bytes), which the 2..24-token GEMVs read. */
+ * quantized weight bytes), which the 2..64-token GEMVs read. */
 int rai_model_open(const char *path, int max_groups, rai_model **out);
 /* Same, from a caller-owned in-memory .raimodel image (copied). */
 int rai_model_from_buffer(const void *data, size_t len, int max_groups, rai_model **out);
@@ -145,7 +145,9 @@ int rai_model_weight_bytes(const rai_model *model, uint64_t *out);
 
 /* --------------------------------------------------------------- KV cache -- */
 /* RaiModel::create_kv_cache (model.rs:350) / KVCache::new (kv_cache.rs:232).
- * f32 [layer][kv_head][max_ctx][head_dim] in HBM, allocated up front. */
+ * f32 [layer][kv_head][max_ctx][head_dim] in HBM, allocated up front.  The
+ * model's own passes over it keep the attention scores of 256 tokens, 256 *
+ * heads * max_ctx floats of the largest cache seen. */
 int rai_kv_create(rai_model *model, size_t max_ctx, rai_kv **out);
 void rai_kv_free(rai_kv *kv);
 /* KVCache::truncate (kv_cache.rs:300-304): filled = min(filled, len). */
@@ -305,7 +307,9 @@ int rai_spec_step(rai_spec *dec, size_t pos, uint32_t last_token, const rai_spec
  * *found = 0 when there is no match. */
 int rai_find_ngram_draft(const uint32_t *tokens, size_t len, size_t min_ngram, size_t max_ngram,
                          size_t max_draft, rai_lookup_match *out, int *found);
-/* LookupDecoder::new (lookup.rs:192-212). */
+/* LookupDecoder::new (lookup.rs:192-212).  Besides its KV cache and the
+ * activations of 1024 tokens, a decoder holds the attention scores of 256
+ * tokens, 256 * heads * max_ctx floats (32 heads, 32768 positions: 1.07 GB). */
 int rai_lookup_create(rai_model *model, size_t max_ctx, rai_lookup **out);
 void rai_lookup_free(rai_lookup *dec);
 /* The decoder's generator for exact sampling: rand::rngs::StdRng::

@@ -303,6 +303,9 @@ class HostStage {
   PinBlock b_;
 };
 
+// Largest verify batch: 63 drafts and the token before them.
+constexpr int kStepTokens = 64;
+
 // Tokens up to which a sparse layer runs entry by entry.
 constexpr int kMoeEntryTokens = 64;
 
@@ -329,7 +332,7 @@ struct DLinear {
   int rows = 0, cols = 0, gs = 0;
   const uint8_t *nib = nullptr, *params = nullptr;
   // The parameters again in 16-row tiles (launch_params_tile16), read by
-  // the matrix-core GEMV of 2..64 tokens; null where that does not apply.
+  // k_gemv_rp (2..64 tokens); null where that does not apply.
   const uint8_t *params_tiled = nullptr;
 };
 
@@ -1164,9 +1167,9 @@ struct rai_lookup {
   // position in the device step record.
   DevBuf step;            // int[5] {pos0, len, start, nd, temperature bits}
   bool graphs = false;
-  // Indexed by verify size m, plus (kAttnTokens + 1) times the mode (0
+  // Indexed by verify size m, plus (kStepTokens + 1) times the mode (0
   // greedy, 1 exact-sampling lookup, 2 the plain sampler), plus
-  // 3 (kAttnTokens + 1) per attention span index.
+  // 3 (kStepTokens + 1) per attention span index.
   std::vector<hipGraphExec_t> graph;
   std::vector<int> graph_uses;
   // Exact sampling: the decoder's StdRng (device), per-row probabilities
@@ -1294,7 +1297,7 @@ static void lookup_step(rai_lookup &d, size_t pos, const uint32_t *context, size
                       (int)cfg.max_draft, (int)d.max_ctx, res + 4, res, s, st);
   };
   HIP_CHECK(hipGetLastError());  // nothing pending from earlier launches
-  if (d.graphs && m <= kAttnTokens) {
+  if (d.graphs && m <= kStepTokens) {
     int *sh = d.pin + 512;
     sh[0] = (int)pos;
     sh[1] = (int)len;
@@ -1311,7 +1314,7 @@ static void lookup_step(rai_lookup &d, size_t pos, const uint32_t *context, size
     HIP_CHECK(hipMemcpyAsync(d.step.p, sh, 11 * sizeof(int), hipMemcpyHostToDevice, s));
     const int *st = d.step.as<int>();
     const int mode = plain ? 2 : sampled ? 1 : 0;
-    const int gi = m + (kAttnTokens + 1) * mode + 3 * (kAttnTokens + 1) * attn_span_index((int)pos + m);
+    const int gi = m + (kStepTokens + 1) * mode + 3 * (kStepTokens + 1) * attn_span_index((int)pos + m);
     if (d.graph[gi]) {
       HIP_CHECK(hipGraphLaunch(d.graph[gi], s));
     } else if (d.graph_uses[gi]++ == 0) {
@@ -1750,12 +1753,12 @@ int rai_w4a8_fused_gate_up_dev(float *gate_out, float *up_out, const rai_qlinear
 // device address (in host code it names a host-side stand-in); it uses the
 // address hipGetSymbolAddress returns on each device, looked up once per
 // device on the first call there.  Layout (bytes): q_nat [m*cols], q_split
-// [m*cols], scales [m*groups] f32, sums [m*groups] f32, then the
-// streamed kernel's activations (2..64 tokens) or the GEMM's activation records
-// (more than 64 tokens: ceil(m/32) tiles of the group count padded to 4, 2
-// or 2 (groups of 32, 64, 128) records of 64 gs + 260 bytes; with m > 64 and
-// m * cols <= 2^20 the largest is 1024 tiles of 4 records at cols = 32, gs =
-// 32: 9.02 MiB).
+// [m*cols], scales [m*groups] f32, sums [m*groups] f32, then, by w4a8_route, the
+// streamed kernel's activations (qa_bytes) or the GEMM's records (mm_pack_bytes).
+// Within the limits below the GEMM (17 tokens and more) needs at most 9.02 MiB
+// (1024 tiles of four records at cols = 32, gs = 32), the streamed kernel at most
+// 11.34 MiB at groups of 64 and 128 and, at group 32, 12 MiB up to three tokens
+// of 349440 columns.
 namespace rai {
 constexpr size_t kNaTokenCols = size_t(1) << 20;  // m * cols
 constexpr size_t kNaGroups = size_t(1) << 16;     // m * ceil(cols / gs)
@@ -1804,8 +1807,8 @@ int rai_w4a8_matmul_noalloc_dev(float *out, const uint8_t *nib, const uint8_t *p
                                  std::to_string(rai::kNaGroups) + " token groups)");
     const bool fast = rai::w4a8_fast_path((int)cols, (int)gs, nib, params);
     // The streamed kernel's activations and the GEMM's records share a place;
-    // what does not fit it (two tokens of more than 393216 columns) takes the
-    // tiled VALU kernel.
+    // what does not fit it (three tokens of 349472 columns or more at group 32)
+    // takes the tiled VALU kernel.
     const rai::W4Route route = m > 1 && fast ? rai::w4a8_route((int)rows, (int)cols, (int)m, (int)gs, false)
                                              : rai::W4Route::kValu;
     const bool wqa = route == rai::W4Route::kStream &&
@@ -2116,8 +2119,8 @@ int rai_lookup_create(rai_model *m, size_t max_ctx, rai_lookup **out) {
     const char *env = std::getenv("RAI_STEP_GRAPHS");
     d->graphs = (m->cfg.num_experts == 0 || rai::moe_on_device(*m)) && !(env && env[0] == '0');
     const size_t spans = (size_t)rai::attn_span_index((int)d->max_ctx) + 1;
-    d->graph.assign(3 * (rai::kAttnTokens + 1) * spans, nullptr);
-    d->graph_uses.assign(3 * (rai::kAttnTokens + 1) * spans, 0);
+    d->graph.assign(3 * (rai::kStepTokens + 1) * spans, nullptr);
+    d->graph_uses.assign(3 * (rai::kStepTokens + 1) * spans, 0);
     d->rng.alloc(sizeof(rai::RngState));
     d->probs.alloc(sizeof(float) * 64 * (size_t)m->cfg.vocab_size);
     d->pscratch.alloc(sizeof(float) * (size_t)m->cfg.vocab_size);

@@ -41,7 +41,7 @@ def test_output_over_its_own_input(rai, ora, name, n, m, gs):
 
 def _tokens(x, m, cols, gs, seed):
     """Ordinary rows, and among them: values so small that the input sums are
-    subnormal, a scale past 2^88 in one group, a zero row, infinite sums."""
+    subnormal, a scale past 2^88 in one group, a zero row."""
     x = x.reshape(m, cols).astype(np.float32)
     r = np.random.default_rng(seed)
     x[r.integers(m)] *= np.float32(1e-39)
