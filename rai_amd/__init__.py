@@ -591,7 +591,8 @@ class RaiModel:
         out = np.empty_like(h)
         p = np.ascontiguousarray(positions, np.uint64)
         n = p.size * self.config.hidden_size
-        out.reshape(-1)[n:] = h.reshape(-1)[n:]  # rows past the positions come back as they are
+        if n < h.size:  # rows past the positions come back as they are
+            out.reshape(-1)[n:] = h.reshape(-1)[n:]
         _check(lib().rai_forward_batch_to(self.h, kv.h, _ptr(h), _ptr(out), _ptr(p), p.size))
         return out
 

@@ -11,9 +11,9 @@
 //
 // Against the DPP-FMA score kernel and the streamed PV kernel (one lane per
 // chain, fused.hip), 256 tokens, 32 heads of 128 on 8 kv heads, 3072 to 4096
-// positions: scores 204 -> 108 us, PV 214 -> 143 (a matrix instruction took
-// about 75 cycles in the scores' independent chains and 95 in PV's one chain
-// per wave, not the 32 of its passes).  PV's chain is as long for one tile of
+// positions: scores 204 -> 108 us, PV 214 -> 143 (counters: a SIMD finishes a
+// matrix instruction every 64 cycles in the scores, whose two or three waves each
+// run a chain, and every 93 in PV's one chain, not the 32 of its passes).  PV's chain is as long for one tile of
 // tokens as for sixteen, so it takes over only past kPvMmTokens of them.
 #include <hip/hip_runtime.h>
 

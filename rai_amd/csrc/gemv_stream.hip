@@ -18,9 +18,9 @@
 // or more, as 1024 + n minus 1024 (a second run over K).
 //
 // Loads.  The L1 serves one 64-byte piece per cycle however many lanes ask
-// for it, so no load goes out in the operand order (neighbouring lanes in
-// different rows: 330 accesses a step and wave; 14336x4096 at group 64, 9
-// tokens, took 39.5 us that way, 21.4 this way): the activations, their scales
+// for it, so no load goes out in the operand order, where neighbouring lanes lie
+// in different rows (14336x4096 at group 64, 9 tokens, took 39.5 us that way, 21.4
+// this way; at group 128 a wave makes 111 accesses a step): the activations, their scales
 // and their sums ("qa", written by the quantizing kernels) lie in lane order
 // and are read a few steps ahead; the codes are read as whole row pieces, four
 // steps (a stage) at a time, and the parameters likewise, a stage or two ahead,
