@@ -4,6 +4,7 @@ a row on the same device buffers, the second with fewer tokens and a smaller
 matrix (the shared scratch keeps the first call's contents), every kernel that
 the route picks, also captured in a graph and replayed, and the size limit."""
 import ctypes
+import gc
 
 import numpy as np
 import pytest
@@ -65,9 +66,16 @@ def test_noalloc_in_a_graph(rai, rows, cols, m, gs):
         assert rc == 0, (name, rc)
 
     hip("hipStreamCreate", ctypes.byref(stream))
-    hip("hipStreamBeginCapture", stream, 1)  # thread-local
-    rc = L.rai_w4a8_matmul_noalloc_dev(do.ptr, dn.ptr, dp.ptr, dx.ptr, rows, cols, m, gs, stream)
-    hip("hipStreamEndCapture", stream, ctypes.byref(graph))
+    # No garbage collection in between: a device array that it frees (hipFree from
+    # the capturing thread) would invalidate the capture.
+    gc.collect()
+    gc.disable()
+    try:
+        hip("hipStreamBeginCapture", stream, 1)  # thread-local
+        rc = L.rai_w4a8_matmul_noalloc_dev(do.ptr, dn.ptr, dp.ptr, dx.ptr, rows, cols, m, gs, stream)
+        hip("hipStreamEndCapture", stream, ctypes.byref(graph))
+    finally:
+        gc.enable()
     assert rc == 0, L.rai_last_error().decode()
     hip("hipGraphInstantiate", ctypes.byref(ex), graph, None, None, ctypes.c_size_t(0))
     for x, w in list(zip(xs, want)) + [(xs[0], want[0])]:
